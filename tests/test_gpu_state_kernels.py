@@ -1,0 +1,122 @@
+"""The state kernels of the segment-state shapes (la_based_state_export, la_based_state_apply) at the
+edges of their tiles, against 64 bits.  Bounds: every output is a fp32 sum of exact products (export)
+or of products with 22-bit state entries (apply), so it is off by at most (steps 2^-24 + 2^-21) times
+the sum of the magnitudes of its terms, steps the additions in a row (two MFMAs for each 16 tokens,
+and the parts; two for each 16 features)."""
+
+import math
+
+import pytest
+import torch
+
+from oracle import reference as ref
+from tests.helpers import rand_qkv
+
+pytestmark = pytest.mark.gpu
+
+
+def _call(fn, *args):
+    from kernels import _lib
+    _lib.check(getattr(_lib.lib(), fn)(*args, torch.cuda.current_stream().cuda_stream), fn)
+
+
+def _ws(B, H, N, d, dv):
+    from kernels import _lib
+    n = int(_lib.lib().la_based_state_workspace_bytes(B, H, N, d, dv))
+    return torch.full((n,), 0x7f, dtype=torch.uint8, device="cuda"), n
+
+
+def _phi(x, scale):
+    d = x.shape[-1]
+    return ref.taylor_feature_map(x.double() * math.sqrt(scale * math.sqrt(d)))
+
+
+def _inputs(B, H, N, d, dv, kscale=1.0, vscale=1.0):
+    q, k, v = rand_qkv(B, H, N, d, dv, seed=N + 131 * d + dv, dtype=torch.float32, scale_qk=0.7)
+    return (q * kscale).bfloat16(), (k * kscale).bfloat16(), (v * vscale).bfloat16()
+
+
+CASES = [(1, 1, 1, 64, 64), (2, 1, 63, 33, 31), (1, 3, 64, 32, 32), (1, 2, 65, 31, 33), (2, 2, 129, 64, 65),
+         (1, 2, 300, 16, 128), (1, 1, 513, 17, 1), (3, 1, 257, 1, 7), (1, 1, 1100, 63, 100), (4, 16, 200, 48, 64),
+         (8, 12, 130, 64, 96)]
+
+
+@pytest.mark.parametrize("with_state", [False, True])
+@pytest.mark.parametrize("B,H,N,d,dv", CASES)
+def test_export(B, H, N, d, dv, with_state):
+    _, k, v = _inputs(B, H, N, d, dv)
+    scale = 1.0 / math.sqrt(d)
+    ph, vx = _phi(k, scale).transpose(-2, -1), torch.cat([v.double(), torch.ones(B, H, N, 1, dtype=torch.float64)], -1)
+    old = torch.randn(B, H, ph.shape[-2], dv + 1) if with_state else torch.zeros(B, H, ph.shape[-2], dv + 1)
+    want, mag = ph @ vx + old.double(), ph.abs() @ vx.abs() + old.abs().double()
+    ws, n = _ws(B, H, N, d, dv)
+    old_d, out = old.cuda(), torch.full_like(old, float("nan"), device="cuda")
+    kd, vd = k.cuda(), v.cuda()
+    _call("la_based_state_export", kd.data_ptr(), vd.data_ptr(), 1, old_d.data_ptr() if with_state else None,
+          out.data_ptr(), B, H, N, d, dv, scale, ws.data_ptr(), n)
+    off = ((out.cpu().double() - want).abs() / mag.clamp_min(1e-30)).max().item()
+    assert off < (N / 8 + 16) * 2.0 ** -24, off
+    if with_state:   # in place
+        _call("la_based_state_export", kd.data_ptr(), vd.data_ptr(), 1, old_d.data_ptr(), old_d.data_ptr(), B, H, N, d,
+              dv, scale, ws.data_ptr(), n)
+        assert torch.equal(old_d, out)
+
+
+@pytest.mark.parametrize("normalize", [0, 1])
+@pytest.mark.parametrize("B,H,N,d,dv", CASES + [(2, 8, 4200, 64, 32)])
+def test_apply(B, H, N, d, dv, normalize):
+    q, _, _ = _inputs(B, H, N, d, dv)
+    scale, eps = 0.8 / math.sqrt(d), 1e-6
+    F = 1 + d + d * (d + 1) // 2
+    g = torch.Generator().manual_seed(N)
+    st = torch.randn(B, H, F, dv + 1, generator=g) * torch.exp(torch.randn(B, H, F, 1, generator=g))
+    st[..., dv] = st[..., dv].abs()
+    st[:, :, 0, dv] += 4.0 * F      # denominators away from zero
+    num, den = torch.randn(B, H, N, dv, generator=g), torch.rand(B, H, N, generator=g) + 1
+    ph = _phi(q, scale)
+    tot, mag = ph @ st.double(), ph.abs() @ st.abs().double()
+    tn, td = tot[..., :dv] + num.double(), tot[..., dv] + den.double()
+    rel = (F / 8 + 16) * 2.0 ** -24 + 2.0 ** -21
+    en, ed = rel * (mag[..., :dv] + num.abs().double()), rel * (mag[..., dv] + den.double())
+    if normalize:
+        want = tn / (td + eps).unsqueeze(-1)
+        bound = (en + want.abs() * ed.unsqueeze(-1)) / td.abs().unsqueeze(-1)
+    else:
+        want, bound = tn, en
+    ws, n = _ws(B, H, N, d, dv)
+    nd, dd, qd, sd = num.cuda(), den.cuda(), q.cuda(), st.cuda()
+    out = torch.full((B, H, N, dv), float("nan"), device="cuda")
+    args = (qd.data_ptr(), 1, sd.data_ptr(), nd.data_ptr(), dd.data_ptr())
+    tail = (0, B, H, N, d, dv, scale, eps, normalize, ws.data_ptr(), n)
+    _call("la_based_state_apply", *args, out.data_ptr(), *tail)
+    off = ((out.cpu().double() - want).abs() / bound).max().item()
+    assert off < 1.1, off      # 1.1: the quotient's own rounding
+    _call("la_based_state_apply", *args, nd.data_ptr(), *tail)   # over the numerator
+    assert torch.equal(nd, out)
+
+
+@pytest.mark.parametrize("kscale,vscale", [(1e-12, 1e-20), (1e3, 1e20), (0.0, 1.0), (1.0, 0.0), (64.0, 2.0 ** -100)])
+def test_scales(kscale, vscale):
+    """Powers far from one (fp16 operands carry exponents of their own) and zeros."""
+    B, H, N, d, dv = 1, 2, 200, 64, 64
+    q, k, v = _inputs(B, H, N, d, dv, kscale, vscale)
+    scale = 1.0 / math.sqrt(d)
+    vx = torch.cat([v.double(), torch.ones(B, H, N, 1, dtype=torch.float64)], -1)
+    ph = _phi(k, scale).transpose(-2, -1)
+    want, mag = ph @ vx, ph.abs() @ vx.abs()
+    ws, n = _ws(B, H, N, d, dv)
+    st = torch.full(want.shape, float("nan"), device="cuda", dtype=torch.float32)
+    kd, vd, qd = k.cuda(), v.cuda(), q.cuda()
+    _call("la_based_state_export", kd.data_ptr(), vd.data_ptr(), 1, None, st.data_ptr(), B, H, N, d, dv, scale,
+          ws.data_ptr(), n)
+    off = (st.cpu().double() - want).abs() - (N / 8 + 16) * 2.0 ** -24 * mag
+    assert float(off.max()) <= 1e-36      # fp32 subnormals
+    num, den = torch.zeros(B, H, N, dv, device="cuda"), torch.zeros(B, H, N, device="cuda")
+    out = torch.empty_like(num)
+    _call("la_based_state_apply", qd.data_ptr(), 1, st.data_ptr(), num.data_ptr(), den.data_ptr(), out.data_ptr(), 0, B,
+          H, N, d, dv, scale, 0.0, 1, ws.data_ptr(), n)
+    pq, s64 = _phi(q, scale), st.cpu().double()
+    z = (pq @ s64[..., dv:])
+    y, m = (pq @ s64[..., :dv]) / z, (pq.abs() @ s64.abs()[..., :dv]) / z
+    rel = 2 * ((ph.shape[-2] / 8 + 16) * 2.0 ** -24 + 2.0 ** -21)
+    assert float(((out.cpu().double() - y).abs() - rel * m).max()) <= 1e-36

@@ -1,4 +1,4 @@
-"""ctypes binding of libbased_la.so (the C ABI declared in include/based_la.h).
+"""ctypes binding of libbased_la.so (the C ABI declared in include/based_la.h and based_la_state.h).
 
 The library is loaded lazily, after ``import torch`` so that its HIP runtime dependency
 resolves to the runtime torch has already mapped; launches go on torch's current stream.
@@ -68,6 +68,11 @@ _SIGNATURES = {
     "la_identity_workspace_bytes": (_c_size, [_c_int, _c_int, _c_int, _c_int, _c_int]),
     "la_identity_linear_fwd": (_c_int, [_c_void, _c_void, _c_void, _c_int, _c_void, _c_int, _c_int, _c_int, _c_int,
                                         _c_int, _c_int, _c_float, _c_void, _c_size, _c_void]),
+    "la_based_state_workspace_bytes": (_c_size, [_c_int, _c_int, _c_int, _c_int, _c_int]),
+    "la_based_state_export": (_c_int, [_c_void, _c_void, _c_int, _c_void, _c_void, _c_int, _c_int, _c_int, _c_int,
+                                       _c_int, _c_float, _c_void, _c_size, _c_void]),
+    "la_based_state_apply": (_c_int, [_c_void, _c_int, _c_void, _c_void, _c_void, _c_void, _c_int, _c_int, _c_int,
+                                      _c_int, _c_int, _c_int, _c_float, _c_float, _c_int, _c_void, _c_size, _c_void]),
     "la_taylor_feature_map": (_c_int, [_c_void, _c_int, _c_void, _c_int, ctypes.c_longlong, _c_int, _c_void]),
 }
 

@@ -155,14 +155,17 @@ def _segment_state_with_state(qc, kc, vc, cdt, kdt, chunk, scale, eps, normalize
     """State export and import for the segment-state shapes (d != 16, dv > 64 or fp32 inputs).
 
     The kernels of la_based_chunked_fwd_num_den give every row's numerator and denominator over
-    these tokens from a zero state; the state enters as plain fp32 GEMMs in the reference
-    feature basis, with phi from la_taylor_feature_map at phi(a x), a = (scale^2 d)^(1/4), so
-    that phi(a q) . phi(a k) = 1 + s + s^2 / 2 for s = scale q.k (a = 1 at scale = 1/sqrt(d)):
+    these tokens from a zero state; the state enters in the reference feature basis, phi of a x
+    with a = (scale^2 d)^(1/4), so that phi(a q) . phi(a k) = 1 + s + s^2 / 2 for s = scale q.k
+    (a = 1 at scale = 1/sqrt(d)):
       import:  num += phi(a Q) S_in[:, :dv],  den += phi(a Q) S_in[:, dv]   (every query row)
       export:  [S | z] = S_in + phi(a K)^T [V | 1]
     The layout of the states is the recurrence path's ((b, h, F, dv + 1), fp32), so states pass
     between the two paths and to based_decode_step (which evaluates phi at scale 1/sqrt(d)).  The
     token count of state_in is its own z[0]; no separate count is needed.
+
+    bf16 inputs take la_based_state_apply and la_based_state_export, which never form phi.  fp32
+    inputs, whose products k_i k_j have 48 bits, take phi from la_taylor_feature_map and fp32 GEMMs.
     """
     b, h, t, d = qc.shape
     dv = vc.shape[-1]
@@ -197,6 +200,22 @@ def _segment_state_with_state(qc, kc, vc, cdt, kdt, chunk, scale, eps, normalize
             b, h, t, d, dv, chunk, scale, _lib.ptr(ws), ws_bytes, _lib.stream_of(qc))
         _lib.check(rc, "la_based_chunked_fwd_num_den")
     state = torch.empty(b, h, F, dv + 1, dtype=torch.float32, device=dev) if return_state else None
+    if cdt == torch.bfloat16 and rows * t > 0:
+        st_bytes = int(L.la_based_state_workspace_bytes(b, h, t, d, dv))
+        ws = torch.empty(st_bytes, dtype=torch.uint8, device=dev)
+        if state_in is not None:
+            out = torch.empty(b, h, t, dv, dtype=kdt, device=dev)
+            rc = L.la_based_state_apply(
+                _lib.ptr(qc), _lib.dtype_code(cdt), _lib.ptr(sin), _lib.ptr(num), _lib.ptr(den), _lib.ptr(out),
+                _lib.dtype_code(kdt), b, h, t, d, dv, scale, eps, 1 if normalize else 0, _lib.ptr(ws), st_bytes,
+                _lib.stream_of(qc))
+            _lib.check(rc, "la_based_state_apply")
+        if return_state:
+            rc = L.la_based_state_export(
+                _lib.ptr(kc), _lib.ptr(vc), _lib.dtype_code(cdt), _lib.ptr(sin if state_in is not None else None),
+                _lib.ptr(state), b, h, t, d, dv, scale, _lib.ptr(ws), st_bytes, _lib.stream_of(qc))
+            _lib.check(rc, "la_based_state_export")
+        return out, state
     per_head = max(1, t * F * 4)
     group = max(1, min(rows, _PHI_BYTES // per_head))
     qf, kf, vf = qc.view(rows, t, d), kc.view(rows, t, d), vc.view(rows, t, dv)
