@@ -1,0 +1,86 @@
+"""The wide parallel kernel (bf16, d <= 64 and dv <= 128 in eights, other than d = 16 with dv <= 64) at
+the edges of its tiles, against 64 bits.  Bound: p = 1 + r with r rounded to fp16 (2^-11 relative) and
+everything else in fp32, in the numerator and in the row sum, so |y - y64| <= (2^-11 + 2^-13)
+(sum |r| |v| + |y| sum |r|) / den + N 2^-24 sum p |v| / den."""
+
+import math
+
+import pytest
+import torch
+
+from tests.helpers import rand_qkv
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(q, k, v, y, den, scale, eps=1e-6):
+    q, k, v = (x.double().cpu() for x in (q, k, v))
+    N = q.shape[2]
+    s = scale * q @ k.transpose(-2, -1)
+    r = torch.tril(s + 0.5 * s * s)
+    one = torch.tril(torch.ones(N, N, dtype=torch.float64))
+    d64 = (r + one).sum(-1, keepdim=True)
+    y64 = (r + one) @ v / (d64 + eps)
+    mag = r.abs().sum(-1, keepdim=True)
+    bound = (2.0 ** -11 + 2.0 ** -13) * (r.abs() @ v.abs() + y64.abs() * mag) / d64
+    bound = bound + (N + 64) * 2.0 ** -24 * ((r.abs() + one) @ v.abs()) / d64 + 1e-30
+    off = ((y.double().cpu() - y64).abs() / bound).max().item()
+    offd = ((den.double().cpu() - d64[..., 0]).abs() / ((2.0 ** -11 + 2.0 ** -13) * mag[..., 0] + N * 2.0 ** -24 * d64[..., 0])).max().item()
+    return off, offd
+
+
+@pytest.mark.parametrize("B,H,N,d,dv", [
+    (1, 1, 1, 64, 64), (1, 2, 31, 8, 8), (2, 1, 63, 24, 40), (1, 3, 64, 32, 32), (1, 1, 65, 40, 64), (1, 2, 127, 64, 72),
+    (3, 1, 128, 16, 128), (1, 8, 129, 48, 96), (1, 1, 255, 56, 16), (2, 2, 257, 64, 128), (1, 2, 515, 32, 64),
+    (4, 128, 257, 64, 64), (4, 128, 200, 32, 32), (2, 256, 130, 16, 72)])   # the last three: 256-query work-groups
+@pytest.mark.parametrize("scale", [None, 0.09])
+def test_edges(B, H, N, d, dv, scale):
+    import kernels as K
+    q, k, v = (x.cuda() for x in rand_qkv(B, H, N, d, dv, seed=N + d + dv, dtype=torch.bfloat16, scale_qk=0.7))
+    y, den = K.based_parallel(q, k, v, scale=scale, out_dtype=torch.float32, return_den=True)
+    off, offd = _check(q, k, v, y, den, 1.0 / math.sqrt(d) if scale is None else scale)
+    assert off < 1 and offd < 1, (off, offd)
+    assert torch.equal(K.based_parallel(q, k, v, scale=scale), y.bfloat16())
+
+
+@pytest.mark.parametrize("dv", [32, 64, 128])
+def test_v_exponents(dv):
+    """Blocks of V that differ by many powers of two (one of them zero): each wave takes the largest
+    exponent among its blocks, and smaller ones multiply apart."""
+    import kernels as K
+    q, k, v = rand_qkv(2, 2, 400, 64, dv, seed=dv, dtype=torch.bfloat16, scale_qk=0.7)
+    f = torch.ones(400)
+    # whole 64-key blocks: inside a block fp16 V^T holds 2^-14 of its largest value in full (bf16's 8 bits
+    # down to 2^-24), so the bound, relative to each row's own terms, needs one magnitude per block
+    f[64:128], f[128:192], f[192:256], f[256:320], f[320:] = 2.0 ** -30, 0.0, 2.0 ** 40, 2.0 ** 41, 2.0 ** 90
+    v = (v.float() * f[:, None]).bfloat16()
+    qd, kd, vd = (x.cuda() for x in (q, k, v))
+    y, den = K.based_parallel(qd, kd, vd, out_dtype=torch.float32, return_den=True)
+    off, offd = _check(q, k, v, y, den, 0.125)
+    assert off < 1 and offd < 1, (off, offd)
+
+
+def test_pre_pass_apart_and_misaligned():
+    """The two halves apart equal the whole call; an output that is not 16-byte aligned takes the
+    register-staged kernel, after the same pre-pass too."""
+    from kernels import _lib
+    L = _lib.lib()
+    B, H, N, d, dv = 1, 3, 300, 64, 64
+    q, k, v = (x.cuda() for x in rand_qkv(B, H, N, d, dv, seed=5, dtype=torch.bfloat16, scale_qk=0.7))
+    n = int(L.la_based_parallel_workspace_bytes(B, H, N, d, dv, 1))
+    st = torch.cuda.current_stream().cuda_stream
+    buf = torch.empty(B * H * N * dv + 8, device="cuda")
+    outs = []
+    for skew, apart in ((0, False), (0, True), (1, False), (1, True)):
+        ws = torch.full((n,), 0x7f, dtype=torch.uint8, device="cuda")
+        out = buf[skew:skew + B * H * N * dv]
+        args = (B, H, N, d, dv)
+        if apart:
+            assert L.la_based_parallel_pack(k.data_ptr(), v.data_ptr(), 1, *args, ws.data_ptr(), n, st) == 0
+        f = L.la_based_parallel_fwd_packed if apart else L.la_based_parallel_fwd
+        assert f(q.data_ptr(), k.data_ptr(), v.data_ptr(), 1, out.data_ptr(), 0, None, *args, 0.125, 1e-6, 1, ws.data_ptr(),
+                 n, st) == 0
+        outs.append(out.clone().view(B, H, N, dv))
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[2], outs[3])
+    for y in outs[::2]:
+        assert _check(q, k, v, y, torch.zeros(1), 0.125)[0] < 1

@@ -826,8 +826,8 @@ int dispatch_mt(const ParallelParams& p, bool vec, bool packed, int stages, hipS
 }  // namespace
 
 // bf16 inputs.  Packed shapes: [V^T blocks: BH * nb64 * vt_block_bytes][statistics prefixes:
-// BH * nb64 * stats_width(DV) fp32].  Other shapes: BH * VR partial maxima of |v| (u32).  The
-// packed layout is never smaller, so a packed shape that falls back to the register-staged
+// BH * nb64 * stats_width(DV) fp32].  Other shapes: BH * VR partial maxima of |v| (u32), then for the
+// wide kernel's its V^T blocks and their column sums.  The packed layout is never smaller, so a packed shape that falls back to the register-staged
 // kernel (misaligned tensors) keeps its partial maxima at the start of the same workspace.
 size_t vrange_bytes(int BH) { return (size_t)BH * VR * 4; }
 
@@ -835,7 +835,7 @@ bool parallel_packed_shape(int d, int dv, bool in_f32) { return !in_f32 && packe
 
 size_t parallel_workspace_bytes(int BH, int N, int d, int dv, bool in_f32) {
   if (in_f32) return f32_split_workspace_bytes(BH, N, d, dv);   // partials of a key split, or 0
-  if (!packed_shape(d, dv)) return vrange_bytes(BH);
+  if (!packed_shape(d, dv)) return vrange_bytes(BH) + (wide_shape(N, d, dv) ? wide_workspace_bytes(BH, N, dv) : 0);
   const size_t nb64 = ((size_t)N + BN - 1) / BN;
   const int DV = dv <= 32 ? 32 : 64;
   return (size_t)BH * nb64 * (vt_block_bytes(dv) + (size_t)stats_width(DV) * 4);
@@ -891,6 +891,20 @@ int launch_based_parallel(const ParallelArgs& a, hipStream_t stream) {
   const bool packed = packed_shape(a.d, a.dv) && a.packed_aligned &&
                       a.workspace_bytes >= parallel_workspace_bytes(a.BH, a.N, a.d, a.dv, false) &&
                       (size_t)p.nb64 * vt_block_bytes(a.dv) < ((size_t)1 << 30) && (size_t)a.N * 32 < ((size_t)1 << 30);
+  // The wide kernel takes its shapes unless a tensor is not 16-byte aligned (its copies and stores
+  // are whole 16-byte units); then, and for d > 64, d % 8 or dv % 8, the register-staged kernel.  A
+  // pre-pass on its own also leaves the maxima of that one, for a later call whose q or out is not
+  // aligned.  B2 H16, whole call, register-staged / wide: d64 dv64 N2048 63 / 36 us, N8192
+  // 453 / 266 us; d32 dv64 N8192 268 / 218; d64 dv128 N8192 593 / 420; B1 H2 N200 d64 18.0 / 18.0.
+  const bool al16 = ((reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.k) |
+                      reinterpret_cast<uintptr_t>(a.v) | reinterpret_cast<uintptr_t>(a.out)) & 15) == 0;
+  if (al16 && wide_shape(a.N, a.d, a.dv)) {
+    if (a.stages == 1)
+      hipLaunchKernelGGL(vrange_kernel, dim3((unsigned)VR, (unsigned)a.BH), dim3(256), 0, stream, p.v, p.N, p.dv,
+                         const_cast<u32*>(p.vmax));
+    const WideScale s{p.inv_c, p.inv_c2, p.fscale, p.qscale, p.ones_hi, p.ones_lo};
+    return launch_wide_parallel(a, static_cast<char*>(a.workspace) + vrange_bytes(a.BH), s, stream);
+  }
   if (a.d <= 16) return dispatch_mt<1>(p, vec, packed, a.stages, stream);
   if (a.d <= 32) return dispatch_mt<2>(p, vec, false, a.stages, stream);
   if (a.d <= 64) return dispatch_mt<4>(p, vec, false, a.stages, stream);

@@ -1,0 +1,540 @@
+// Fused causal BASED attention, parallel form, for the bf16 head dims the packed d = 16 kernel does
+// not take: d <= 64 with d % 8 == 0, dv <= 128 with dv % 8 == 0, 16-byte aligned tensors.  Same
+// function, precision and range as based_parallel.hip (see there: u = (q.k + 1/c)^2 - 1/c^2 in
+// fp16, V^T in fp16 with exponents, the 1 of p kept exact), other data paths:
+//
+//   wide_pack_kernel  one work-group per 64-key block: V as an fp16 V^T block in the main kernel's
+//                     LDS layout with an exponent of its own, and its fp32 column sums;
+//   wide_kernel       K rows (from the caller's tensor) and V^T blocks copied global -> LDS with
+//                     buffer_load ... lds into a ring; S^T = K Q^T on bf16 MFMAs, u in registers,
+//                     O^T += V^T u^T on fp16 MFMAs, row sums of u with v_dot2.
+//
+// There is no scan between them: a work-group adds the column sums of the blocks before its own
+// queries itself (DV floats per block, against 2 (d + dv) 64 bytes of K and V that it reads of each),
+// and a wave takes the largest exponent of the blocks it attends to; a block with a smaller one
+// (rare) multiplies into cleared accumulators that are added in fp32 with the power of two.
+//
+// What bounds it: matrix cores and LDS reads.  A wave owns 64 queries (two 32-wide tiles), so a K
+// or V^T fragment read (1 KB, 16 bytes a lane) feeds two MFMAs: d = dv = 64 reads 16 KB per 32 MFMAs
+// and wave, 64 of 128 bytes a clock at full MFMA rate; with one tile (32 queries) it would be all of
+// them.  256-query work-groups (four waves) where they fill the CUs twice; else 128-query ones, whose
+// wave pairs share queries and take one 32-key half of every block each (their accumulators meet
+// in LDS at the end), so that the grid is twice as large at the same reads per MFMA.
+//
+// Measured (pre-pass + kernel, us; the register-staged kernel and its max pass before): B2 H16 d64 dv64
+// N2048 7 + 29 (5 + 62), N8192 14 + 252 (8 + 445): 1.04 PFLOP/s, matrix cores busy 57 % of the
+// cycles at the 1.9 GHz that the card holds under this load.  At N2048 20 of the 29 us are the loop
+// of the longest work-groups (16 steps), the rest launch, queries, column sums and the epilogue.
+#include <type_traits>
+
+#include "../../include/based_la.h"
+#include "la_common.hpp"
+#include "la_internal.hpp"
+#include "la_pack.hpp"
+
+namespace la {
+namespace {
+
+struct WideParams {
+  const uint16_t* q;
+  const uint16_t* k;
+  const uint16_t* v;
+  uint16_t* vt;          // [BH][nb][32 MT rows][64] fp16
+  float* sums;           // [BH][nb][32 MT] column sums of V
+  int* eb;               // [BH][nb] V exponents
+  void* out;
+  float* den;
+  int BH, N, d, dv, nqb, nb;
+  float inv_c, inv_c2, fscale, eps, qscale;
+  u32 ones_hi, ones_lo;
+  int normalize, out_f32, xcd_cus;
+};
+
+// V^T rows: 64 keys = eight 16-byte units; unit 2 m + h of a row holds keys 16 m + 4 h + {0..3, 8..11}
+// (the order of a score accumulator's registers, so a unit is a whole A operand of the P.V MFMA),
+// stored at unit ^ wswz(row).  K rows of 2 KS 16-byte chunks: chunk c at c ^ kwz(key).  Both make
+// the 16 lanes of a ds_read_b128 pass touch all 64 banks once.
+__device__ __forceinline__ int wswz(int r) { return ((r >> 2) & 7) ^ ((r & 2) << 1); }
+template <int KS>
+__device__ __forceinline__ int kwz(int key) {
+  return KS == 1 ? ((key >> 2) ^ (key >> 3)) & 1 : KS == 2 ? (key >> 2) & 3 : wswz(key);
+}
+
+// ---------------------------------------------------------------- V^T blocks
+// Thread -> keys 2 kp, 2 kp + 1 and eight columns; column sums through LDS.  Any dv: rows past dv
+// and keys past N are zero.
+template <int MT>
+__global__ __launch_bounds__(256) void wide_pack_kernel(const WideParams p) {
+  constexpr int DV = 32 * MT, CPR = DV / 8, IT = (32 * CPR + 255) / 256;
+  __shared__ __attribute__((aligned(16))) uint16_t img[DV * BN];
+  __shared__ float csum[32][DV + 1];
+  __shared__ u32 vmx[4];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int bh = blockIdx.x / p.nb, blk = blockIdx.x - bh * p.nb, dv = p.dv;
+  const __amdgpu_buffer_rsrc_t rv = make_rsrc(p.v + (size_t)bh * p.N * dv, (u32)p.N * (u32)dv * 2u);
+  u32x4 a[IT], b[IT];
+  u32 m = 0u;
+#pragma unroll
+  for (int x = 0; x < IT; ++x) {
+    const int t = tid + 256 * x, kp = t / CPR, col = 8 * (t % CPR);
+    const int off = kp < 32 && col < dv ? ((blk * BN + 2 * kp) * dv + col) * 2 : kOffOutOfRange;
+    a[x] = buf_load_b128(rv, off);
+    b[x] = buf_load_b128(rv, off == kOffOutOfRange ? off : off + 2 * dv);
+  }
+#pragma unroll
+  for (int x = 0; x < IT; ++x)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const u32 y = a[x][i] & 0x7fff7fffu, z = b[x][i] & 0x7fff7fffu;
+      m = max(m, max(max(y & 0xffffu, y >> 16), max(z & 0xffffu, z >> 16)));
+    }
+  m = wave_max_u32(m);
+  if (lane == 0) vmx[w] = m;
+  __syncthreads();
+  const int eb = vexp_step(max(max(vmx[0], vmx[1]), max(vmx[2], vmx[3])) << 16);
+#pragma unroll
+  for (int x = 0; x < IT; ++x) {
+    const int t = tid + 256 * x, kp = t / CPR, col = 8 * (t % CPR);
+    if (kp >= 32) continue;
+    // keys 2 kp, 2 kp + 1 = 16 m + 8 (e / 4) + 4 h + e % 4
+    const int r = (2 * kp) & 15, unit = 2 * (kp >> 3) + ((r >> 2) & 1), e = ((r >> 3) << 2) | (r & 3);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      const float f0 = (c & 1) ? bf16_hi_to_f32(a[x][c >> 1]) : bf16_lo_to_f32(a[x][c >> 1]);
+      const float f1 = (c & 1) ? bf16_hi_to_f32(b[x][c >> 1]) : bf16_lo_to_f32(b[x][c >> 1]);
+      const int row = col + c;
+      csum[kp][row] = f0 + f1;
+      *reinterpret_cast<u32*>(&img[row * BN + ((unit ^ wswz(row)) << 3) + e]) =
+          pack_f16x2(__builtin_ldexpf(f0, -eb), __builtin_ldexpf(f1, -eb));
+    }
+  }
+  __syncthreads();
+  const size_t rec = (size_t)bh * p.nb + blk;
+  u32x4* dst = reinterpret_cast<u32x4*>(p.vt + rec * (DV * BN));
+  for (int i = tid; i < DV * BN / 8; i += 256) dst[i] = reinterpret_cast<const u32x4*>(img)[i];
+  if (tid < DV) {
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < 32; ++i) s += csum[i][tid];
+    p.sums[rec * DV + tid] = s;
+  }
+  if (tid == 0) p.eb[rec] = eb;
+}
+
+// ---------------------------------------------------------------- attention
+// KS: 16-wide steps of d; MT: 32-wide tiles of dv; QT: 32-query tiles per wave; NKH: waves sharing a
+// query group (2: each takes one 32-key half of every block).  UNIT: 1/c scales to exactly 1/2.
+template <int KS, int MT, int QT, int NKH, bool UNIT>
+__global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
+  constexpr int DV = 32 * MT, NQW = 4 / NKH, BM = 32 * QT * NQW;
+  constexpr int UB = NKH;                           // blocks per step (two 32-key units per wave either way)
+  constexpr int UK = 2 * KS, UV = 4 * MT;           // 1 KB copy units of a block
+  constexpr int CW = (UK + UV + 3) / 4;             // copies per wave and block
+  constexpr int BLK = 4 * CW * 512;                 // halves per block in LDS
+  constexpr int NSR = NKH == 2 ? 2 : CW <= 4 ? 4 : 3;   // steps in the ring
+  __shared__ __attribute__((aligned(16))) uint16_t ring[NSR * UB][BLK];
+  __shared__ float vsl[NQW][DV];
+
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), h = lane >> 5, n = lane & 31;
+  const int qg = NKH == 2 ? wv >> 1 : wv, kh = NKH == 2 ? wv & 1 : 0;
+  const int N = p.N, d = p.d, dv = p.dv;
+  int bh, qb;
+  map_causal_block(blockIdx.x, p.BH, p.nqb, bh, qb, p.xcd_cus);
+  const int q0 = qb * BM, jb0 = q0 / BN;
+  const int nblk = min(p.nb, (q0 + BM + BN - 1) / BN), nstep = (nblk + UB - 1) / UB;
+  const int wq0 = q0 + 32 * QT * qg, jd = wq0 / BN;
+  const bool live = wq0 < N;
+  const size_t hrow = (size_t)bh * N;
+
+  // ---- ring copies: unit u < UK of a block are K rows, then V^T rows (then padding, never read)
+  const u32x4 rk = buffer_rsrc(p.k + hrow * d, (u32)N * (u32)d * 2u);
+  const u32x4 rv = buffer_rsrc(p.vt + (size_t)bh * p.nb * (DV * BN), (u32)p.nb * (u32)(DV * BN * 2));
+  int uoff[CW];
+#pragma unroll
+  for (int x = 0; x < CW; ++x) {
+    const int u = 4 * x + wv;
+    if (u < UK) {
+      const int sl = 64 * u + lane, key = sl / (2 * KS), c = (sl % (2 * KS)) ^ kwz<KS>(key);
+      uoff[x] = 8 * c < d ? key * d * 2 + 16 * c : kOffOutOfRange;
+    } else {
+      uoff[x] = u < UK + UV ? 1024 * (u - UK) + 16 * lane : kOffOutOfRange;
+    }
+  }
+  auto issue = [&](int s) {   // steps and blocks past the last read nothing: the counts stay equal
+#pragma unroll
+    for (int t = 0; t < UB; ++t) {
+      const int j = UB * s + t;
+      const u32 lds = lds_addr(&ring[(s % NSR) * UB + t][0]);
+#pragma unroll
+      for (int x = 0; x < CW; ++x) {
+        const int u = 4 * x + wv;
+        const bool isk = u < UK;
+        const int off = j < nblk && uoff[x] != kOffOutOfRange ? uoff[x] + j * (isk ? BN * 2 * d : DV * BN * 2) : kOffOutOfRange;
+        lds_copy16(isk ? rk : rv, lds + 1024 * u, off);
+      }
+    }
+  };
+#pragma unroll
+  for (int s = 0; s < NSR - 1; ++s) issue(s);
+
+  // ---- queries (B operand of S^T = K Q^T): q[query][16 kk + 8 h .. + 7], scaled by a power of two
+  u32x4 qf[QT][KS];
+#pragma unroll
+  for (int qt = 0; qt < QT; ++qt) {
+    const int query = wq0 + 32 * qt + n;
+#pragma unroll
+    for (int kk = 0; kk < KS; ++kk) {
+      const int col = 16 * kk + 8 * h;
+      u32x4 x = {0u, 0u, 0u, 0u};
+      if (query < N && col < d) x = *reinterpret_cast<const u32x4*>(p.q + (hrow + query) * d + col);
+      qf[qt][kk] = scale_bf16x8(x, p.qscale);
+    }
+  }
+  // ---- exponents of the blocks this wave attends to
+  const int* __restrict__ ebs = p.eb + (size_t)bh * p.nb;
+  int emax = -128, emin = 1 << 20;
+  if (live)
+    for (int j = lane; j <= jd; j += 64) {
+      const int e = ebs[j];
+      emax = max(emax, e);
+      emin = min(emin, e);
+    }
+  emax = (int)wave_max_u32((u32)(emax + 1024)) - 1024;
+  emin = (1 << 21) - (int)wave_max_u32((u32)((1 << 21) - emin));
+  const bool mixed = live && emin != emax;
+  // ---- column sums of V over the blocks before each query group's diagonal block
+  {
+    constexpr int PARTS = 256 / DV, PF = 8;
+    float* psum = reinterpret_cast<float*>(&ring[(NSR - 1) * UB][0]);   // the last step's place, still free
+    const float* __restrict__ sm = p.sums + (size_t)bh * p.nb * DV + tid % DV;
+    float s = 0.f;
+    for (int j = tid / DV; j < jb0; j += PARTS * PF) {
+      float y[PF];
+#pragma unroll
+      for (int t = 0; t < PF; ++t) y[t] = j + PARTS * t < jb0 ? sm[(size_t)(j + PARTS * t) * DV] : 0.f;
+#pragma unroll
+      for (int t = 0; t < PF; ++t) s += y[t];
+    }
+    psum[tid] = s;
+    __syncthreads();
+    if (kh == 0)
+      for (int c = lane; c < DV; c += 64) {
+        float t = 0.f;
+#pragma unroll
+        for (int x = 0; x < PARTS; ++x) t += psum[x * DV + c];
+        for (int j = jb0; j < min(jd, p.nb); ++j) t += p.sums[((size_t)bh * p.nb + j) * DV + c];
+        vsl[qg][c] = t;
+      }
+    __syncthreads();   // psum read before the ring takes its place
+  }
+
+  f32x16 acc[QT][MT];
+  float rsum[QT];
+#pragma unroll
+  for (int qt = 0; qt < QT; ++qt) {
+    rsum[qt] = 0.f;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) acc[qt][mt] = splat16(0.f);
+  }
+  const float inv_c = UNIT ? 0.5f : p.inv_c, inv_c2 = UNIT ? 0.25f : p.inv_c2;
+  constexpr u32 kOnes = 0x3c003c00u;   // packed fp16 (1, 1)
+
+  auto kfrag = [&](const uint16_t* st, int ks, int kk) {
+    const int key = 32 * ks + n;
+    return *reinterpret_cast<const u32x4*>(st + key * (16 * KS) + (((2 * kk + h) ^ kwz<KS>(key)) << 3));
+  };
+  auto vfrag = [&](const uint16_t* st, int ks, int m, int mt) {
+    const int row = 32 * mt + n;
+    return *reinterpret_cast<const u32x4*>(st + UK * 512 + row * BN + (((4 * ks + 2 * m + h) ^ wswz(row)) << 3));
+  };
+  // pieces of a full 32-key unit: scores b = K Q^T + 1/c; u = b b - 1/c^2 in fp16 and its row sums;
+  // acc += V^T u^T
+  auto S = [&](const uint16_t* st, int ks, f32x16 (&b)[QT]) {
+    u32x4 kf[KS];
+#pragma unroll
+    for (int kk = 0; kk < KS; ++kk) kf[kk] = kfrag(st, ks, kk);
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) {
+      b[qt] = splat16(inv_c);
+#pragma unroll
+      for (int kk = 0; kk < KS; ++kk) b[qt] = mfma32x32x16(kf[kk], qf[qt][kk], b[qt]);
+    }
+  };
+  auto E = [&](const f32x16 (&b)[QT], u32x4 (&pf)[QT][2]) {
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt)
+#pragma unroll
+      for (int m = 0; m < 2; ++m)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          pf[qt][m][c] = sq_plus_f16x2(b[qt][8 * m + 2 * c], b[qt][8 * m + 2 * c + 1], -inv_c2);
+          rsum[qt] = dot2_f16(pf[qt][m][c], kOnes, rsum[qt]);
+        }
+  };
+  auto P = [&](const uint16_t* st, int ks, const u32x4 (&pf)[QT][2]) {
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+        const u32x4 vf = vfrag(st, ks, m, mt);
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt) acc[qt][mt] = mfma32x32x16_f16(vf, pf[qt][m], acc[qt][mt]);
+      }
+  };
+  // acc += 2^e V^T x^T for operands x[nx][QT][2], through cleared accumulators
+  auto Pscaled = [&](const uint16_t* st, int ks, const u32x4 (*x)[QT][2], int nx, const bool (&act)[QT], int e) {
+    const float f = __builtin_ldexpf(1.0f, e);
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      const u32x4 v0 = vfrag(st, ks, 0, mt), v1 = vfrag(st, ks, 1, mt);
+#pragma unroll
+      for (int qt = 0; qt < QT; ++qt) {
+        if (!act[qt]) continue;
+        f32x16 t = splat16(0.f);
+#pragma unroll
+        for (int y = 0; y < 3; ++y) {
+          if (y >= nx) continue;
+          t = mfma32x32x16_f16(v0, x[y][qt][0], t);
+          t = mfma32x32x16_f16(v1, x[y][qt][1], t);
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[qt][mt][r] = __builtin_fmaf(f, t[r], acc[qt][mt][r]);
+      }
+    }
+  };
+  // a unit of the wave's diagonal block, or a full unit of a block with a smaller V exponent
+  auto general = [&](const uint16_t* st, int j, int ks) {
+    const int kb = BN * j + 32 * ks, e = mixed ? max(ebs[j] - emax, -126) : 0;
+    u32x4 x[3][QT][2];   // u, then the mask times W's hi and lo parts (the exact 1 of p)
+    bool act[QT];
+    f32x16 b[QT];
+    S(st, ks, b);
+    const bool diag = j == jd;
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) {
+      const int qbase = wq0 + 32 * qt, query = qbase + n;
+      act[qt] = kb <= qbase + 31 && qbase < N;
+#pragma unroll
+      for (int m = 0; m < 2; ++m)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const int i = 8 * m + 2 * c, k0 = kb + c32_row(i, h);   // keys k0, k0 + 1
+          const float u0 = __builtin_fmaf(b[qt][i], b[qt][i], -inv_c2), u1 = __builtin_fmaf(b[qt][i + 1], b[qt][i + 1], -inv_c2);
+          const bool in0 = k0 <= query, in1 = k0 + 1 <= query;
+          x[0][qt][m][c] = pack_f16x2(in0 ? u0 : 0.f, in1 ? u1 : 0.f);
+          x[1][qt][m][c] = (in0 ? p.ones_hi & 0xffffu : 0u) | (in1 ? p.ones_hi & 0xffff0000u : 0u);
+          x[2][qt][m][c] = (in0 ? p.ones_lo & 0xffffu : 0u) | (in1 ? p.ones_lo & 0xffff0000u : 0u);
+          if (act[qt]) rsum[qt] = dot2_f16(x[0][qt][m][c], kOnes, rsum[qt]);
+        }
+    }
+    Pscaled(st, ks, x, !diag ? 1 : p.ones_lo != 0u ? 3 : 2, act, e);
+  };
+
+  // step s of this wave landed (NSR - 2 later ones may be in flight), then every wave's; every wave is
+  // past step s - 1, whose place the next copies take
+  auto begin = [&](int s) {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"i"((NSR - 2) * UB * CW) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    issue(s + NSR - 1);
+  };
+  // The step's two units: the halves of block s (NKH = 1), or this wave's half of blocks 2 s, 2 s + 1.
+  // Steps before the wave's diagonal block in a loop of their own: as one branch of a common loop the
+  // accumulators were copied at its end (32 v_mov_b64 per step).  The waves leave it at different steps
+  // and meet at the same count of barriers.
+  const int nfull = !live || mixed ? 0 : min(jd / UB, nstep);
+  for (int s = 0; s < nfull; ++s) {
+    begin(s);
+    const uint16_t* s0 = &ring[(s % NSR) * UB][0];
+    const uint16_t* s1 = NKH == 2 ? &ring[(s % NSR) * UB + 1][0] : s0;
+    const int k0 = NKH == 2 ? kh : 0, k1 = NKH == 2 ? kh : 1;
+    f32x16 b0[QT], b1[QT];
+    u32x4 p0[QT][2], p1[QT][2];
+    S(s0, k0, b0);
+    S(s1, k1, b1);
+    E(b0, p0);
+    P(s0, k0, p0);
+    E(b1, p1);
+    P(s1, k1, p1);
+  }
+#pragma unroll 1
+  for (int s = nfull; s < nstep; ++s) {
+    begin(s);
+#pragma unroll 1
+    for (int t = 0; t < 2; ++t) {
+      const int j = UB * s + (NKH == 2 ? t : 0), ks = NKH == 2 ? kh : t;
+      if (live && j <= jd && BN * j + 32 * ks <= wq0 + 32 * QT - 1) general(&ring[(s % NSR) * UB + (NKH == 2 ? t : 0)][0], j, ks);
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no copy in flight into the ring
+  __syncthreads();
+
+  // ---- the halves' sums: the wave pair splits its two query tiles, each adds the other's part
+  constexpr int QE = QT / NKH;   // query tiles a wave finishes, from tile e0
+  static_assert(NKH == 1 || QT == 2, "a wave pair finishes one tile each");
+  const int e0 = NKH == 2 ? kh : 0;
+  f32x16 fin[QE][MT];
+  float rs[QE];
+  if constexpr (NKH == 2) {
+    float* mine = reinterpret_cast<float*>(&ring[0][0]) + wv * ((16 * MT + 1) * 64) + lane;
+    float* other = reinterpret_cast<float*>(&ring[0][0]) + (wv ^ 1) * ((16 * MT + 1) * 64) + lane;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) mine[(16 * mt + r) * 64] = kh ? acc[0][mt][r] : acc[1][mt][r];
+    mine[16 * MT * 64] = kh ? rsum[0] : rsum[1];
+    __syncthreads();
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) fin[0][mt][r] = (kh ? acc[1][mt][r] : acc[0][mt][r]) + other[(16 * mt + r) * 64];
+    rs[0] = (kh ? rsum[1] : rsum[0]) + other[16 * MT * 64];
+    __syncthreads();   // read before the output tiles take their place
+  } else {
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) {
+      rs[qt] = rsum[qt];
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) fin[qt][mt] = acc[qt][mt];
+    }
+  }
+  if (!live) return;
+
+  // ---- out = (acc 2^E / W + column sums) / (t + 1 + row sum / W + eps), 32 rows x 64 columns at a
+  // time through this wave's own LDS, so that stores write whole lines
+  const float fscale = p.fscale, afs = fscale * __builtin_ldexpf(1.0f, emax);
+  auto store = [&](auto f32_tag) {
+    constexpr bool F32 = decltype(f32_tag)::value;
+    constexpr int CT = MT == 1 ? 1 : 2, EB = F32 ? 4 : 2, RB = 32 * CT * EB, RS = RB + 16, CPR = RB / 16;
+    static_assert(4 * 32 * RS <= (int)sizeof(ring), "output tiles fit in the ring");
+    char* tile = reinterpret_cast<char*>(&ring[0][0]) + wv * (32 * RS);
+#pragma unroll
+    for (int qe = 0; qe < QE; ++qe) {
+      const int qbase = wq0 + 32 * (e0 + qe), query = qbase + n;
+      const float r2 = rs[qe] + __shfl_xor(rs[qe], 32);
+      const float den = (float)(query + 1) + fscale * r2;
+      const float inv = p.normalize ? 1.0f / (den + p.eps) : 1.0f;
+      if (p.den != nullptr && h == 0 && query < N) p.den[hrow + query] = den;
+#pragma unroll
+      for (int ct = 0; ct < MT; ct += CT) {
+#pragma unroll
+        for (int mt = 0; mt < CT; ++mt)
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            float y[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              y[e] = (afs * fin[qe][ct + mt][4 * g + e] + vsl[qg][32 * (ct + mt) + 8 * g + 4 * h + e]) * inv;
+            char* dst = tile + n * RS + (32 * mt + 8 * g + 4 * h) * EB;
+            if (F32)
+              *reinterpret_cast<f32x4*>(dst) = (f32x4){y[0], y[1], y[2], y[3]};
+            else
+              *reinterpret_cast<u32x2*>(dst) = (u32x2){pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])};
+          }
+        char* out = static_cast<char*>(p.out) + ((hrow + qbase) * (size_t)dv + 32 * ct) * EB;
+        const int cols = (dv - 32 * ct) * EB;   // bytes of a row from this column on
+#pragma unroll
+        for (int it = 0; it < CPR / 2; ++it) {
+          const int idx = 64 * it + lane, r = idx / CPR, c = idx % CPR;
+          const u32x4 y = *reinterpret_cast<const u32x4*>(tile + r * RS + 16 * c);
+          if (qbase + r < N && 16 * c < cols) *reinterpret_cast<u32x4*>(out + (size_t)r * dv * EB + 16 * c) = y;
+        }
+      }
+    }
+  };
+  if (p.out_f32)
+    store(std::true_type{});
+  else
+    store(std::false_type{});
+}
+
+template <int KS, int MT, int QT, int NKH>
+int launch_main(const WideParams& pp, hipStream_t stream) {
+  WideParams p = pp;
+  constexpr int BM = 128 * QT / NKH;
+  p.nqb = (p.N + BM - 1) / BM;
+  const dim3 grid((unsigned)(p.nqb * p.BH)), block(256);
+  if (p.inv_c == 0.5f && p.inv_c2 == 0.25f)
+    hipLaunchKernelGGL((wide_kernel<KS, MT, QT, NKH, true>), grid, block, 0, stream, p);
+  else
+    hipLaunchKernelGGL((wide_kernel<KS, MT, QT, NKH, false>), grid, block, 0, stream, p);
+  return (int)hipGetLastError();
+}
+
+template <int KS, int MT>
+int launch_wide(const WideParams& p, int stages, hipStream_t stream) {
+  if (stages & 1) {
+    hipLaunchKernelGGL((wide_pack_kernel<MT>), dim3((unsigned)(p.BH * p.nb)), dim3(256), 0, stream, p);
+    const int e = (int)hipGetLastError();
+    if (e != 0) return e;
+  }
+  if (!(stages & 2)) return 0;
+  if constexpr (MT == 4) {
+    return launch_main<KS, 4, 1, 1>(p, stream);   // 64-query waves would need 128 accumulators more
+  } else {
+    const long long wg256 = (long long)((p.N + 255) / 256) * p.BH;
+    return wg256 >= 2LL * device_cu_count() ? launch_main<KS, MT, 2, 1>(p, stream) : launch_main<KS, MT, 2, 2>(p, stream);
+  }
+}
+
+int mt_of(int dv) { return dv <= 32 ? 1 : dv <= 64 ? 2 : 4; }
+size_t up256(size_t x) { return (x + 255) & ~(size_t)255; }
+
+}  // namespace
+
+bool wide_shape(int N, int d, int dv) {
+  const size_t nb = ((size_t)N + BN - 1) / BN;
+  return d % 8 == 0 && d <= 64 && dv % 8 == 0 && dv <= 128 && !(d == 16 && dv <= 64) &&
+         nb * (size_t)(32 * mt_of(dv) * BN * 2) < ((size_t)1 << 30) && (size_t)N * d * 2 < ((size_t)1 << 30) &&
+         (size_t)N * dv * 2 < ((size_t)1 << 30);
+}
+
+size_t wide_workspace_bytes(int BH, int N, int dv) {
+  const size_t nb = ((size_t)N + BN - 1) / BN, DV = 32 * mt_of(dv);
+  return up256(BH * nb * DV * BN * 2) + up256(BH * nb * DV * 4) + up256(BH * nb * 4);
+}
+
+int launch_wide_parallel(const ParallelArgs& a, void* workspace, const WideScale& s, hipStream_t stream) {
+  WideParams p{};
+  p.q = static_cast<const uint16_t*>(a.q);
+  p.k = static_cast<const uint16_t*>(a.k);
+  p.v = static_cast<const uint16_t*>(a.v);
+  p.out = a.out;
+  p.den = a.den;
+  p.BH = a.BH;
+  p.N = a.N;
+  p.d = a.d;
+  p.dv = a.dv;
+  p.nb = (a.N + BN - 1) / BN;
+  const size_t DV = 32 * mt_of(a.dv), blocks = (size_t)a.BH * p.nb;
+  char* ws = static_cast<char*>(workspace);
+  p.vt = reinterpret_cast<uint16_t*>(ws);
+  p.sums = reinterpret_cast<float*>(ws + up256(blocks * DV * BN * 2));
+  p.eb = reinterpret_cast<int*>(ws + up256(blocks * DV * BN * 2) + up256(blocks * DV * 4));
+  p.inv_c = s.inv_c;
+  p.inv_c2 = s.inv_c2;
+  p.fscale = s.fscale;
+  p.qscale = s.qscale;
+  p.ones_hi = s.ones_hi;
+  p.ones_lo = s.ones_lo;
+  p.eps = a.eps;
+  p.normalize = a.normalize ? 1 : 0;
+  p.out_f32 = a.out_f32 ? 1 : 0;
+  p.xcd_cus = device_cu_count() / 8;
+  const int ks = a.d <= 16 ? 1 : a.d <= 32 ? 2 : 4, mt = mt_of(a.dv);
+#define LA_WIDE(K, M) \
+  if (ks == K && mt == M) return launch_wide<K, M>(p, a.stages, stream)
+  LA_WIDE(1, 1);
+  LA_WIDE(1, 2);
+  LA_WIDE(1, 4);
+  LA_WIDE(2, 1);
+  LA_WIDE(2, 2);
+  LA_WIDE(2, 4);
+  LA_WIDE(4, 1);
+  LA_WIDE(4, 2);
+  LA_WIDE(4, 4);
+#undef LA_WIDE
+  return LA_ERR_UNSUPPORTED_DIM;
+}
+
+}  // namespace la
