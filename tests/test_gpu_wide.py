@@ -84,3 +84,37 @@ def test_pre_pass_apart_and_misaligned():
     assert torch.equal(outs[0], outs[1]) and torch.equal(outs[2], outs[3])
     for y in outs[::2]:
         assert _check(q, k, v, y, torch.zeros(1), 0.125)[0] < 1
+
+
+@pytest.mark.parametrize("big", [1.0, 30.0, 3000.0])
+@pytest.mark.parametrize("B,H,N,d,dv", [(1, 2, 513, 64, 64), (1, 2, 700, 32, 128), (4, 128, 514, 64, 32), (1, 3, 1024, 24, 16)])
+def test_chunked_calls_any_scores(B, H, N, d, dv, big):
+    """Chunked calls of several segments take this kernel too, with scores of any size: a query whose
+    bound on |s| passes fp16's range scales its u by 2^-2e, e from sum |q| max |k| <= 128 2^e / qscale.
+    The bound above, and u's subnormal step 2^-25 2^2e / W.  Some queries and keys are `big` times the
+    others, numerator and normalised."""
+    import kernels as K
+    q, k, v = rand_qkv(B, H, N, d, dv, seed=N + d, dtype=torch.float32, scale_qk=0.7)
+    q[:, :, 5::7] *= big
+    k[:, :, 3::11] *= big
+    q, k, v = (x.bfloat16() for x in (q, k, v))
+    c = 1.0 / math.sqrt(d)
+    qd, kd, vd = (x.cuda() for x in (q, k, v))
+    y = K.based_chunked(qd, kd, vd, out_dtype=torch.float32)
+    num = K.based_chunked(qd, kd, vd, normalize=False, out_dtype=torch.float32)
+    heads = slice(0, 2)          # the oracle's N x N in 64 bits: two heads of the last batch
+    q, k, v = (x[-1:, heads].double() for x in (q, k, v))
+    s = c * q @ k.transpose(-2, -1)
+    r, one = torch.tril(s + 0.5 * s * s), torch.tril(torch.ones(N, N, dtype=torch.float64))
+    d64, n64 = (r + one).sum(-1, keepdim=True), (r + one) @ v
+    reach = c * q.abs().sum(-1, keepdim=True) * k.abs().max()     # bound on |s|
+    # u = W r, W >= 0.18, in units of 2^2e <= (reach / c qscale / 64)^2; 1 / (c qscale) <= 1.2 by W
+    step = 2.0 ** -25 / 0.18 * (1.0 + (1.2 * reach / 64) ** 2) * one
+    rel = 2.0 ** -11 + 2.0 ** -13
+    en = (rel * r.abs() + step) @ v.abs() + (N + 64) * 2.0 ** -23 * ((r.abs() + one) @ v.abs())
+    ed = (rel * r.abs() + step).sum(-1, keepdim=True) + N * 2.0 ** -23 * (r.abs() + one).sum(-1, keepdim=True)
+    off = ((num[-1:, heads].double().cpu() - n64).abs() / en).max().item()
+    assert off < 1, off
+    y64 = n64 / (d64 + 1e-6)
+    off = ((y[-1:, heads].double().cpu() - y64).abs() / ((en + y64.abs() * ed) / d64)).max().item()
+    assert off < 1.01, off

@@ -843,6 +843,28 @@ size_t parallel_workspace_bytes(int BH, int N, int d, int dv, bool in_f32) {
 
 int launch_based_parallel_fp32(const ParallelArgs& a, hipStream_t stream);
 
+WideScale parallel_scale(float scale) {
+  // Work in u'' = 2^-2k u with u = (q.k + 1/c)^2 - 1/c^2 = (2/c^2) r, k chosen so that the weight
+  // of "1", W = 2^-2k * 2/c^2, lies in (0.18, 0.71] (u'' = W r): r up to 65504 / W stays inside
+  // fp16 (|s| up to ~430, 511 at scale = 1/4, where W = 1/2 and 1/c scales to 1/2).
+  const double ic = 1.0 / (double)scale;
+  const int k = (int)__builtin_lround(0.5 * __builtin_log2(2.0 * ic * ic) + 0.75);
+  const double qs = __builtin_ldexp(1.0, -k);
+  const float icf = (float)(ic * qs);
+  const double w = 2.0 * (double)icf * (double)icf;   // weight of "1" in u'' units
+  const _Float16 whi = (_Float16)w;
+  const _Float16 wlo = (_Float16)(w - (double)whi);
+  const u32 hb = __builtin_bit_cast(uint16_t, whi), lb = __builtin_bit_cast(uint16_t, wlo);
+  WideScale r{};
+  r.qscale = (float)qs;
+  r.inv_c = icf;
+  r.inv_c2 = (float)((double)icf * (double)icf);
+  r.fscale = (float)(1.0 / w);
+  r.ones_hi = hb | (hb << 16);
+  r.ones_lo = ((double)wlo == 0.0) ? 0u : (lb | (lb << 16));
+  return r;
+}
+
 int launch_based_parallel(const ParallelArgs& a, hipStream_t stream) {
   if (a.in_f32) return (a.stages & 2) ? launch_based_parallel_fp32(a, stream) : 0;
   ParallelParams p{};
@@ -862,23 +884,13 @@ int launch_based_parallel(const ParallelArgs& a, hipStream_t stream) {
   p.d = a.d;
   p.dv = a.dv;
   p.xcd_cus = device_cu_count() / 8;
-  // Work in u'' = 2^-2k u with u = (q.k + 1/c)^2 - 1/c^2 = (2/c^2) r, k chosen so that the weight
-  // of "1", W = 2^-2k * 2/c^2, lies in (0.18, 0.71] (u'' = W r): r up to 65504 / W stays inside
-  // fp16 (|s| up to ~430, 511 at scale = 1/4, where W = 1/2 and 1/c scales to 1/2).
-  const double ic = 1.0 / (double)a.scale;
-  const int k = (int)__builtin_lround(0.5 * __builtin_log2(2.0 * ic * ic) + 0.75);
-  const double qs = __builtin_ldexp(1.0, -k);
-  const float icf = (float)(ic * qs);
-  p.qscale = (float)qs;
-  p.inv_c = icf;
-  p.inv_c2 = (float)((double)icf * (double)icf);
-  const double w = 2.0 * (double)icf * (double)icf;   // weight of "1" in u'' units
-  p.fscale = (float)(1.0 / w);
-  const _Float16 whi = (_Float16)w;
-  const _Float16 wlo = (_Float16)(w - (double)whi);
-  const u32 hb = __builtin_bit_cast(uint16_t, whi), lb = __builtin_bit_cast(uint16_t, wlo);
-  p.ones_hi = hb | (hb << 16);
-  p.ones_lo = ((double)wlo == 0.0) ? 0u : (lb | (lb << 16));
+  const WideScale sc = parallel_scale(a.scale);
+  p.qscale = sc.qscale;
+  p.inv_c = sc.inv_c;
+  p.inv_c2 = sc.inv_c2;
+  p.fscale = sc.fscale;
+  p.ones_hi = sc.ones_hi;
+  p.ones_lo = sc.ones_lo;
   p.eps = a.eps;
   p.normalize = a.normalize ? 1 : 0;
   p.out_f32 = a.out_f32 ? 1 : 0;
@@ -902,8 +914,7 @@ int launch_based_parallel(const ParallelArgs& a, hipStream_t stream) {
     if (a.stages == 1)
       hipLaunchKernelGGL(vrange_kernel, dim3((unsigned)VR, (unsigned)a.BH), dim3(256), 0, stream, p.v, p.N, p.dv,
                          const_cast<u32*>(p.vmax));
-    const WideScale s{p.inv_c, p.inv_c2, p.fscale, p.qscale, p.ones_hi, p.ones_lo};
-    return launch_wide_parallel(a, static_cast<char*>(a.workspace) + vrange_bytes(a.BH), s, stream);
+    return launch_wide_parallel(a, static_cast<char*>(a.workspace) + vrange_bytes(a.BH), false, stream);
   }
   if (a.d <= 16) return dispatch_mt<1>(p, vec, packed, a.stages, stream);
   if (a.d <= 32) return dispatch_mt<2>(p, vec, false, a.stages, stream);

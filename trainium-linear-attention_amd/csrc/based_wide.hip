@@ -21,6 +21,9 @@
 // wave pairs share queries and take one 32-key half of every block each (their accumulators meet
 // in LDS at the end), so that the grid is twice as large at the same reads per MFMA.
 //
+// Chunked calls of the same shapes take these kernels too (chunked_general.hip), with scores of any
+// size (`any_range`: the pre-pass then also reads K for its largest magnitude per block).
+//
 // Measured (pre-pass + kernel, us; the register-staged kernel and its max pass before): B2 H16 d64 dv64
 // N2048 7 + 29 (5 + 62), N8192 14 + 252 (8 + 445): 1.04 PFLOP/s, matrix cores busy 57 % of the
 // cycles at the 1.9 GHz that the card holds under this load.  At N2048 20 of the 29 us are the loop
@@ -42,6 +45,7 @@ struct WideParams {
   uint16_t* vt;          // [BH][nb][32 MT rows][64] fp16
   float* sums;           // [BH][nb][32 MT] column sums of V
   int* eb;               // [BH][nb] V exponents
+  u32* kmx;              // optional [BH][nb]: largest finite |k| (bf16 bits); bounds |s| (any-range calls)
   void* out;
   float* den;
   int BH, N, d, dv, nqb, nb;
@@ -68,7 +72,7 @@ __global__ __launch_bounds__(256) void wide_pack_kernel(const WideParams p) {
   constexpr int DV = 32 * MT, CPR = DV / 8, IT = (32 * CPR + 255) / 256;
   __shared__ __attribute__((aligned(16))) uint16_t img[DV * BN];
   __shared__ float csum[32][DV + 1];
-  __shared__ u32 vmx[4];
+  __shared__ u32 vmx[4], kmxl[4];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int bh = blockIdx.x / p.nb, blk = blockIdx.x - bh * p.nb, dv = p.dv;
   const __amdgpu_buffer_rsrc_t rv = make_rsrc(p.v + (size_t)bh * p.N * dv, (u32)p.N * (u32)dv * 2u);
@@ -90,7 +94,23 @@ __global__ __launch_bounds__(256) void wide_pack_kernel(const WideParams p) {
     }
   m = wave_max_u32(m);
   if (lane == 0) vmx[w] = m;
+  if (p.kmx != nullptr) {   // rows of d % 8 == 0, contiguous
+    const __amdgpu_buffer_rsrc_t rk = make_rsrc(p.k + (size_t)bh * p.N * p.d, (u32)p.N * (u32)p.d * 2u);
+    u32 mk = 0u;
+    for (int x = tid; x < BN * p.d / 8; x += 256) {
+      const u32x4 y = buf_load_b128(rk, (blk * BN * p.d + 8 * x) * 2);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const u32 lo = y[i] & 0x7fffu, hi = (y[i] >> 16) & 0x7fffu;
+        mk = max(mk, max(lo < 0x7f80u ? lo : 0u, hi < 0x7f80u ? hi : 0u));
+      }
+    }
+    mk = wave_max_u32(mk);
+    if (lane == 0) kmxl[w] = mk;
+  }
   __syncthreads();
+  if (p.kmx != nullptr && tid == 0)
+    p.kmx[(size_t)bh * p.nb + blk] = max(max(kmxl[0], kmxl[1]), max(kmxl[2], kmxl[3]));
   const int eb = vexp_step(max(max(vmx[0], vmx[1]), max(vmx[2], vmx[3])) << 16);
 #pragma unroll
   for (int x = 0; x < IT; ++x) {
@@ -193,15 +213,48 @@ __global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
   // ---- exponents of the blocks this wave attends to
   const int* __restrict__ ebs = p.eb + (size_t)bh * p.nb;
   int emax = -128, emin = 1 << 20;
+  u32 km = 0u;
   if (live)
     for (int j = lane; j <= jd; j += 64) {
       const int e = ebs[j];
       emax = max(emax, e);
       emin = min(emin, e);
+      if (p.kmx != nullptr) km = max(km, p.kmx[(size_t)bh * p.nb + j]);
     }
   emax = (int)wave_max_u32((u32)(emax + 1024)) - 1024;
   emin = (1 << 21) - (int)wave_max_u32((u32)((1 << 21) - emin));
-  const bool mixed = live && emin != emax;
+  bool mixed = live && emin != emax;
+  // u in fp16 holds |s| up to about 430.  Any-range calls bound a query's |q.k| by its sum of |q| times
+  // the largest |k|, and a query whose bound is higher takes q, 1/c and W smaller by 2^-eq (u by
+  // 2^-2 eq); its wave then runs every block through `general`.
+  int eq[QT];
+#pragma unroll
+  for (int qt = 0; qt < QT; ++qt) eq[qt] = 0;
+  if (p.kmx != nullptr) {
+    const float kmax = __builtin_bit_cast(float, wave_max_u32(km) << 16);
+    bool far = false;
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) {
+      float l1 = 0.f;
+#pragma unroll
+      for (int kk = 0; kk < KS; ++kk)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          l1 += __builtin_fabsf(bf16_lo_to_f32(qf[qt][kk][e])) + __builtin_fabsf(bf16_hi_to_f32(qf[qt][kk][e]));
+      l1 += __shfl_xor(l1, 32);
+      // |b| = |q~ k + 1/c| <= 240 keeps u = b^2 - 1/c^2 below 57600
+      const float bound = l1 * kmax + p.inv_c;
+      if (!(bound <= 240.f)) {
+        int e;
+        (void)__builtin_frexpf(__builtin_fminf(bound, 3.0e38f) * (1.0f / 128.0f), &e);   // bound / 2^e <= 128; NaN and inf: the largest
+        eq[qt] = e;
+        far = true;
+#pragma unroll
+        for (int kk = 0; kk < KS; ++kk) qf[qt][kk] = scale_bf16x8(qf[qt][kk], __builtin_ldexpf(1.0f, -e));
+      }
+    }
+    if (__ballot(far) != 0ull) mixed = live;
+  }
   // ---- column sums of V over the blocks before each query group's diagonal block
   {
     constexpr int PARTS = 256 / DV, PF = 8;
@@ -307,27 +360,38 @@ __global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
     const int kb = BN * j + 32 * ks, e = mixed ? max(ebs[j] - emax, -126) : 0;
     u32x4 x[3][QT][2];   // u, then the mask times W's hi and lo parts (the exact 1 of p)
     bool act[QT];
-    f32x16 b[QT];
-    S(st, ks, b);
+    u32x4 kf[KS];
+#pragma unroll
+    for (int kk = 0; kk < KS; ++kk) kf[kk] = kfrag(st, ks, kk);
     const bool diag = j == jd;
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt) {
       const int qbase = wq0 + 32 * qt, query = qbase + n;
       act[qt] = kb <= qbase + 31 && qbase < N;
+      const float ic = __builtin_ldexpf(inv_c, -eq[qt]), ic2 = __builtin_ldexpf(inv_c2, -2 * eq[qt]);
+      u32 whi = p.ones_hi, wlo = p.ones_lo;
+      if (eq[qt] != 0) {
+        const float wq = __builtin_ldexpf(1.0f / p.fscale, -2 * eq[qt]);
+        whi = pack_f16x2(wq, wq);
+        wlo = pack_f16x2(wq - f16_lo_to_f32(whi), wq - f16_lo_to_f32(whi));
+      }
+      f32x16 b = splat16(ic);
+#pragma unroll
+      for (int kk = 0; kk < KS; ++kk) b = mfma32x32x16(kf[kk], qf[qt][kk], b);
 #pragma unroll
       for (int m = 0; m < 2; ++m)
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
           const int i = 8 * m + 2 * c, k0 = kb + c32_row(i, h);   // keys k0, k0 + 1
-          const float u0 = __builtin_fmaf(b[qt][i], b[qt][i], -inv_c2), u1 = __builtin_fmaf(b[qt][i + 1], b[qt][i + 1], -inv_c2);
+          const float u0 = __builtin_fmaf(b[i], b[i], -ic2), u1 = __builtin_fmaf(b[i + 1], b[i + 1], -ic2);
           const bool in0 = k0 <= query, in1 = k0 + 1 <= query;
           x[0][qt][m][c] = pack_f16x2(in0 ? u0 : 0.f, in1 ? u1 : 0.f);
-          x[1][qt][m][c] = (in0 ? p.ones_hi & 0xffffu : 0u) | (in1 ? p.ones_hi & 0xffff0000u : 0u);
-          x[2][qt][m][c] = (in0 ? p.ones_lo & 0xffffu : 0u) | (in1 ? p.ones_lo & 0xffff0000u : 0u);
+          x[1][qt][m][c] = (in0 ? whi & 0xffffu : 0u) | (in1 ? whi & 0xffff0000u : 0u);
+          x[2][qt][m][c] = (in0 ? wlo & 0xffffu : 0u) | (in1 ? wlo & 0xffff0000u : 0u);
           if (act[qt]) rsum[qt] = dot2_f16(x[0][qt][m][c], kOnes, rsum[qt]);
         }
     }
-    Pscaled(st, ks, x, !diag ? 1 : p.ones_lo != 0u ? 3 : 2, act, e);
+    Pscaled(st, ks, x, !diag ? 1 : p.ones_lo != 0u || p.kmx != nullptr ? 3 : 2, act, e);
   };
 
   // step s of this wave landed (NSR - 2 later ones may be in flight), then every wave's; every wave is
@@ -375,6 +439,7 @@ __global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
   const int e0 = NKH == 2 ? kh : 0;
   f32x16 fin[QE][MT];
   float rs[QE];
+  int ef[QE];   // the queries' exponents
   if constexpr (NKH == 2) {
     float* mine = reinterpret_cast<float*>(&ring[0][0]) + wv * ((16 * MT + 1) * 64) + lane;
     float* other = reinterpret_cast<float*>(&ring[0][0]) + (wv ^ 1) * ((16 * MT + 1) * 64) + lane;
@@ -389,11 +454,13 @@ __global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) fin[0][mt][r] = (kh ? acc[1][mt][r] : acc[0][mt][r]) + other[(16 * mt + r) * 64];
     rs[0] = (kh ? rsum[1] : rsum[0]) + other[16 * MT * 64];
+    ef[0] = kh ? eq[1] : eq[0];
     __syncthreads();   // read before the output tiles take their place
   } else {
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt) {
       rs[qt] = rsum[qt];
+      ef[qt] = eq[qt];
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) fin[qt][mt] = acc[qt][mt];
     }
@@ -412,9 +479,10 @@ __global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
     for (int qe = 0; qe < QE; ++qe) {
       const int qbase = wq0 + 32 * (e0 + qe), query = qbase + n;
       const float r2 = rs[qe] + __shfl_xor(rs[qe], 32);
-      const float den = (float)(query + 1) + fscale * r2;
+      const float den = (float)(query + 1) + __builtin_ldexpf(fscale * r2, 2 * ef[qe]);
       const float inv = p.normalize ? 1.0f / (den + p.eps) : 1.0f;
       if (p.den != nullptr && h == 0 && query < N) p.den[hrow + query] = den;
+      const float aq = __builtin_ldexpf(afs, 2 * ef[qe]);
 #pragma unroll
       for (int ct = 0; ct < MT; ct += CT) {
 #pragma unroll
@@ -424,7 +492,7 @@ __global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
             float y[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-              y[e] = (afs * fin[qe][ct + mt][4 * g + e] + vsl[qg][32 * (ct + mt) + 8 * g + 4 * h + e]) * inv;
+              y[e] = (aq * fin[qe][ct + mt][4 * g + e] + vsl[qg][32 * (ct + mt) + 8 * g + 4 * h + e]) * inv;
             char* dst = tile + n * RS + (32 * mt + 8 * g + 4 * h) * EB;
             if (F32)
               *reinterpret_cast<f32x4*>(dst) = (f32x4){y[0], y[1], y[2], y[3]};
@@ -491,10 +559,11 @@ bool wide_shape(int N, int d, int dv) {
 
 size_t wide_workspace_bytes(int BH, int N, int dv) {
   const size_t nb = ((size_t)N + BN - 1) / BN, DV = 32 * mt_of(dv);
-  return up256(BH * nb * DV * BN * 2) + up256(BH * nb * DV * 4) + up256(BH * nb * 4);
+  return up256(BH * nb * DV * BN * 2) + up256(BH * nb * DV * 4) + 2 * up256(BH * nb * 4);
 }
 
-int launch_wide_parallel(const ParallelArgs& a, void* workspace, const WideScale& s, hipStream_t stream) {
+int launch_wide_parallel(const ParallelArgs& a, void* workspace, bool any_range, hipStream_t stream) {
+  const WideScale s = parallel_scale(a.scale);
   WideParams p{};
   p.q = static_cast<const uint16_t*>(a.q);
   p.k = static_cast<const uint16_t*>(a.k);
@@ -511,6 +580,7 @@ int launch_wide_parallel(const ParallelArgs& a, void* workspace, const WideScale
   p.vt = reinterpret_cast<uint16_t*>(ws);
   p.sums = reinterpret_cast<float*>(ws + up256(blocks * DV * BN * 2));
   p.eb = reinterpret_cast<int*>(ws + up256(blocks * DV * BN * 2) + up256(blocks * DV * 4));
+  p.kmx = any_range ? reinterpret_cast<u32*>(reinterpret_cast<char*>(p.eb) + up256(blocks * 4)) : nullptr;
   p.inv_c = s.inv_c;
   p.inv_c2 = s.inv_c2;
   p.fscale = s.fscale;

@@ -901,6 +901,37 @@ int launch_general_chunked(const ChunkedArgs& a, hipStream_t stream) {
   if (!general_chunked_shape(a.d, a.dv, a.in_f32)) return LA_ERR_UNSUPPORTED_DIM;
   if (a.in_f32) return launch_general_chunked_f32(a, stream);
   const int DP = dp_of(a.d), DVT = dvt_of(a.dv);
+  // Sequences of several segments up to kWideMax tokens run the parallel kernel on the whole sequence
+  // (its work grows with N^2, this path's with N, but at about five times the rate per operation): us,
+  // this path / parallel: B2 H16 d64 dv64 N1024 102 / 23, N8192 428 / 264, N16384 868 / 953; d32 dv64
+  // N8192 297 / 216; B1 H4 N16384 141 / 139; B2 H16 d16 dv128 N4096 190 / 106, N8192 339 / 338; d64 dv128
+  // N8192 1035 / 422.  One segment keeps this path: no workspace, one launch.
+  {
+    const int kWideMax = DP == 16 ? 8192 : 12288;
+    const size_t need = general_chunked_bytes(a.BH, a.N, a.d, a.dv, false);
+    if (a.N > GL && a.N <= kWideMax && wide_shape(a.N, a.d, a.dv) && wide_workspace_bytes(a.BH, a.N, a.dv) <= need &&
+        ((reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.k) | reinterpret_cast<uintptr_t>(a.v) |
+          reinterpret_cast<uintptr_t>(a.out)) & 15) == 0) {
+      if (a.workspace == nullptr || a.workspace_bytes < need) return LA_ERR_WORKSPACE;
+      if (reinterpret_cast<uintptr_t>(a.workspace) & 15) return LA_ERR_BAD_ALIGNMENT;
+      ParallelArgs w{};
+      w.q = a.q;
+      w.k = a.k;
+      w.v = a.v;
+      w.out = a.out;
+      w.den = a.den_out;
+      w.stages = 3;
+      w.BH = a.BH;
+      w.N = a.N;
+      w.d = a.d;
+      w.dv = a.dv;
+      w.scale = a.scale;
+      w.eps = a.eps;
+      w.normalize = a.normalize;
+      w.out_f32 = a.out_f32;
+      return launch_wide_parallel(w, a.workspace, true, stream);
+    }
+  }
   GParams p{};
   p.q = static_cast<const uint16_t*>(a.q);
   p.k = static_cast<const uint16_t*>(a.k);

@@ -105,16 +105,18 @@ int f32_split_slots(int BH, int N);                         // fp32 key split: s
 int f32_x6_split_parts(int BH, int N, int d, int dv);       // fp32 three-term key split: parts, or 0
 size_t f32_split_workspace_bytes(int BH, int N, int d, int dv);   // partials of either split (or 0)
 bool parallel_packed_shape(int d, int dv, bool in_f32);   // shapes of the packed (pre-pass) kernel
-// Scalars of the parallel bf16 kernels (launch_based_parallel derives them from the scale).
+// Scalars of the parallel bf16 kernels for a scale (based_parallel.hip).
 struct WideScale {
   float inv_c, inv_c2, fscale, qscale;
   uint32_t ones_hi, ones_lo;
 };
+WideScale parallel_scale(float scale);
 // Parallel kernel for bf16 head dims other than the packed one's (based_wide.hip); needs 16-byte
 // aligned tensors.
 bool wide_shape(int N, int d, int dv);
 size_t wide_workspace_bytes(int BH, int N, int dv);
-int launch_wide_parallel(const ParallelArgs& a, void* workspace, const WideScale& s, hipStream_t stream);
+// any_range: |s| of any size (the packed and register-staged kernels hold up to about 430).
+int launch_wide_parallel(const ParallelArgs& a, void* workspace, bool any_range, hipStream_t stream);
 int launch_sliding_window(const SlidingArgs& a, hipStream_t stream);
 size_t chunked_workspace_bytes(int BH, int N, int d, int dv, int chunk);
 int chunked_chunk_tokens();   // tokens per chunk of the chunked kernels
