@@ -113,3 +113,29 @@ def test_split_rows_match_one_group_per_head(B, H, d, dv):
         torch.cuda.synchronize()
         assert torch.equal(st_one, st_split)
         assert err(y_split, y_one.cpu()) < 1e-4   # the fp32 bar (2145-term sums at d = 64)
+
+
+@pytest.mark.parametrize("B,H,d,dv", [(1, 1, 1, 1), (1, 2, 4, 16), (2, 1, 16, 17), (1, 3, 16, 32), (1, 1, 16, 33), (40, 16, 16, 64),
+                                      (1, 1, 16, 65), (1, 2, 17, 64), (9, 3, 40, 100), (1, 1, 64, 128), (260, 1, 24, 128)])
+def test_rows_and_columns(B, H, d, dv):
+    """Edges of the row sweep (16, 32, 64 or 2 x 64 lanes a row, four or eight waves, split heads or
+    not): the state is the fp32 sum rounded once (phi(k) has roundings of its own); the output is off its 64-bit value by at
+    most (rows 2^-24 + 2^-21) times its terms (phi has three roundings)."""
+    import kernels as K
+    F = 1 + d + d * (d + 1) // 2
+    g = torch.Generator().manual_seed(d * 131 + dv)
+    st = torch.randn(B, H, F, dv + 1, generator=g)
+    st[..., dv] = st[..., dv].abs() + 1
+    q, k = (torch.randn(B, H, d, generator=g).abs() for _ in range(2))
+    v = torch.randn(B, H, dv, generator=g)
+    sd = st.cuda()
+    y = K.based_decode_step(q.cuda(), k.cuda(), v.cuda(), sd)
+    pq, pk = (K.taylor_feature_map(x.cuda()).cpu().double() for x in (q, k))
+    vx = torch.cat([v, torch.ones(B, H, 1)], -1).double()
+    new = st.double() + pk.unsqueeze(-1) * vx.unsqueeze(-2)
+    assert float(((sd.cpu().double() - new).abs() / (new.abs() * 2.0 ** -24 + (pk.unsqueeze(-1) * vx.unsqueeze(-2)).abs() * 2.0 ** -22 + 1e-30)).max()) <= 1.01
+    num, den = (pq.unsqueeze(-2) @ new)[..., 0, :dv], (pq.unsqueeze(-2) @ new)[..., 0, dv:]
+    want = num / (den + 1e-6)
+    mag = (pq.unsqueeze(-2) @ new.abs())[..., 0, :dv]
+    bound = 2 * (F * 2.0 ** -24 + 2.0 ** -21) * (mag + want.abs() * den) / den
+    assert float(((y.cpu().double() - want).abs() / bound).max()) < 1

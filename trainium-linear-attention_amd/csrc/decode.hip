@@ -10,17 +10,20 @@
 // token (its intra-chunk term phi(q).phi(k) v is the contribution of the token's own row of the
 // update).  The reference has no decode path; this continues a prefill that exported its state.
 //
-// A head whose state fits in LDS (F (dv + 1) <= 10240 floats) runs in one 1024-thread
-// work-group that loads the whole state at once (based_decode_wide_kernel).  Otherwise a
-// head's F state rows are split into R groups of consecutive rows, one work-group each: phi(q)
-// and phi(k) of the group's rows go to LDS, then the group's rows are swept linearly
-// (coalesced) in tiles of 32 rows, each element updated in place, and the column sums of phi(q)
-// times the updated state are taken per tile through LDS in row order.  With R = 1 the
-// work-group normalises and stores the output itself; with R > 1 it stores its column sums to
-// a workspace and a combine kernel adds the R partial sums of every column in group order
-// (deterministic) and normalises.  R is chosen so that small batches still launch enough
-// work-groups to cover the chip.  HBM-bound: the state is read and written once
-// (4 F (dv + 1) bytes each way per head).
+// A head's F state rows are one work-group's, or R groups of consecutive rows, one work-group
+// each, when the heads alone are too few.  A wave takes whole rows, a lane the same column of
+// each, so a row is one coalesced load and store, phi(q) and phi(k) of the row are LDS broadcasts,
+// the column sums stay in registers and no element needs its row or column worked out.  The loads
+// of a work-group's rows (up to 20 per lane) are issued before anything else.  With R = 1 the
+// work-group adds its waves' column sums in wave order, normalises and stores the output itself;
+// with R > 1 it stores them to a workspace and a combine kernel adds the R partial sums of every
+// column in group order (deterministic) and normalises.
+//
+// HBM-bound in large batches: the state is read and written once (4 F (dv + 1) bytes each way per
+// head).  Whole calls, us (a sweep by linear element index, with a division per element, products
+// through LDS and one tile of loads at a time / this): B64 H16 d16 dv64 27.0 / 18.2 (4.5 TB/s), dv128
+// 41.3 / 30.1, B64 H16 d64 dv64 498 / 260 (4.4 TB/s), B16 H16 d64 136 / 72; B2 H16 d16 dv64 8.4 / 7.1 on
+// the device (launch and two memory latencies).
 #include <math.h>
 
 #include <algorithm>
@@ -39,7 +42,7 @@ struct DecodeParams {
   float* state;
   void* out;
   int BH, d, dv, F;
-  float eps;
+  float eps, r4, rsq, rd;   // d^(-1/4), 1 / sqrt(2 d), 1 / sqrt(d)
   int normalize, in_f32, out_f32;
 };
 
@@ -47,11 +50,11 @@ constexpr int kDecThreads = 256;
 constexpr int kDecMaxD = 64;
 constexpr int kDecMaxC = 129;   // dv + 1 for dv <= 128
 constexpr int kDecMaxF = 1 + kDecMaxD + kDecMaxD * (kDecMaxD + 1) / 2;
-constexpr int kDecRows = 32;    // state rows per reduction tile
 constexpr int kDecMinRows = 8;  // fewest state rows per work-group when a head is split
-constexpr int kWideThreads = 1024;
-constexpr int kWideMaxElems = 10240;   // F (dv + 1) state floats of one head held in LDS (40 KB)
-constexpr int kWidePer = kWideMaxElems / kWideThreads;
+constexpr int kDecLoads = 20;   // state elements of a lane in flight
+// States of at most this many floats per head (40 KB; d = 16 with dv <= 65) stay with one
+// work-group: the second launch of a split costs as much as it saves.
+constexpr int kOneGroupElems = 10240;
 #ifndef LA_DECODE_TARGET_WGS
 #define LA_DECODE_TARGET_WGS 1024   // split heads until about this many work-groups launch
 #endif
@@ -68,136 +71,119 @@ __device__ __forceinline__ float feature(const float* x, int f, int d, float r4,
     const float t = x[f - 1 - d];
     return t * t * rsq;
   }
-  int t = f - 1 - 2 * d, i = 0;
-  while (t >= d - 1 - i) {   // row i of the strict upper triangle holds d - 1 - i pairs
-    t -= d - 1 - i;
-    ++i;
-  }
-  return x[i] * x[i + 1 + t] * rd;
+  // pair t of the strict upper triangle: row i starts at i (2 d - i - 1) / 2
+  const int t = f - 1 - 2 * d;
+  const float b = (float)(2 * d - 1);
+  int i = (int)((b - __builtin_sqrtf(b * b - 8.0f * (float)t)) * 0.5f);
+  while (i > 0 && i * (2 * d - i - 1) / 2 > t) --i;
+  while ((i + 1) * (2 * d - i - 2) / 2 <= t) ++i;
+  return x[i] * x[i + 1 + t - i * (2 * d - i - 1) / 2] * rd;
 }
 
-// Rows [g RW, min(F, (g + 1) RW)) of head bh = blockIdx.x, g = blockIdx.y.  PARTIAL: store
-// the group's column sums to part[(bh R + g) C + c]; else (R = 1) normalise and store the output.
-template <bool PARTIAL>
-__global__ __launch_bounds__(kDecThreads) void based_decode_kernel(const DecodeParams p, int RW, float* part) {
-  __shared__ float xq[kDecMaxD], xk[kDecMaxD], vv[kDecMaxC];
+__device__ __forceinline__ float wave_sum(float x) {
+#pragma unroll
+  for (int m = 1; m < 64; m <<= 1) x += __shfl_xor(x, m);
+  return x;
+}
+
+// Rows [g RW, min(F, (g + 1) RW)) of head bh = blockIdx.x, g = blockIdx.y.  LPR lanes per row, CPL
+// columns per lane (LPR CPL >= dv), NW waves.  PARTIAL: store the group's column sums to
+// part[(bh R + g) C + c]; else (R = 1) normalise and store the output.
+template <int LPR, int CPL, int NW, bool PARTIAL>
+__global__ __launch_bounds__(64 * NW) void based_decode_kernel(const DecodeParams p, int RW, float* part) {
+  constexpr int NT = 64 * NW, RPW = 64 / LPR;          // rows per load of a wave
+  constexpr int PF = kDecLoads / CPL / 2, WR = PF * RPW, BR = NW * WR;   // rows per wave and block batch
+  static_assert(WR <= 64, "a lane per row for the K-sum column");
+  __shared__ float xq[kDecMaxD], xk[kDecMaxD];
   __shared__ float phq[kDecMaxF], phk[kDecMaxF];
-  __shared__ float tile[kDecRows * kDecMaxC];
-  const int bh = blockIdx.x, g = blockIdx.y, tid = threadIdx.x;
+  __shared__ float red[NW][LPR * CPL], zred[NW];
+  const int bh = blockIdx.x, g = blockIdx.y, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int d = p.d, dv = p.dv, F = p.F, C = dv + 1;
-  const int rb = g * RW, re = min(F, rb + RW);
-  if (tid < d) {
-    xq[tid] = load_elem(p.q, (size_t)bh * d + tid, p.in_f32);
-    xk[tid] = load_elem(p.k, (size_t)bh * d + tid, p.in_f32);
-  }
-  if (tid < dv) vv[tid] = load_elem(p.v, (size_t)bh * dv + tid, p.in_f32);
-  if (tid == 0) vv[dv] = 1.f;
+  const int rb = g * RW, re = min(F, rb + RW), rows = re - rb;
+  const int col = lane % LPR, r0 = w * WR;
+  float* __restrict__ st = p.state + (size_t)bh * F * C + (size_t)rb * C;
+
+  // A wave takes WR consecutive rows at a time and lane l < WR the K-sum entry of row l, so that the
+  // lines between two rows are touched once (the K-sum column in a pass of its own, or rows dealt out
+  // one by one, cost HBM a second read and write of those lines).  Two register sets: while one is
+  // updated and stored the other's loads are in flight.
+  float s[2][PF][CPL], z[2];
+  auto load = [&](int set, int first) {
+#pragma unroll
+    for (int i = 0; i < PF; ++i)
+#pragma unroll
+      for (int c = 0; c < CPL; ++c) {
+        const int r = first + RPW * i + lane / LPR;
+        s[set][i][c] = r < rows && col + LPR * c < dv ? st[(size_t)r * C + col + LPR * c] : 0.f;
+      }
+    z[set] = lane < WR && first + lane < rows ? st[(size_t)(first + lane) * C + dv] : 0.f;
+  };
+  load(0, r0);
+  load(1, r0 + BR);
+  float v[CPL];
+#pragma unroll
+  for (int c = 0; c < CPL; ++c) v[c] = col + LPR * c < dv ? load_elem(p.v, (size_t)bh * dv + col + LPR * c, p.in_f32) : 0.f;
+  if (tid < d) xq[tid] = load_elem(p.q, (size_t)bh * d + tid, p.in_f32);
+  if (tid >= NT - d) xk[tid - (NT - d)] = load_elem(p.k, (size_t)bh * d + tid - (NT - d), p.in_f32);
   __syncthreads();
-  const float rd = 1.0f / sqrtf((float)d), r4 = sqrtf(rd), rsq = rd * 0.70710678118654752f;
-  for (int f = rb + tid; f < re; f += kDecThreads) {
-    phq[f - rb] = feature(xq, f, d, r4, rsq, rd);
-    phk[f - rb] = feature(xk, f, d, r4, rsq, rd);
+  for (int f = tid; f < rows; f += NT) {
+    phq[f] = feature(xq, rb + f, d, p.r4, p.rsq, p.rd);
+    phk[f] = feature(xk, rb + f, d, p.r4, p.rsq, p.rd);
   }
   __syncthreads();
 
-  // The rows sweep linearly (coalesced) in tiles of kDecRows rows: every element is updated in
-  // place and its phi(q)-weighted value parked in LDS, then thread c < C adds the tile's column
-  // c in row order.
-  float* __restrict__ st = p.state + (size_t)bh * F * C;
-  float colsum = 0.f;
-  for (int r0 = rb; r0 < re; r0 += kDecRows) {
-    const int ne = min(kDecRows, re - r0) * C;
-    float* __restrict__ base = st + (size_t)r0 * C;
-    const float* pk = phk + (r0 - rb);
-    const float* pq = phq + (r0 - rb);
-    for (int e = tid; e < ne; e += kDecThreads) {
-      const int fr = e / C, c = e - fr * C;
-      const float s = __builtin_fmaf(pk[fr], vv[c], base[e]);
-      base[e] = s;
-      tile[e] = pq[fr] * s;
+  float sum[CPL], zsum = 0.f;
+#pragma unroll
+  for (int c = 0; c < CPL; ++c) sum[c] = 0.f;
+  auto update = [&](int set, int first) {
+#pragma unroll
+    for (int i = 0; i < PF; ++i) {
+      const int r = first + RPW * i + lane / LPR;
+      if (r >= rows) break;
+      const float a = phk[r], b = phq[r];
+#pragma unroll
+      for (int c = 0; c < CPL; ++c) {
+        const float y = __builtin_fmaf(a, v[c], s[set][i][c]);
+        if (col + LPR * c < dv) st[(size_t)r * C + col + LPR * c] = y;
+        sum[c] = __builtin_fmaf(b, y, sum[c]);
+      }
     }
-    __syncthreads();
-    if (tid < C)
-      for (int e = tid; e < ne; e += C) colsum += tile[e];
-    __syncthreads();
+    if (lane < WR && first + lane < rows) {
+      const float y = phk[first + lane] + z[set];
+      st[(size_t)(first + lane) * C + dv] = y;
+      zsum = __builtin_fmaf(phq[first + lane], y, zsum);
+    }
+  };
+  for (int first = r0; first < rows; first += 2 * BR) {
+    update(0, first);
+    if (first + 2 * BR < rows) load(0, first + 2 * BR);
+    update(1, first + BR);
+    if (first + 3 * BR < rows) load(1, first + 3 * BR);
   }
+  // column sums: the rows of a wave, then the waves in order
+#pragma unroll
+  for (int c = 0; c < CPL; ++c) {
+#pragma unroll
+    for (int m = LPR; m < 64; m <<= 1) sum[c] += __shfl_xor(sum[c], m);
+    if (lane < LPR) red[w][lane + LPR * c] = sum[c];
+  }
+  zsum = wave_sum(zsum);
+  if (lane == 0) zred[w] = zsum;
+  __syncthreads();
+  float num = 0.f, den = 0.f;
+  if (tid < dv)
+#pragma unroll
+    for (int x = 0; x < NW; ++x) num += red[x][tid];
+#pragma unroll
+  for (int x = 0; x < NW; ++x) den += zred[x];
   if (PARTIAL) {
-    if (tid < C) part[((size_t)bh * gridDim.y + g) * C + tid] = colsum;
+    float* o = part + ((size_t)bh * gridDim.y + g) * C;
+    if (tid < dv) o[tid] = num;
+    if (tid == dv) o[dv] = den;
     return;
   }
-  __shared__ float den;
-  if (tid == dv) den = colsum;
-  __syncthreads();
   if (tid < dv) {
-    const float y = p.normalize ? colsum / (den + p.eps) : colsum;
-    const size_t o = (size_t)bh * dv + tid;
-    if (p.out_f32)
-      static_cast<float*>(p.out)[o] = y;
-    else
-      static_cast<uint16_t*>(p.out)[o] = f32_to_bf16_bits(y);
-  }
-}
-
-// Heads whose whole state fits in LDS (F (dv + 1) <= kWideMaxElems): one work-group of
-// kWideThreads per head.  Every state element of the head is loaded at the start (one memory
-// latency instead of one per tile), updated in place, and its phi(q)-weighted value parked in
-// LDS; thread (segment, c) then adds rows [segment RS, (segment + 1) RS) of column c in row order
-// and thread c adds the segments in order (deterministic).
-__global__ __launch_bounds__(kWideThreads) void based_decode_wide_kernel(const DecodeParams p) {
-  __shared__ float xq[kDecMaxD], xk[kDecMaxD], vv[kDecMaxC];
-  __shared__ float phq[kDecMaxF], phk[kDecMaxF];
-  __shared__ float tile[kWideMaxElems];
-  __shared__ float part[kWideThreads];
-  __shared__ float den;
-  const int bh = blockIdx.x, tid = threadIdx.x;
-  const int d = p.d, dv = p.dv, F = p.F, C = dv + 1, FC = F * C;
-  float* __restrict__ st = p.state + (size_t)bh * FC;
-  float pre[kWidePer];
-#pragma unroll
-  for (int i = 0; i < kWidePer; ++i) {
-    const int e = tid + kWideThreads * i;
-    pre[i] = e < FC ? st[e] : 0.f;
-  }
-  if (tid < d) {
-    xq[tid] = load_elem(p.q, (size_t)bh * d + tid, p.in_f32);
-    xk[tid] = load_elem(p.k, (size_t)bh * d + tid, p.in_f32);
-  }
-  if (tid < dv) vv[tid] = load_elem(p.v, (size_t)bh * dv + tid, p.in_f32);
-  if (tid == 0) vv[dv] = 1.f;
-  __syncthreads();
-  const float rd = 1.0f / sqrtf((float)d), r4 = sqrtf(rd), rsq = rd * 0.70710678118654752f;
-  for (int f = tid; f < F; f += kWideThreads) {
-    phq[f] = feature(xq, f, d, r4, rsq, rd);
-    phk[f] = feature(xk, f, d, r4, rsq, rd);
-  }
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < kWidePer; ++i) {
-    const int e = tid + kWideThreads * i;
-    if (e < FC) {
-      const int fr = e / C, c = e - fr * C;
-      const float s = __builtin_fmaf(phk[fr], vv[c], pre[i]);
-      st[e] = s;
-      tile[e] = phq[fr] * s;
-    }
-  }
-  __syncthreads();
-  const int NS = kWideThreads / C, RS = (F + NS - 1) / NS;
-  const int seg = tid / C, col = tid - seg * C;
-  if (seg < NS) {
-    float r = 0.f;
-    const int r1 = min(F, (seg + 1) * RS);
-    for (int f = seg * RS; f < r1; ++f) r += tile[f * C + col];
-    part[seg * C + col] = r;
-  }
-  __syncthreads();
-  float colsum = 0.f;
-  if (tid < C)
-    for (int sg = 0; sg < NS; ++sg) colsum += part[sg * C + tid];
-  if (tid == dv) den = colsum;
-  __syncthreads();
-  if (tid < dv) {
-    const float y = p.normalize ? colsum / (den + p.eps) : colsum;
+    const float y = p.normalize ? num / (den + p.eps) : num;
     const size_t o = (size_t)bh * dv + tid;
     if (p.out_f32)
       static_cast<float*>(p.out)[o] = y;
@@ -252,14 +238,31 @@ static void decode_groups(long long BH, int d, int& R, int& RW) {
   R = (F + RW - 1) / RW;
 }
 
-static bool decode_wide(int d, int dv) { return (1 + d + d * (d + 1) / 2) * (dv + 1) <= kWideMaxElems; }
+static bool decode_one_group(int d, int dv) { return (1 + d + d * (d + 1) / 2) * (dv + 1) <= kOneGroupElems; }
 
 size_t decode_workspace_bytes(long long BH, int d, int dv) {
-  if (decode_wide(d, dv)) return 0;
+  if (decode_one_group(d, dv)) return 0;
   int R, RW;
   decode_groups(BH, d, R, RW);
   return R > 1 ? (size_t)BH * R * (dv + 1) * sizeof(float) : 0;
 }
+
+namespace {
+
+template <int NW, bool PARTIAL>
+void launch_rows(const DecodeParams& p, int R, int RW, float* part, hipStream_t stream) {
+  const dim3 grid((unsigned)p.BH, (unsigned)R), block(64 * NW);
+  if (p.dv <= 16)
+    hipLaunchKernelGGL((based_decode_kernel<16, 1, NW, PARTIAL>), grid, block, 0, stream, p, RW, part);
+  else if (p.dv <= 32)
+    hipLaunchKernelGGL((based_decode_kernel<32, 1, NW, PARTIAL>), grid, block, 0, stream, p, RW, part);
+  else if (p.dv <= 64)
+    hipLaunchKernelGGL((based_decode_kernel<64, 1, NW, PARTIAL>), grid, block, 0, stream, p, RW, part);
+  else
+    hipLaunchKernelGGL((based_decode_kernel<64, 2, NW, PARTIAL>), grid, block, 0, stream, p, RW, part);
+}
+
+}  // namespace
 
 int launch_decode_step(const DecodeArgs& a, hipStream_t stream) {
   DecodeParams p{};
@@ -273,22 +276,25 @@ int launch_decode_step(const DecodeArgs& a, hipStream_t stream) {
   p.dv = a.dv;
   p.F = 1 + a.d + a.d * (a.d + 1) / 2;
   p.eps = a.eps;
+  p.rd = 1.0f / sqrtf((float)a.d);
+  p.r4 = sqrtf(p.rd);
+  p.rsq = p.rd * 0.70710678118654752f;
   p.normalize = a.normalize ? 1 : 0;
   p.in_f32 = a.in_f32 ? 1 : 0;
   p.out_f32 = a.out_f32 ? 1 : 0;
-  if (decode_wide(a.d, a.dv)) {
-    hipLaunchKernelGGL(based_decode_wide_kernel, dim3((unsigned)a.BH), dim3(kWideThreads), 0, stream, p);
-    return (int)hipGetLastError();
-  }
   int R = 1, RW = p.F;
-  if (a.workspace != nullptr) decode_groups(a.BH, a.d, R, RW);
+  if (a.workspace != nullptr && !decode_one_group(a.d, a.dv)) decode_groups(a.BH, a.d, R, RW);
   if (R == 1) {
-    hipLaunchKernelGGL(based_decode_kernel<false>, dim3((unsigned)a.BH, 1), dim3(kDecThreads), 0, stream, p, RW,
-                       static_cast<float*>(nullptr));
+    // four waves per work-group where heads fill the chip (B64 H16 d16 dv64, with one register set: 20.1
+    // us, eight 21.5, sixteen 29.1), eight where their latency counts or rows have 128 columns (B64 H16
+    // dv128 32.2 us, 33.0 with four)
+    if (a.dv <= 64 && a.BH > device_cu_count())
+      launch_rows<4, false>(p, 1, RW, nullptr, stream);
+    else
+      launch_rows<8, false>(p, 1, RW, nullptr, stream);
   } else {
     float* part = static_cast<float*>(a.workspace);
-    hipLaunchKernelGGL(based_decode_kernel<true>, dim3((unsigned)a.BH, (unsigned)R), dim3(kDecThreads), 0, stream,
-                       p, RW, part);
+    launch_rows<4, true>(p, R, RW, part, stream);
     hipLaunchKernelGGL(decode_combine_kernel, dim3((unsigned)a.BH), dim3(kDecThreads), 0, stream, p, R,
                        static_cast<const float*>(part));
   }
