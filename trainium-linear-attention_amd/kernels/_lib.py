@@ -138,7 +138,13 @@ def ptr(t) -> int:
     return 0 if t is None else t.data_ptr()
 
 
+# torch's current stream as a handle, without the Stream object around it (0.1 against 1.9 us a call)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_of(t: torch.Tensor) -> int:
+    if _raw_stream is not None:
+        return _raw_stream(t.get_device())
     return torch.cuda.current_stream(t.device).cuda_stream
 
 
