@@ -786,13 +786,16 @@ int launch_packed(const ParallelParams& pp, int stages, hipStream_t stream) {
 template <int KS, int MT, int QT>
 int launch_bf16(const ParallelParams& pp, bool vec, bool packed, int stages, hipStream_t stream) {
   if constexpr (KS == 1 && MT <= 2) {
-    // 256-query work-groups once they fill every CU's slots, else 128-query ones (twice as many,
-    // the longest one half as long).  Slots per CU: two (LDS, registers); at dv <= 32 the
+    // 256-query work-groups where they fill every CU's slots, else 128-query ones (twice as many, the
+    // longest one half as long).  Slots per CU: two (LDS, registers) at dv > 32; at dv <= 32 the
     // 128-query kernel fits three, and measured faster up to 2-3 256-query work-groups per CU.
+    // Smaller grids than two per CU run the wide kernel (launch_based_parallel), unless V is only
+    // 8-byte aligned.
     if (packed) {
-      const long long wg256 = (long long)((pp.N + 255) / 256) * pp.BH;
-      return wg256 >= (MT == 1 ? 3LL : 2LL) * device_cu_count() ? launch_packed<MT, 2>(pp, stages, stream)
-                                                                 : launch_packed<MT, 1>(pp, stages, stream);
+      if constexpr (MT == 1) {
+        if ((long long)((pp.N + 255) / 256) * pp.BH < 3LL * device_cu_count()) return launch_packed<MT, 1>(pp, stages, stream);
+      }
+      return launch_packed<MT, 2>(pp, stages, stream);
     }
   }
   if (stages & 1) {
@@ -835,7 +838,7 @@ bool parallel_packed_shape(int d, int dv, bool in_f32) { return !in_f32 && packe
 
 size_t parallel_workspace_bytes(int BH, int N, int d, int dv, bool in_f32) {
   if (in_f32) return f32_split_workspace_bytes(BH, N, d, dv);   // partials of a key split, or 0
-  if (!packed_shape(d, dv)) return vrange_bytes(BH) + (wide_shape(N, d, dv) ? wide_workspace_bytes(BH, N, dv) : 0);
+  if (!packed_shape(d, dv)) return vrange_bytes(BH) + (N > BN && wide_shape(N, d, dv) ? wide_workspace_bytes(BH, N, dv) : 0);
   const size_t nb64 = ((size_t)N + BN - 1) / BN;
   const int DV = dv <= 32 ? 32 : 64;
   return (size_t)BH * nb64 * (vt_block_bytes(dv) + (size_t)stats_width(DV) * 4);
@@ -908,9 +911,18 @@ int launch_based_parallel(const ParallelArgs& a, hipStream_t stream) {
   // pre-pass on its own also leaves the maxima of that one, for a later call whose q or out is not
   // aligned.  B2 H16, whole call, register-staged / wide: d64 dv64 N2048 63 / 36 us, N8192
   // 453 / 266 us; d32 dv64 N8192 268 / 218; d64 dv128 N8192 593 / 420; B1 H2 N200 d64 18.0 / 18.0.
+  // Of the packed kernel's shapes it takes those whose 256-query work-groups do not fill the CUs
+  // twice: its pre-pass needs no scan and no k k^T, which counts more there than the row sums that it
+  // adds per key (packed / wide, us: B2 H16 d16 dv64 N256 19.5 / 15.7, N2048 33.5 / 30.2, N3000
+  // 50.8 / 48.5, N4096, which fills them, 67.1 / 71.7, N8192 183 / 199; dv32 N2048 27.5 / 22.7, N4096
+  // 53.1 / 56.6).  A single 64-key block of another shape stays register-staged: there is nothing to
+  // stream, and it needs no V^T block.
   const bool al16 = ((reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.k) |
                       reinterpret_cast<uintptr_t>(a.v) | reinterpret_cast<uintptr_t>(a.out)) & 15) == 0;
-  if (al16 && wide_shape(a.N, a.d, a.dv)) {
+  const bool few = (long long)((a.N + 255) / 256) * a.BH < 2LL * device_cu_count();
+  const bool pshape = packed_shape(a.d, a.dv);
+  if (al16 && wide_shape(a.N, a.d, a.dv) && (pshape ? few : a.N > BN) &&
+      vrange_bytes(a.BH) + wide_workspace_bytes(a.BH, a.N, a.dv) <= parallel_workspace_bytes(a.BH, a.N, a.d, a.dv, false)) {
     if (a.stages == 1)
       hipLaunchKernelGGL(vrange_kernel, dim3((unsigned)VR, (unsigned)a.BH), dim3(256), 0, stream, p.v, p.N, p.dv,
                          const_cast<u32*>(p.vmax));

@@ -1,6 +1,6 @@
-// Fused causal BASED attention, parallel form, for the bf16 head dims the packed d = 16 kernel does
-// not take: d <= 64 with d % 8 == 0, dv <= 128 with dv % 8 == 0, 16-byte aligned tensors.  Same
-// function, precision and range as based_parallel.hip (see there: u = (q.k + 1/c)^2 - 1/c^2 in
+// Fused causal BASED attention, parallel form, bf16, for the head dims the packed d = 16 kernel does
+// not take (d <= 64 with d % 8 == 0, dv <= 128 with dv % 8 == 0, 16-byte aligned tensors) and for that
+// kernel's own where the grid is small.  Same function, precision and range as based_parallel.hip (see there: u = (q.k + 1/c)^2 - 1/c^2 in
 // fp16, V^T in fp16 with exponents, the 1 of p kept exact), other data paths:
 //
 //   wide_pack_kernel  one work-group per 64-key block: V as an fp16 V^T block in the main kernel's
@@ -552,8 +552,7 @@ size_t up256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 bool wide_shape(int N, int d, int dv) {
   const size_t nb = ((size_t)N + BN - 1) / BN;
-  return d % 8 == 0 && d <= 64 && dv % 8 == 0 && dv <= 128 && !(d == 16 && dv <= 64) &&
-         nb * (size_t)(32 * mt_of(dv) * BN * 2) < ((size_t)1 << 30) && (size_t)N * d * 2 < ((size_t)1 << 30) &&
+  return d % 8 == 0 && d <= 64 && dv % 8 == 0 && dv <= 128 && nb * (size_t)(32 * mt_of(dv) * BN * 2) < ((size_t)1 << 30) && (size_t)N * d * 2 < ((size_t)1 << 30) &&
          (size_t)N * dv * 2 < ((size_t)1 << 30);
 }
 
