@@ -118,3 +118,35 @@ def test_chunked_calls_any_scores(B, H, N, d, dv, big):
     y64 = n64 / (d64 + 1e-6)
     off = ((y[-1:, heads].double().cpu() - y64).abs() / ((en + y64.abs() * ed) / d64)).max().item()
     assert off < 1.01, off
+
+
+@pytest.mark.parametrize("B,N,H,d", [(1, 65, 2, 64), (3, 200, 4, 24), (2, 257, 16, 16), (2, 2048, 32, 64), (1, 130, 3, 8)])
+def test_strided_projection_equals_copies(B, N, H, d):
+    """q, k, v read in place in a (b, t, 3, h, d) projection and the heads written merged: bit for bit
+    what the same kernel gives on contiguous copies; the rows around the output stay untouched."""
+    import kernels as K
+    from kernels import pytorch_attention as P
+    g = torch.Generator(device="cuda").manual_seed(N)
+    qkv = (torch.randn(B, N, 3, H, d, generator=g, device="cuda") / math.sqrt(math.sqrt(d))).bfloat16()
+    y = P.parallel_from_projection(qkv, 1e-6)
+    q, k, v = qkv.permute(2, 0, 3, 1, 4).contiguous().unbind(0)
+    assert y is not None and torch.equal(y, K.solution_nki(q, k, v).transpose(1, 2).reshape(B, N, H * d))
+
+
+def test_strided_arguments():
+    import ctypes
+
+    from kernels import _lib
+    L = _lib.lib()
+    x = torch.zeros(1, 128, 3, 2, 64, dtype=torch.bfloat16, device="cuda")
+    n = int(L.la_based_parallel_workspace_bytes(1, 2, 128, 64, 64, 1))
+    ws = torch.empty(n, dtype=torch.uint8, device="cuda")
+    S = ctypes.c_longlong * 3
+
+    def call(N=128, d=64, k=(49152, 64, 384), ptr=x.data_ptr(), bytes_=n):
+        return L.la_based_parallel_fwd_strided(ptr, ptr, ptr, x.data_ptr(), 1, 2, N, d, 64, S(*k), S(*k), S(*k), 0.125, 1e-6,
+                                               ws.data_ptr(), bytes_, torch.cuda.current_stream().cuda_stream)
+
+    assert call(k=(49152, 64, 380)) == -8 and call(ptr=x.data_ptr() + 2) == -8 and call(k=(0, -64, 384)) == -2
+    assert call(N=64) == -5 and call(d=60) == -5 and call(d=72) == -5 and call(k=(49152, 64, 56)) == -5
+    assert call(bytes_=n - 1) == -6 and call(N=0) == 0

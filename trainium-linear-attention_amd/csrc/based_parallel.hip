@@ -846,6 +846,12 @@ size_t parallel_workspace_bytes(int BH, int N, int d, int dv, bool in_f32) {
 
 int launch_based_parallel_fp32(const ParallelArgs& a, hipStream_t stream);
 
+bool wide_parallel_call(int BH, int N, int d, int dv) {   // the rule is explained in launch_based_parallel
+  const bool few = (long long)((N + 255) / 256) * BH < 2LL * device_cu_count();
+  return wide_shape(N, d, dv) && (packed_shape(d, dv) ? few : N > BN) &&
+         vrange_bytes(BH) + wide_workspace_bytes(BH, N, dv) <= parallel_workspace_bytes(BH, N, d, dv, false);
+}
+
 WideScale parallel_scale(float scale) {
   // Work in u'' = 2^-2k u with u = (q.k + 1/c)^2 - 1/c^2 = (2/c^2) r, k chosen so that the weight
   // of "1", W = 2^-2k * 2/c^2, lies in (0.18, 0.71] (u'' = W r): r up to 65504 / W stays inside
@@ -919,10 +925,7 @@ int launch_based_parallel(const ParallelArgs& a, hipStream_t stream) {
   // stream, and it needs no V^T block.
   const bool al16 = ((reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.k) |
                       reinterpret_cast<uintptr_t>(a.v) | reinterpret_cast<uintptr_t>(a.out)) & 15) == 0;
-  const bool few = (long long)((a.N + 255) / 256) * a.BH < 2LL * device_cu_count();
-  const bool pshape = packed_shape(a.d, a.dv);
-  if (al16 && wide_shape(a.N, a.d, a.dv) && (pshape ? few : a.N > BN) &&
-      vrange_bytes(a.BH) + wide_workspace_bytes(a.BH, a.N, a.dv) <= parallel_workspace_bytes(a.BH, a.N, a.d, a.dv, false)) {
+  if (al16 && wide_parallel_call(a.BH, a.N, a.d, a.dv)) {
     if (a.stages == 1)
       hipLaunchKernelGGL(vrange_kernel, dim3((unsigned)VR, (unsigned)a.BH), dim3(256), 0, stream, p.v, p.N, p.dv,
                          const_cast<u32*>(p.vmax));

@@ -48,7 +48,9 @@ struct WideParams {
   u32* kmx;              // optional [BH][nb]: largest finite |k| (bf16 bits); bounds |s| (any-range calls)
   void* out;
   float* den;
-  int BH, N, d, dv, nqb, nb;
+  int BH, H, N, d, dv, nqb, nb;
+  // element strides {batch, head, token} of q and k, of v and of the output
+  long long ks[3], vs[3], os[3];
   float inv_c, inv_c2, fscale, eps, qscale;
   u32 ones_hi, ones_lo;
   int normalize, out_f32, xcd_cus;
@@ -64,6 +66,12 @@ __device__ __forceinline__ int kwz(int key) {
   return KS == 1 ? ((key >> 2) ^ (key >> 3)) & 1 : KS == 2 ? (key >> 2) & 3 : wswz(key);
 }
 
+__device__ __forceinline__ size_t head_offset(const WideParams& p, const long long (&s)[3], int bh) {
+  if (p.H == p.BH) return (size_t)bh * s[1];   // one batch: no division
+  const int b = bh / p.H;
+  return (size_t)(b * s[0] + (bh - b * p.H) * s[1]);
+}
+
 // ---------------------------------------------------------------- V^T blocks
 // Thread -> keys 2 kp, 2 kp + 1 and eight columns; column sums through LDS.  Any dv: rows past dv
 // and keys past N are zero.
@@ -75,15 +83,17 @@ __global__ __launch_bounds__(256) void wide_pack_kernel(const WideParams p) {
   __shared__ u32 vmx[4], kmxl[4];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int bh = blockIdx.x / p.nb, blk = blockIdx.x - bh * p.nb, dv = p.dv;
-  const __amdgpu_buffer_rsrc_t rv = make_rsrc(p.v + (size_t)bh * p.N * dv, (u32)p.N * (u32)dv * 2u);
+  const int vrow = (int)p.vs[2];   // elements per token
+  const __amdgpu_buffer_rsrc_t rv =
+      make_rsrc(p.v + head_offset(p, p.vs, bh), ((u32)(p.N - 1) * (u32)vrow + (u32)dv) * 2u);
   u32x4 a[IT], b[IT];
   u32 m = 0u;
 #pragma unroll
   for (int x = 0; x < IT; ++x) {
     const int t = tid + 256 * x, kp = t / CPR, col = 8 * (t % CPR);
-    const int off = kp < 32 && col < dv ? ((blk * BN + 2 * kp) * dv + col) * 2 : kOffOutOfRange;
+    const int off = kp < 32 && col < dv ? ((blk * BN + 2 * kp) * vrow + col) * 2 : kOffOutOfRange;
     a[x] = buf_load_b128(rv, off);
-    b[x] = buf_load_b128(rv, off == kOffOutOfRange ? off : off + 2 * dv);
+    b[x] = buf_load_b128(rv, off == kOffOutOfRange ? off : off + 2 * vrow);
   }
 #pragma unroll
   for (int x = 0; x < IT; ++x)
@@ -94,7 +104,7 @@ __global__ __launch_bounds__(256) void wide_pack_kernel(const WideParams p) {
     }
   m = wave_max_u32(m);
   if (lane == 0) vmx[w] = m;
-  if (p.kmx != nullptr) {   // rows of d % 8 == 0, contiguous
+  if (p.kmx != nullptr) {   // contiguous k rows, d % 8 == 0
     const __amdgpu_buffer_rsrc_t rk = make_rsrc(p.k + (size_t)bh * p.N * p.d, (u32)p.N * (u32)p.d * 2u);
     u32 mk = 0u;
     for (int x = tid; x < BN * p.d / 8; x += 256) {
@@ -167,7 +177,9 @@ __global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
   const size_t hrow = (size_t)bh * N;
 
   // ---- ring copies: unit u < UK of a block are K rows, then V^T rows (then padding, never read)
-  const u32x4 rk = buffer_rsrc(p.k + hrow * d, (u32)N * (u32)d * 2u);
+  const int krow = (int)p.ks[2] * 2;   // bytes per token
+  const size_t kbase = head_offset(p, p.ks, bh);
+  const u32x4 rk = buffer_rsrc(p.k + kbase, (u32)(N - 1) * (u32)krow + (u32)d * 2u);
   const u32x4 rv = buffer_rsrc(p.vt + (size_t)bh * p.nb * (DV * BN), (u32)p.nb * (u32)(DV * BN * 2));
   int uoff[CW];
 #pragma unroll
@@ -175,7 +187,7 @@ __global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
     const int u = 4 * x + wv;
     if (u < UK) {
       const int sl = 64 * u + lane, key = sl / (2 * KS), c = (sl % (2 * KS)) ^ kwz<KS>(key);
-      uoff[x] = 8 * c < d ? key * d * 2 + 16 * c : kOffOutOfRange;
+      uoff[x] = 8 * c < d ? key * krow + 16 * c : kOffOutOfRange;
     } else {
       uoff[x] = u < UK + UV ? 1024 * (u - UK) + 16 * lane : kOffOutOfRange;
     }
@@ -189,7 +201,7 @@ __global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
       for (int x = 0; x < CW; ++x) {
         const int u = 4 * x + wv;
         const bool isk = u < UK;
-        const int off = j < nblk && uoff[x] != kOffOutOfRange ? uoff[x] + j * (isk ? BN * 2 * d : DV * BN * 2) : kOffOutOfRange;
+        const int off = j < nblk && uoff[x] != kOffOutOfRange ? uoff[x] + j * (isk ? BN * krow : DV * BN * 2) : kOffOutOfRange;
         lds_copy16(isk ? rk : rv, lds + 1024 * u, off);
       }
     }
@@ -206,7 +218,7 @@ __global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
     for (int kk = 0; kk < KS; ++kk) {
       const int col = 16 * kk + 8 * h;
       u32x4 x = {0u, 0u, 0u, 0u};
-      if (query < N && col < d) x = *reinterpret_cast<const u32x4*>(p.q + (hrow + query) * d + col);
+      if (query < N && col < d) x = *reinterpret_cast<const u32x4*>(p.q + kbase + (size_t)query * p.ks[2] + col);
       qf[qt][kk] = scale_bf16x8(x, p.qscale);
     }
   }
@@ -475,6 +487,8 @@ __global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
     constexpr int CT = MT == 1 ? 1 : 2, EB = F32 ? 4 : 2, RB = 32 * CT * EB, RS = RB + 16, CPR = RB / 16;
     static_assert(4 * 32 * RS <= (int)sizeof(ring), "output tiles fit in the ring");
     char* tile = reinterpret_cast<char*>(&ring[0][0]) + wv * (32 * RS);
+    char* obase = static_cast<char*>(p.out) + head_offset(p, p.os, bh) * EB;
+    const u32 orow = (u32)p.os[2] * EB;   // bytes per token
 #pragma unroll
     for (int qe = 0; qe < QE; ++qe) {
       const int qbase = wq0 + 32 * (e0 + qe), query = qbase + n;
@@ -499,13 +513,13 @@ __global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
             else
               *reinterpret_cast<u32x2*>(dst) = (u32x2){pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])};
           }
-        char* out = static_cast<char*>(p.out) + ((hrow + qbase) * (size_t)dv + 32 * ct) * EB;
+        char* out = obase + ((size_t)qbase * p.os[2] + 32 * ct) * EB;
         const int cols = (dv - 32 * ct) * EB;   // bytes of a row from this column on
 #pragma unroll
         for (int it = 0; it < CPR / 2; ++it) {
           const int idx = 64 * it + lane, r = idx / CPR, c = idx % CPR;
           const u32x4 y = *reinterpret_cast<const u32x4*>(tile + r * RS + 16 * c);
-          if (qbase + r < N && 16 * c < cols) *reinterpret_cast<u32x4*>(out + (size_t)r * dv * EB + 16 * c) = y;
+          if (qbase + r < N && 16 * c < cols) *reinterpret_cast<u32x4*>(out + (u32)r * orow + 16 * c) = y;   // orow < 2^26
         }
       }
     }
@@ -550,10 +564,12 @@ size_t up256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 }  // namespace
 
-bool wide_shape(int N, int d, int dv) {
+bool wide_shape(int N, int d, int dv) { return wide_shape(N, d, dv, d, dv); }
+
+bool wide_shape(int N, int d, int dv, long long krow, long long vrow) {   // rows of krow, vrow elements
   const size_t nb = ((size_t)N + BN - 1) / BN;
-  return d % 8 == 0 && d <= 64 && dv % 8 == 0 && dv <= 128 && nb * (size_t)(32 * mt_of(dv) * BN * 2) < ((size_t)1 << 30) && (size_t)N * d * 2 < ((size_t)1 << 30) &&
-         (size_t)N * dv * 2 < ((size_t)1 << 30);
+  return d % 8 == 0 && d <= 64 && dv % 8 == 0 && dv <= 128 && nb * (size_t)(32 * mt_of(dv) * BN * 2) < ((size_t)1 << 30) && (unsigned long long)N * krow * 2 < ((size_t)1 << 30) &&
+         (unsigned long long)N * vrow * 2 < ((size_t)1 << 30);
 }
 
 size_t wide_workspace_bytes(int BH, int N, int dv) {
@@ -561,7 +577,7 @@ size_t wide_workspace_bytes(int BH, int N, int dv) {
   return up256(BH * nb * DV * BN * 2) + up256(BH * nb * DV * 4) + 2 * up256(BH * nb * 4);
 }
 
-int launch_wide_parallel(const ParallelArgs& a, void* workspace, bool any_range, hipStream_t stream) {
+int launch_wide_parallel(const ParallelArgs& a, void* workspace, bool any_range, hipStream_t stream, const WideStrides* st) {
   const WideScale s = parallel_scale(a.scale);
   WideParams p{};
   p.q = static_cast<const uint16_t*>(a.q);
@@ -570,9 +586,16 @@ int launch_wide_parallel(const ParallelArgs& a, void* workspace, bool any_range,
   p.out = a.out;
   p.den = a.den;
   p.BH = a.BH;
+  p.H = st != nullptr ? st->H : a.BH;
   p.N = a.N;
   p.d = a.d;
   p.dv = a.dv;
+  for (int i = 0; i < 3; ++i) {   // contiguous: one batch of BH heads
+    const long long n[3] = {0, a.N, 1};
+    p.ks[i] = st != nullptr ? st->k[i] : n[i] * a.d;
+    p.vs[i] = st != nullptr ? st->v[i] : n[i] * a.dv;
+    p.os[i] = st != nullptr ? st->out[i] : n[i] * a.dv;
+  }
   p.nb = (a.N + BN - 1) / BN;
   const size_t DV = 32 * mt_of(a.dv), blocks = (size_t)a.BH * p.nb;
   char* ws = static_cast<char*>(workspace);

@@ -8,6 +8,7 @@
 #include <mutex>
 
 #include "../../include/based_la.h"
+#include "../../include/based_la_ext.h"
 #include "la_internal.hpp"
 
 namespace {
@@ -131,6 +132,50 @@ int la_based_parallel_fwd_packed(const void* q, const void* k, const void* v, in
                                  void* hip_stream) {
   return parallel_entry(q, k, v, in_dtype, out, out_dtype, den_or_null, B, H, N, d, dv, scale, eps, normalize,
                         workspace, workspace_bytes, hip_stream, 2);
+}
+
+int la_based_parallel_fwd_strided(const void* q, const void* k, const void* v, void* out, int B, int H, int N, int d,
+                                  int dv, const long long* k_strides, const long long* v_strides,
+                                  const long long* out_strides, float scale, float eps, void* workspace,
+                                  size_t workspace_bytes, void* hip_stream) {
+  int rc = check_common(q, k, v, out, LA_BF16, LA_BF16, B, H, N, d, dv);
+  if (rc != LA_OK) return rc;
+  if (!finite_f(scale) || !(scale > 0.f) || !finite_f(eps) || eps < 0.f) return LA_ERR_BAD_SCALAR;
+  if ((long long)B * H * N == 0) return LA_OK;
+  if (k_strides == nullptr || v_strides == nullptr || out_strides == nullptr) return LA_ERR_NULL_POINTER;
+  if (!al(q, 16) || !al(k, 16) || !al(v, 16) || !al(out, 16)) return LA_ERR_BAD_ALIGNMENT;
+  for (int i = 0; i < 3; ++i) {
+    if (k_strides[i] < 0 || v_strides[i] < 0 || out_strides[i] < 0) return LA_ERR_BAD_SHAPE;
+    if ((k_strides[i] | v_strides[i] | out_strides[i]) & 7) return LA_ERR_BAD_ALIGNMENT;
+  }
+  if (!la::wide_parallel_call(B * H, N, d, dv) || k_strides[2] < d || v_strides[2] < dv || out_strides[2] < dv ||
+      k_strides[2] > (1 << 24) || v_strides[2] > (1 << 24) || out_strides[2] > (1 << 24) || !la::wide_shape(N, d, dv, k_strides[2], v_strides[2]))
+    return LA_ERR_UNSUPPORTED_DIM;
+  const size_t need = la::parallel_workspace_bytes(B * H, N, d, dv, false);
+  if (workspace == nullptr || workspace_bytes < need) return LA_ERR_WORKSPACE;
+  if (!al(workspace, 16)) return LA_ERR_BAD_ALIGNMENT;
+  la::ParallelArgs a{};
+  a.q = q;
+  a.k = k;
+  a.v = v;
+  a.out = out;
+  a.stages = 3;
+  a.BH = B * H;
+  a.N = N;
+  a.d = d;
+  a.dv = dv;
+  a.scale = scale;
+  a.eps = eps;
+  a.normalize = true;
+  la::WideStrides st{};
+  st.H = H;
+  for (int i = 0; i < 3; ++i) {
+    st.k[i] = k_strides[i];
+    st.v[i] = v_strides[i];
+    st.out[i] = out_strides[i];
+  }
+  return la::launch_wide_parallel(a, static_cast<char*>(workspace) + la::vrange_bytes(B * H), false,
+                                  static_cast<hipStream_t>(hip_stream), &st);
 }
 
 size_t la_based_chunked_workspace_bytes(int B, int H, int N, int d, int dv, int chunk) {

@@ -114,9 +114,18 @@ WideScale parallel_scale(float scale);
 // Parallel kernel for bf16 head dims other than the packed one's (based_wide.hip); needs 16-byte
 // aligned tensors.
 bool wide_shape(int N, int d, int dv);
+bool wide_shape(int N, int d, int dv, long long krow, long long vrow);
+struct WideStrides {   // element strides {batch, head, token}; k's serve q
+  int H;
+  long long k[3], v[3], out[3];
+};
 size_t wide_workspace_bytes(int BH, int N, int dv);
 // any_range: |s| of any size (the packed and register-staged kernels hold up to about 430).
-int launch_wide_parallel(const ParallelArgs& a, void* workspace, bool any_range, hipStream_t stream);
+int launch_wide_parallel(const ParallelArgs& a, void* workspace, bool any_range, hipStream_t stream,
+                         const WideStrides* st = nullptr);
+// Whether la_based_parallel_fwd runs an aligned call of this shape on it.
+bool wide_parallel_call(int BH, int N, int d, int dv);
+size_t vrange_bytes(int BH);   // the part of the parallel workspace before the wide kernel's
 int launch_sliding_window(const SlidingArgs& a, hipStream_t stream);
 size_t chunked_workspace_bytes(int BH, int N, int d, int dv, int chunk);
 int chunked_chunk_tokens();   // tokens per chunk of the chunked kernels

@@ -25,7 +25,7 @@
 //   spack_kernel    a state's rows as fp16 hi / lo MFMA fragments, 1 KB each, i-major
 //   sapply_kernel   phi(a q) [S | z] added to a numerator and denominator, and the division
 #include "../../include/based_la.h"
-#include "../../include/based_la_state.h"
+#include "../../include/based_la_ext.h"
 #include "la_common.hpp"
 #include "la_internal.hpp"
 #include "la_stage.hpp"

@@ -1,4 +1,4 @@
-"""ctypes binding of libbased_la.so (the C ABI declared in include/based_la.h and based_la_state.h).
+"""ctypes binding of libbased_la.so (the C ABI declared in include/based_la.h and based_la_ext.h).
 
 The library is loaded lazily, after ``import torch`` so that its HIP runtime dependency
 resolves to the runtime torch has already mapped; launches go on torch's current stream.
@@ -18,6 +18,7 @@ LIB_PATH = os.environ.get("BASED_LA_LIB", os.path.join(_PKG, "libbased_la.so"))
 
 LA_F32 = 0
 LA_BF16 = 1
+LA_ERR_UNSUPPORTED_DIM = -5
 
 _lib = None
 _lock = threading.Lock()
@@ -73,6 +74,9 @@ _SIGNATURES = {
                                        _c_int, _c_float, _c_void, _c_size, _c_void]),
     "la_based_state_apply": (_c_int, [_c_void, _c_int, _c_void, _c_void, _c_void, _c_void, _c_int, _c_int, _c_int,
                                       _c_int, _c_int, _c_int, _c_float, _c_float, _c_int, _c_void, _c_size, _c_void]),
+    "la_based_parallel_fwd_strided": (_c_int, [_c_void, _c_void, _c_void, _c_void, _c_int, _c_int, _c_int, _c_int,
+                                               _c_int, _c_void, _c_void, _c_void, _c_float, _c_float, _c_void,
+                                               _c_size, _c_void]),
     "la_taylor_feature_map": (_c_int, [_c_void, _c_int, _c_void, _c_int, ctypes.c_longlong, _c_int, _c_void]),
 }
 

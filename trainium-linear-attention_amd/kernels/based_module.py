@@ -7,12 +7,13 @@ forward, so their state dicts load unchanged.
 Steps of a forward (hidden (b, t, dim) -> (b, t, dim)):
   * one GEMM for q, k and v over the three weights concatenated (rocBLAS / hipBLASLt through
     torch); the concatenation is cached and rebuilt when a weight is replaced or changed in place;
-  * its (b, t, 3, heads, head_dim) output permuted to (3, b, heads, t, head_dim) by one copy,
-    so that q, k and v are contiguous per-head operands (the kernels read each head's rows
-    contiguously; the wrappers then pass them on without copying);
   * the attention kernel: the fused parallel kernel (``solution_nki``, as the reference's NKI
-    module) or ``solution`` (the chunked kernel from ``CHUNKED_MIN_T`` tokens);
-  * the heads merged back to (b, t, dim), cast to the input dtype, and ``o_proj``.
+    module) or ``solution`` (the chunked kernel from ``CHUNKED_MIN_T`` tokens).  In bf16 the fused
+    kernel reads q, k and v in place in the (b, t, 3, heads, head_dim) projection and writes the heads
+    merged (``parallel_from_projection``; the copies before and after it took 28 of 107 us at
+    dim 1024, 16 heads, (2, 2048) tokens).  Otherwise one copy permutes the projection to
+    (3, b, heads, t, head_dim), contiguous per-head operands, and one merges the heads back;
+  * a cast to the input dtype, and ``o_proj``.
 
 The attention kernels are forward-only, as the reference's NKI kernel is: a backward pass that
 reaches them raises instead of returning wrong gradients.
@@ -24,18 +25,18 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from .pytorch_attention import solution, solution_nki
+from .pytorch_attention import parallel_from_projection, solution, solution_is_chunked, solution_nki
 
 
 class _ForwardOnly(torch.autograd.Function):
     """Runs an attention kernel under autograd; its backward raises."""
 
     @staticmethod
-    def forward(ctx, attn, q, k, v):
-        return attn(q, k, v)
+    def forward(ctx, attn, *operands):
+        return attn(*operands)
 
     @staticmethod
-    def backward(ctx, grad):
+    def backward(ctx, *grad):
         raise RuntimeError("the BASED attention kernels are forward-only: no gradient flows through them")
 
 
@@ -83,14 +84,21 @@ class TrainiumBasedLinearAttentionNKI(nn.Module):
     def forward(self, hidden_states: torch.Tensor) -> torch.Tensor:
         b, t, _ = hidden_states.size()
         qkv = F.linear(hidden_states, self._qkv_weight()).view(b, t, 3, self.num_heads, self.head_dim)
+        y = _ForwardOnly.apply(self._attention, qkv)
+        return self.o_proj(y.to(hidden_states.dtype))
+
+    def _attention(self, qkv):
+        """(b, t, 3, heads, head_dim) -> (b, t, dim)."""
+        b, t, _, _, d = qkv.shape
+        if self.dispatch == "fused" or not solution_is_chunked(t, d, d, qkv.dtype):
+            y = parallel_from_projection(qkv, self.eps)
+            if y is not None:
+                return y
         # one permuting copy to (3, b, heads, t, head_dim): q, k and v are then contiguous
         # slices, which the kernel wrappers take as they are (no copy per operand)
         q, k, v = qkv.permute(2, 0, 3, 1, 4).contiguous().unbind(0)
-        kernel = self._DISPATCH[self.dispatch]
-        eps = self.eps
-        y = _ForwardOnly.apply(lambda q_, k_, v_: kernel(q_, k_, v_, eps=eps), q, k, v)
-        y = y.transpose(1, 2).reshape(b, t, -1)
-        return self.o_proj(y.to(hidden_states.dtype))
+        y = self._DISPATCH[self.dispatch](q, k, v, eps=self.eps)
+        return y.transpose(1, 2).reshape(b, t, -1)
 
 
 class TrainiumBasedLinearAttention(TrainiumBasedLinearAttentionNKI):

@@ -25,6 +25,7 @@ outside this package.
 
 from __future__ import annotations
 
+import ctypes
 import math
 
 import torch
@@ -96,6 +97,30 @@ def based_parallel(q, k, v, eps=1e-6, scale=None, normalize=True, out_dtype=None
     return (out, den) if return_den else out
 
 
+def parallel_from_projection(qkv, eps):
+    """``solution_nki`` on the output of a fused projection, without copies: qkv (b, t, 3, heads, d),
+    contiguous bf16; returns (b, t, heads * d), the heads merged, or None for shapes that the strided
+    kernel does not take (``la_based_parallel_fwd_strided``)."""
+    b, t, _, h, d = qkv.shape
+    if qkv.dtype != torch.bfloat16 or d % 8 or d > 64 or t <= 64 or not qkv.is_contiguous() or qkv.data_ptr() % 16:
+        return None
+    _lib.require_gpu(qkv)
+    L = _lib.lib()
+    ws_bytes = int(L.la_based_parallel_workspace_bytes(b, h, t, d, d, _lib.LA_BF16))
+    out = torch.empty(b, t, h * d, dtype=qkv.dtype, device=qkv.device)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=qkv.device)
+    row = h * d
+    strides = ctypes.c_longlong * 3
+    s_in, s_out = strides(3 * t * row, d, 3 * row), strides(t * row, d, row)
+    p = qkv.data_ptr()
+    rc = L.la_based_parallel_fwd_strided(p, p + 2 * row, p + 4 * row, _lib.ptr(out), b, h, t, d, d, s_in, s_in, s_out,
+                                         1.0 / math.sqrt(d), float(eps), _lib.ptr(ws), ws_bytes, _lib.stream_of(qkv))
+    if rc == _lib.LA_ERR_UNSUPPORTED_DIM:
+        return None
+    _lib.check(rc, "la_based_parallel_fwd_strided")
+    return out
+
+
 def solution_nki(q, k, v, eps=1e-6):
     """BASED causal attention via the fused MI355X kernel (reference :44-78).
 
@@ -138,10 +163,15 @@ def solution(q, k, v, eps=1e-6):
     the segment-state path for other head dims and fp32 inputs from ``GENERAL_CHUNKED_MIN_T``;
     shorter sequences and other shapes go to the fused kernel.  There is no PyTorch fallback.
     """
-    from .chunked_attention import chunked_based_attn, chunked_supported, general_chunked_supported
-    t, d, dv = q.shape[-2], q.shape[-1], v.shape[-1]
-    cdt = _compute_dtype(q.dtype)
-    if (t >= CHUNKED_MIN_T and chunked_supported(d, dv, cdt)) or (
-            t >= GENERAL_CHUNKED_MIN_T and general_chunked_supported(d, dv, cdt)):
+    from .chunked_attention import chunked_based_attn
+    if solution_is_chunked(q.shape[-2], q.shape[-1], v.shape[-1], q.dtype):
         return chunked_based_attn(q, k, v, eps=eps)
     return based_parallel(q, k, v, eps=eps)
+
+
+def solution_is_chunked(t, d, dv, dtype):
+    """Whether ``solution`` takes the chunked kernels for these sizes."""
+    from .chunked_attention import chunked_supported, general_chunked_supported
+    cdt = _compute_dtype(dtype)
+    return (t >= CHUNKED_MIN_T and chunked_supported(d, dv, cdt)) or (
+        t >= GENERAL_CHUNKED_MIN_T and general_chunked_supported(d, dv, cdt))
