@@ -310,3 +310,22 @@ def test_v_extreme_scales_other_paths(vscale):
     e = rounded_err(yd[:, :, 0], want[:, :, 300])
     print(f"decode after prefill v x {vscale:g}: err={e:.3e}")
     assert torch.isfinite(yd).all() and e < TOL
+
+
+@pytest.mark.parametrize("dv", [64, 40, 13])                       # 16-byte and element-wise v loads
+@pytest.mark.parametrize("B,H,N", [(1, 1, 2053), (8, 16, 2053)])   # one chunk per segment; four, and a ragged tail
+@pytest.mark.parametrize("rot", range(4))
+def test_segment_waves_of_different_scales(B, H, N, dv, rot):
+    """V scaled by 1e-5, 1, 1e5 and 0 over the 32-token tiles of every 128-token chunk, so that each wave of a
+    segment's state sum works in its own unit (or on zeros alone); the state holds the segments' sums, to the bf16 bar
+    of its rms per head."""
+    scale = torch.tensor([1e-5, 1.0, 1e5, 0.0]).roll(rot).repeat_interleave(32).repeat(N // 128 + 1)[:N, None]
+    q, k, v = _scaled(B, H, N, 16, dv, seed=29)
+    v = (v.float() * scale).bfloat16()
+    qd, kd, vd = to_dev(q, k, v)
+    y, st = _kernels().based_chunked(qd, kd, vd, normalize=False, out_dtype=torch.float32, return_state=True)
+    want = ref.taylor_feature_map(k.double()).transpose(-1, -2).contiguous() @ v.double()
+    e = max(head_errs(y, ref.based_dense(q, k, v)[1]))
+    es = max(head_errs(st[..., :dv].contiguous(), want))
+    print(f"B{B} H{H} dv={dv} rot={rot}: num_err={e:.3e} state_err={es:.3e}")
+    assert e < TOL and es < TOL

@@ -59,7 +59,7 @@ namespace {
 using namespace chunk_basis;
 
 constexpr int NWAVE_OUT = 4;
-constexpr int NWAVE_SEG = 5;
+constexpr int NWAVE_SEG = 4;
 constexpr int MAX_SEG = 32;
 
 
@@ -106,15 +106,6 @@ struct LayerLds {
 __device__ __forceinline__ uint16_t* vtab(OutLds& L, int) { return L.VT; }
 template <int DSW>
 __device__ __forceinline__ uint16_t* vtab(LayerLds<DSW>& L, int slot) { return L.VT2[slot]; }
-
-struct SegTables {
-  uint16_t KT[KT_ROWS * KRS];
-  uint16_t VT[64 * KRS];
-};
-struct SegLds {
-  SegTables buf[2];
-};
-
 
 // ---- staging: global -> registers -> (convert) -> LDS
 //
@@ -206,8 +197,7 @@ __device__ __forceinline__ void stage_convert_qk(const StageRegs& s, StageConv& 
 
 // The kernels' main path converts V as is (exponent 0, the usual case); when a work-group's
 // exponent is not 0 a separate rare path converts it again with stage_convert_v_scaled and
-// rewrites the table before the readers' barrier.  (One conversion with a run-time choice
-// between the two costs registers the segment kernel does not have at three waves per SIMD.)
+// rewrites the table before the readers' barrier.
 __device__ __forceinline__ void stage_convert_v(const StageRegs& s, StageConv& o) {
 #pragma unroll
   for (int pp = 0; pp < 2; ++pp) {
@@ -368,160 +358,206 @@ __device__ __forceinline__ void gram_update(const uint16_t* KT, f32x16& G, int g
 
 
 // -------------------------------------------------------------------------------------------
-// Kernel 1: state increment of every segment but the last.  Work-group (head, segment); wave w
-// owns feature block w (all dv) and K-steps w, w + 5 of the Gram matrix; waves 0..3 stage.
-// A work-group runs two segments side by side (waves 0..4 and 5..9, each with its own LDS
-// tables; barriers are shared): two 5-wave work-groups per CU do not get co-scheduled, one
-// 10-wave work-group spreads 3 / 3 / 2 / 2 waves over the SIMDs.
-constexpr int SEG_PER_WG = 2;
+// Kernel 1: state increment of every segment but the last.  Work-group (head, segment), four waves;
+// wave w accumulates all 160 feature slots (all dv) over its own 32 tokens of every chunk, through
+// table columns that only it writes and reads: no barrier in the loop, and eight waves per CU at
+// their own pace.  The four partial states are summed through LDS at the end.
+// The bound is the k and v read (waits on it are 57 % of the wave cycles; MFMAs keep the matrix cores
+// 23 % busy, LDS its port 38 %): 168 MB in 47 us = 3.5 TB/s at B1 H16 N65536.  Splitting the features
+// instead (five waves on one block each, shared tables, a barrier per chunk) read every V^T operand
+// five times and took 58 us; whole calls: B1 H4 N32768 63.4 -> 57.1 us, B2 H16 N2048 34.2 -> 32.8,
+// B2 H16 N8192 and B1 H16 N65536 within 1 %.
+// A wave's tables of 32 tokens: rows of 80 bytes, eight of which start in eight different groups of
+// four banks (the 16-byte operand reads); the extra halves per octet of rows spread the octets that one
+// staging store writes at once.  Row and token offsets are immediates of one address per table.
+struct SegTables {
+  uint16_t KT[KT_ROWS * 40 + 16];
+  uint16_t VT[64 * 40 + 8 * 8];
+};
+__device__ __forceinline__ int seg_kt(int row) { return row * 40 + (row >= 8 ? 16 : 0); }
+__device__ __forceinline__ int seg_vt(int row) { return row * 40 + (row >> 3) * 8; }
+struct SegLds {
+  union {
+    SegTables t[NWAVE_SEG];
+    f32x4 red[4][NWAVE_SEG - 1][4][64];   // accumulator tiles on their way to the wave that sums them
+  };
+  u32 smx[NWAVE_SEG];   // max |S| per wave at the end
+  int U[NWAVE_SEG];     // V exponent of each wave's partial state
+};
 template <bool VEC_V>
-__global__ __launch_bounds__(64 * NWAVE_SEG * SEG_PER_WG) void chunked_segment_kernel(const ChunkParams p) {
-  __shared__ __attribute__((aligned(16))) SegLds Ls[SEG_PER_WG];
-  __shared__ u32 vx[2][SEG_PER_WG][4];      // max |v| of the next chunk per staging wave (by chunk parity)
-  __shared__ u32 smx[SEG_PER_WG][NWAVE_SEG];   // max |S| per wave at the end
-  const int wall = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int sub = wall / NWAVE_SEG, w = wall - sub * NWAVE_SEG;
-  const int tid = threadIdx.x - sub * 64 * NWAVE_SEG, lane = tid & 63;
+__global__ __launch_bounds__(64 * NWAVE_SEG, 2) void chunked_segment_kernel(const ChunkParams p) {
+  __shared__ __attribute__((aligned(16))) SegLds L;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
   const int r = lane & 31, h = lane >> 5;
-  SegLds& L = Ls[sub];
-  const int nseg_total = p.BH * (p.P - 1);
-  int gseg = blockIdx.x * SEG_PER_WG + sub;
-  const bool active = gseg < nseg_total;   // the last work-group may have an idle half
-  if (!active) gseg = nseg_total - 1;
   int bh, seg;
-  map_segment(gseg, p.BH, p.P - 1, bh, seg);
+  map_segment(blockIdx.x, p.BH, p.P - 1, bh, seg);
   const size_t hrow = (size_t)bh * p.N;
   const uint16_t* kh = p.k + hrow * 16;
   const uint16_t* vh = p.v + hrow * p.dv;
   const int c0 = seg * p.seg_chunks, nch = p.seg_chunks;
-  const bool stager = w < 4 && active;
 
-  const KRows kr = krows(block_slot(w, r));
-  const int ra[1] = {kt_row(kr.a) * KRS}, rb[1] = {kt_row(kr.b) * KRS};
-  const int grow = kt_row(gram_row(r)) * KRS;
-  f32x16 S[1][2] = {{splat16(0.f), splat16(0.f)}};
+  constexpr int NB = NF / 32;
+  u32 rab[NB];   // the two K^T rows of the lane's slot in each block, 16 bits each
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    const KRows kr = krows(block_slot(b, r));
+    rab[b] = (u32)(seg_kt(kr.a) + 8 * h) | ((u32)(seg_kt(kr.b) + 8 * h) << 16);
+  }
+  f32x16 S[NB][2];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) S[b][0] = S[b][1] = splat16(0.f);
   f32x16 G = splat16(0.f);
 
-  init_kt_constants(L.buf[0].KT, tid, 64 * NWAVE_SEG);
-  init_kt_constants(L.buf[1].KT, tid, 64 * NWAVE_SEG);
-  // two chunks of loads in flight: chunk c + 1 sits in registers while chunk c is processed
-  StageRegs sa, sb;
-  StageConv cv;
-  const int last = c0 + nch - 1;
-  // V exponent of this half (Uo) and of the other one (Ux): every wave tracks both, so that the
-  // rare extra barrier below is taken by the whole work-group; S accumulates in units of 2^Uo
-  static_assert(SEG_PER_WG == 2, "two halves");
-  int Uo, Ux;
-  auto publish_vmax = [&](int par, const StageRegs& x, bool has) {
-    const u32 m = wave_max_u32(has ? stage_vmax(x) : 0u);
-    if (w < 4 && lane == 0) vx[par][sub][w] = m;
-  };
-  auto read_vexp = [&](int par, int sb_) -> int { return exp_of_f32bits(lds_max4(vx[par][sb_]) << 16); };
-  if (stager) {
-    stage_load<VEC_V, false>(sa, p, nullptr, kh, vh, c0 * CH, lane, w);
-    stage_load<VEC_V, false>(sb, p, nullptr, kh, vh, min(c0 + 1, last) * CH, lane, w, nch > 1);
-  }
-  publish_vmax(0, sa, stager);
-  if (stager) {
-    stage_convert_qk<false>(sa, cv, p.qs, p.ks, lane);
-    stage_convert_v(sa, cv);
-    stage_write<false>(cv, nullptr, nullptr, L.buf[0].KT, L.buf[0].VT, lane, w);
-  }
-  lds_barrier();
-  Uo = first_unit(read_vexp(0, sub));
-  Ux = first_unit(read_vexp(0, sub ^ 1));
-  if (Uo != 0 || Ux != 0) {   // V outside [2^-6, 2^13): convert the first chunk again, scaled
-    if (Uo != 0 && stager) {
-      stage_convert_v_scaled(sa, cv, __builtin_ldexpf(1.0f, -Uo));
-      stage_write_v(cv, L.buf[0].VT, lane, w);
-    }
-    lds_barrier();
-  }
-  auto step = [&](int c, StageRegs& nxt, StageRegs& ahead) {
-    // nxt holds chunk c + 1; ahead (free) receives chunk c + 2.  Issued by every wave (empty for
-    // the non-staging one) so that the wait for nxt below counts only older loads.
-    stage_load<VEC_V, false>(ahead, p, nullptr, kh, vh, min(c0 + c + 2, last) * CH, lane, w, stager && c + 2 < nch);
-    const SegTables& T = L.buf[c & 1];
-    // scheduling hint: interleave the state update's MFMAs with the work around them (B2 H16
-    // N8192 51.74 -> 51.18 us, B1 H16 N16384 53.6 -> 53.0 us in one process, outputs identical)
-    __builtin_amdgcn_iglp_opt(0);
-    update_blocks<1>(T.KT, T.VT, S, ra, rb, r, h);
-    gram_update(T.KT, G, grow, h, w, NWAVE_SEG);
-    const bool more = stager && c + 1 < nch;
-    publish_vmax((c + 1) & 1, nxt, more);
-    if (more) {
-      SegTables& Tn = L.buf[(c + 1) & 1];
-      stage_convert_qk<false>(nxt, cv, p.qs, p.ks, lane);
-      stage_convert_v(nxt, cv);
-      stage_pin<false>(cv);
-      stage_write<false>(cv, nullptr, nullptr, Tn.KT, Tn.VT, lane, w);
-    }
-    lds_barrier();
-    // a half whose next V needs a higher exponent raises it and rescales its state; a half at
-    // exponent != 0 converts that V again, scaled, reloading it rather than keeping its
-    // registers across the barrier (uniform over the work-group)
-    const int Uon = next_unit(Uo, kNoExp, read_vexp((c + 1) & 1, sub));
-    const int Uxn = next_unit(Ux, kNoExp, read_vexp((c + 1) & 1, sub ^ 1));
-    if (c + 1 < nch && (Uon != Uo || Uxn != Ux || Uon != 0 || Uxn != 0)) {
-      if (Uon != Uo) acc_scale<1>(S, __builtin_ldexpf(1.0f, Uo - Uon));
-      if (Uon != 0 && more) {
-        StageRegs again;
-        stage_load<VEC_V, false>(again, p, nullptr, kh, vh, (c0 + c + 1) * CH, lane, w);
-        stage_convert_v_scaled(again, cv, __builtin_ldexpf(1.0f, -Uon));
-        stage_write_v(cv, L.buf[(c + 1) & 1].VT, lane, w);
-      }
-      Uo = Uon;
-      Ux = Uxn;
-      lds_barrier();
+  StageRegs cur;
+  // chunk c of the segment (whole, in range), nothing for c = nch
+  const int voff = 8 * (lane & 7) < p.dv ? (2 * (lane >> 3) * p.dv + 8 * (lane & 7)) * 2 : kOffOutOfRange;
+  auto load = [&](int c) {
+    if constexpr (VEC_V) {
+      const int row0 = (c0 + min(c, nch - 1)) * CH + 32 * w;
+      const u32 n = c < nch ? 32u : 0u;   // a wave's rows
+      cur.k = buf_load_b128(make_rsrc(kh + (size_t)row0 * 16, n * 32u), 16 * lane);
+#pragma unroll
+      for (int pp = 0; pp < 2; ++pp)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          cur.v[pp][j] = buf_load_b128(make_rsrc(vh + (size_t)(row0 + 16 * pp + j) * p.dv,
+                                                 c < nch ? (n - 16 * pp - j) * (u32)p.dv * 2u : 0u), voff);
+    } else {
+      stage_load<false, false>(cur, p, nullptr, kh, vh, (c0 + min(c, nch - 1)) * CH, lane, w, c < nch);
     }
   };
-  for (int c = 0; c < nch; c += 2) {
-    step(c, sb, sa);
-    if (c + 1 < nch) step(c + 1, sa, sb);
-  }
-  // increment: S^T fp16 [dv][slot] in units of 2^EI, EI from max |S| over the waves (values
-  // below 2^14); Gram partials of the waves summed through LDS
-  const size_t slot = (size_t)bh * p.P + seg;
-  uint16_t* ws = p.wsS + slot * (64 * NF);
+  load(0);
+  SegTables& T = L.t[w];
   {
-    const u32 m = wave_max_u32(acc_absmax<1>(S));
-    if (lane == 0) smx[sub][w] = m;
+    const int row = R_ONES + (lane >> 4);
+    const u32 val = row == R_ONES ? 0x38003800u : (row == R_TWOS ? 0x3c003c00u : 0u);
+    *reinterpret_cast<u32*>(&T.KT[seg_kt(row) + 2 * (lane & 15)]) = val;
   }
-  float* red = reinterpret_cast<float*>(&L);   // 5 x 64 x 16 floats = 20 KB, tables no longer read
+  u32 wr0 = (u32)(seg_kt(8 * (lane & 1) + 4 * ((lane >> 1) & 1)) + 2 * (lane >> 2)) |
+            ((u32)(seg_vt(8 * (lane & 7)) + 2 * (lane >> 3)) << 16);
+  u32 rd0 = (u32)(seg_vt(r) + 8 * h) | ((u32)(seg_kt(gram_row(r)) + 8 * h) << 16);
+  // V and S of this wave in units of 2^U
+  int U = first_unit(exp_of_f32bits(wave_max_u32(stage_vmax(cur)) << 16));
+  for (int c = 0; c < nch; ++c) {
+    const int eV = exp_of_f32bits(wave_max_u32(stage_vmax(cur)) << 16);
+    const int Un = next_unit(U, kNoExp, eV);
+    StageConv cv;
+    stage_convert_qk<false>(cur, cv, p.qs, p.ks, lane);
+    if (Un == 0)
+      stage_convert_v(cur, cv);
+    else
+      stage_convert_v_scaled(cur, cv, __builtin_ldexpf(1.0f, -Un));
+    if (Un != U) {
+      acc_scale<NB>(S, __builtin_ldexpf(1.0f, U - Un));
+      U = Un;
+    }
+    asm volatile("" : "+v"(wr0)::"memory");   // the tables are this wave's alone, and LDS keeps its order
 #pragma unroll
-  for (int e = 0; e < 16; e += 4)
-    *reinterpret_cast<f32x4*>(&red[(w * 64 + lane) * 16 + e]) = (f32x4){G[e], G[e + 1], G[e + 2], G[e + 3]};
+    for (int i = 0; i < 4; ++i) *reinterpret_cast<u32*>(&T.KT[(wr0 & 0xffffu) + 40 * i]) = cv.kt[i];
+#pragma unroll
+    for (int pp = 0; pp < 2; ++pp)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) *reinterpret_cast<u32*>(&T.VT[(wr0 >> 16) + 16 * pp + 40 * e]) = cv.vt[pp][e];
+    asm volatile("" ::: "memory");
+    load(c + 1);
+    // kept packed in the loop: unpacked, they would take registers that the accumulators leave none of
+    asm volatile("" : "+v"(rab[0]), "+v"(rab[1]), "+v"(rab[2]), "+v"(rab[3]), "+v"(rab[4]), "+v"(rd0));
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      u32x4 bv[2];
+#pragma unroll
+      for (int n = 0; n < 2; ++n)
+        bv[n] = *reinterpret_cast<const u32x4*>(&T.VT[(rd0 & 0xffffu) + (seg_vt(32) * n) + 16 * s]);
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        const u32x4 x = *reinterpret_cast<const u32x4*>(&T.KT[(rab[b] & 0xffffu) + 16 * s]);
+        const u32x4 y = *reinterpret_cast<const u32x4*>(&T.KT[(rab[b] >> 16) + 16 * s]);
+        u32x4 a;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) a[i] = pk_mul_f16(x[i], y[i]);
+#pragma unroll
+        for (int n = 0; n < 2; ++n) S[b][n] = mfma32x32x16_f16(a, bv[n], S[b][n]);
+      }
+      const u32x4 g = *reinterpret_cast<const u32x4*>(&T.KT[(rd0 >> 16) + 16 * s]);
+      G = mfma32x32x16_f16(g, g, G);
+    }
+  }
+
+  // the partial states in the largest unit of the four, then summed: wave w gets dv half w & 1 of
+  // blocks w >> 1 and 2 + (w >> 1), waves 0 and 1 also a half of block 4, wave 2 the Gram matrix
+  if (lane == 0) L.U[w] = U;
   lds_barrier();
-  u32 msub = 0u;
+  const int Uo = __builtin_amdgcn_readfirstlane(max(max(L.U[0], L.U[1]), max(L.U[2], L.U[3])));
+  if (U != Uo) acc_scale<NB>(S, __builtin_ldexpf(1.0f, U - Uo));
+  auto put = [&](int i, const f32x16& a) {   // to wave i
+    f32x4(*dst)[64] = L.red[i][w > i ? w - 1 : w];
 #pragma unroll
-  for (int i = 0; i < NWAVE_SEG; ++i) msub = max(msub, smx[sub][i]);
-  msub = (u32)__builtin_amdgcn_readfirstlane((int)msub);
-  const int eS = exp_of_f32bits(msub);
+    for (int e = 0; e < 4; ++e) dst[e][lane] = (f32x4){a[4 * e], a[4 * e + 1], a[4 * e + 2], a[4 * e + 3]};
+  };
+  auto get = [&](f32x16& a) {
+#pragma unroll
+    for (int k = 0; k < NWAVE_SEG - 1; ++k)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const f32x4 x = L.red[w][k][e][lane];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) a[4 * e + i] += x[i];
+      }
+  };
+  f32x16 R[3];
+#pragma unroll
+  for (int t = 0; t < 3; ++t) {
+    R[t] = splat16(0.f);
+#pragma unroll
+    for (int i = 0; i < (t < 2 ? 4 : 3); ++i) {
+      const f32x16& a = t == 2 && i == 2 ? G : S[t < 2 ? 2 * t + (i >> 1) : 4][i & 1];
+      if (w == i)
+        R[t] = a;
+      else
+        put(i, a);
+    }
+    lds_barrier();
+    if (t < 2 || w < 3) get(R[t]);
+    if (t < 2) lds_barrier();
+  }
+  // increment: S^T fp16 [dv][slot] in units of 2^EI, EI from max |S| over the waves (values below 2^14)
+  float m = 0.f;
+#pragma unroll
+  for (int t = 0; t < 3; ++t)
+    if (t < 2 || w < 2) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) m = __builtin_fmaxf(m, __builtin_fabsf(R[t][i]));
+    }
+  const u32 mw = wave_max_u32(__builtin_bit_cast(u32, m));
+  if (lane == 0) L.smx[w] = mw;
+  lds_barrier();
+  const int eS = exp_of_f32bits(lds_max4(L.smx));
   // S 2^es in fp16, es = 13 - eS, clamped so that the factor stays finite (the stored exponent
   // follows the clamp; a state more than 2^114 below 1 in units of 2^Uo has lost nothing of use)
   const int es = eS == kNoExp ? 0 : min(13 - eS, 127);
   const int EI = eS == kNoExp ? kNoExp : Uo - es;
   const float f = eS == kNoExp ? 0.f : __builtin_ldexpf(1.0f, es);
+  const size_t slot = (size_t)bh * p.P + seg;
+  uint16_t* ws = p.wsS + slot * (64 * NF);
 #pragma unroll
-  for (int n = 0; n < (active ? 2 : 0); ++n) {
+  for (int t = 0; t < 3; ++t) {
+    if (t == 2 && w >= 2) continue;
+    const int blk = t < 2 ? 2 * t + (w >> 1) : 4;
 #pragma unroll
     for (int J = 0; J < 2; ++J) {
-      const f32x16& a = S[0][n];
+      const f32x16& a = R[t];
       const u32x4 pk = {pack_f16x2(a[8 * J + 0] * f, a[8 * J + 1] * f), pack_f16x2(a[8 * J + 2] * f, a[8 * J + 3] * f),
                         pack_f16x2(a[8 * J + 4] * f, a[8 * J + 5] * f), pack_f16x2(a[8 * J + 6] * f, a[8 * J + 7] * f)};
-      *reinterpret_cast<u32x4*>(&ws[(32 * n + r) * NF + 32 * w + 16 * J + 8 * h]) = pk;
+      *reinterpret_cast<u32x4*>(&ws[(32 * (w & 1) + r) * NF + 32 * blk + 16 * J + 8 * h]) = pk;
     }
   }
-  if (w == 0 && lane == 0 && active) p.wsE[slot] = EI;
-  if (w == 0 && active) {
+  if (w == 0 && lane == 0) p.wsE[slot] = EI;
+  if (w == 2) {
     float* gout = p.wsG + slot * 1024 + lane * 16;
 #pragma unroll
-    for (int e = 0; e < 16; e += 4) {
-      f32x4 acc = *reinterpret_cast<const f32x4*>(&red[lane * 16 + e]);
-#pragma unroll
-      for (int ww = 1; ww < NWAVE_SEG; ++ww) acc += *reinterpret_cast<const f32x4*>(&red[(ww * 64 + lane) * 16 + e]);
-      *reinterpret_cast<f32x4*>(&gout[e]) = acc;
-    }
+    for (int e = 0; e < 16; e += 4)
+      *reinterpret_cast<f32x4*>(&gout[e]) = (f32x4){R[2][e], R[2][e + 1], R[2][e + 2], R[2][e + 3]};
   }
 }
 
@@ -1462,8 +1498,8 @@ int launch_increments(const ChunkParams& p, bool vec_v, hipStream_t stream) {
     if (e != 0) return e;
   }
   if (p.P > 1) {
-    const dim3 grid((unsigned)((p.BH * (p.P - 1) + SEG_PER_WG - 1) / SEG_PER_WG));
-    const dim3 block(64 * NWAVE_SEG * SEG_PER_WG);
+    const dim3 grid((unsigned)(p.BH * (p.P - 1)));
+    const dim3 block(64 * NWAVE_SEG);
     if (vec_v)
       hipLaunchKernelGGL(chunked_segment_kernel<true>, grid, block, 0, stream, p);
     else
