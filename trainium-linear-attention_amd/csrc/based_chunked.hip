@@ -366,7 +366,8 @@ __device__ __forceinline__ void gram_update(const uint16_t* KT, f32x16& G, int g
 // 23 % busy, LDS its port 38 %): 168 MB in 47 us = 3.5 TB/s at B1 H16 N65536.  Splitting the features
 // instead (five waves on one block each, shared tables, a barrier per chunk) read every V^T operand
 // five times and took 58 us; whole calls: B1 H4 N32768 63.4 -> 57.1 us, B2 H16 N2048 34.2 -> 32.8,
-// B2 H16 N8192 and B1 H16 N65536 within 1 %.
+// B2 H16 N8192 51.4 -> 50.7, B1 H16 N65536 155 -> 152 (no better while two values spilled: scratch makes a
+// launch slower by about a microsecond; hence the packed addresses, and the lane id read anew below).
 // A wave's tables of 32 tokens: rows of 80 bytes, eight of which start in eight different groups of
 // four banks (the 16-byte operand reads); the extra halves per octet of rows spread the octets that one
 // staging store writes at once.  Row and token offsets are immediates of one address per table.
@@ -486,21 +487,22 @@ __global__ __launch_bounds__(64 * NWAVE_SEG, 2) void chunked_segment_kernel(cons
 
   // the partial states in the largest unit of the four, then summed: wave w gets dv half w & 1 of
   // blocks w >> 1 and 2 + (w >> 1), waves 0 and 1 also a half of block 4, wave 2 the Gram matrix
-  if (lane == 0) L.U[w] = U;
+  const int ln = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));   // lane, not kept over the loop
+  if (ln == 0) L.U[w] = U;
   lds_barrier();
   const int Uo = __builtin_amdgcn_readfirstlane(max(max(L.U[0], L.U[1]), max(L.U[2], L.U[3])));
   if (U != Uo) acc_scale<NB>(S, __builtin_ldexpf(1.0f, U - Uo));
   auto put = [&](int i, const f32x16& a) {   // to wave i
     f32x4(*dst)[64] = L.red[i][w > i ? w - 1 : w];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) dst[e][lane] = (f32x4){a[4 * e], a[4 * e + 1], a[4 * e + 2], a[4 * e + 3]};
+    for (int e = 0; e < 4; ++e) dst[e][ln] = (f32x4){a[4 * e], a[4 * e + 1], a[4 * e + 2], a[4 * e + 3]};
   };
   auto get = [&](f32x16& a) {
 #pragma unroll
     for (int k = 0; k < NWAVE_SEG - 1; ++k)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const f32x4 x = L.red[w][k][e][lane];
+        const f32x4 x = L.red[w][k][e][ln];
 #pragma unroll
         for (int i = 0; i < 4; ++i) a[4 * e + i] += x[i];
       }
@@ -530,7 +532,7 @@ __global__ __launch_bounds__(64 * NWAVE_SEG, 2) void chunked_segment_kernel(cons
       for (int i = 0; i < 16; ++i) m = __builtin_fmaxf(m, __builtin_fabsf(R[t][i]));
     }
   const u32 mw = wave_max_u32(__builtin_bit_cast(u32, m));
-  if (lane == 0) L.smx[w] = mw;
+  if (ln == 0) L.smx[w] = mw;
   lds_barrier();
   const int eS = exp_of_f32bits(lds_max4(L.smx));
   // S 2^es in fp16, es = 13 - eS, clamped so that the factor stays finite (the stored exponent
@@ -549,12 +551,12 @@ __global__ __launch_bounds__(64 * NWAVE_SEG, 2) void chunked_segment_kernel(cons
       const f32x16& a = R[t];
       const u32x4 pk = {pack_f16x2(a[8 * J + 0] * f, a[8 * J + 1] * f), pack_f16x2(a[8 * J + 2] * f, a[8 * J + 3] * f),
                         pack_f16x2(a[8 * J + 4] * f, a[8 * J + 5] * f), pack_f16x2(a[8 * J + 6] * f, a[8 * J + 7] * f)};
-      *reinterpret_cast<u32x4*>(&ws[(32 * (w & 1) + r) * NF + 32 * blk + 16 * J + 8 * h]) = pk;
+      *reinterpret_cast<u32x4*>(&ws[(32 * (w & 1) + (ln & 31)) * NF + 32 * blk + 16 * J + 8 * (ln >> 5)]) = pk;
     }
   }
-  if (w == 0 && lane == 0) p.wsE[slot] = EI;
+  if (w == 0 && ln == 0) p.wsE[slot] = EI;
   if (w == 2) {
-    float* gout = p.wsG + slot * 1024 + lane * 16;
+    float* gout = p.wsG + slot * 1024 + ln * 16;
 #pragma unroll
     for (int e = 0; e < 16; e += 4)
       *reinterpret_cast<f32x4*>(&gout[e]) = (f32x4){R[2][e], R[2][e + 1], R[2][e + 2], R[2][e + 3]};
