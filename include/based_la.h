@@ -64,7 +64,8 @@ const char* la_status_string(int status);
  * workspace: device scratch of at least la_based_parallel_workspace_bytes(...) bytes, 16-byte
  * aligned (may be NULL when that is 0).  It holds V repacked as fp16 V^T blocks and prefix
  * sums over 64-key blocks of the column sums of V, of k and of k k^T for the bf16, d = 16,
- * dv % 8 == 0, dv <= 64 kernel; for fp32 inputs on small grids (2 to 255 query blocks of 128
+ * dv % 8 == 0, dv <= 64 kernel; for the other bf16 shapes, and for that one on small grids, fp16
+ * V^T blocks with an exponent and fp32 column sums each; for fp32 inputs on small grids (2 to 255 query blocks of 128
  * tokens in all heads together) the partial numerators and row sums of every (query block,
  * pair of 64-key blocks), which a second kernel adds; its contents on return are unspecified.
  * Limits: 1 <= d <= 128, 1 <= dv <= 128, scale > 0 and finite, eps >= 0 and finite.
@@ -117,8 +118,10 @@ int la_based_parallel_fwd_packed(const void* q, const void* k, const void* v, in
  * against its segment's prefix plus the quadratic form inside the segment; fp32 arithmetic
  * throughout for fp32 inputs), which has no state export here (LA_ERR_UNSUPPORTED_DIM with
  * state_out_or_null set): a caller continues such a sequence with la_based_chunked_fwd_num_den
- * and the state's contraction with phi(q) (the Python layer does this with
- * la_taylor_feature_map and fp32 GEMMs).  Both are linear in N.
+ * and the state's contraction with phi(q) (la_based_state_apply and la_based_state_export of
+ * based_la_ext.h for bf16; the Python layer uses la_taylor_feature_map and fp32 GEMMs for fp32).
+ * Both are linear in N; aligned bf16 calls of 513 to 8192 tokens (12288 for d > 16) run the
+ * parallel form instead, which is faster there, in the same workspace.
  */
 size_t la_based_chunked_workspace_bytes(int B, int H, int N, int d, int dv, int chunk);
 
@@ -250,7 +253,7 @@ int la_based_decode_step(const void* q, const void* k, const void* v, int in_dty
  * la_based_decode_step).  The workspace lets a small batch split every head's state rows over
  * several work-groups, whose partial column sums are then added in a fixed order
  * (deterministic, but rounded differently from la_based_decode_step).
- * la_based_decode_workspace_bytes gives the size.  It is 0 when a head's state fits in LDS
+ * la_based_decode_workspace_bytes gives the size.  It is 0 when a head's state is small
  * (F*(dv+1) <= 10240 floats), when one work-group per head already fills the device, or for
  * shapes outside the limits; the workspace can then be NULL, and the call is
  * la_based_decode_step.  Otherwise it holds B*H*R*(dv+1) floats for R row groups per

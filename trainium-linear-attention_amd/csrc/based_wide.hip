@@ -1,7 +1,8 @@
 // Fused causal BASED attention, parallel form, bf16, for the head dims the packed d = 16 kernel does
 // not take (d <= 64 with d % 8 == 0, dv <= 128 with dv % 8 == 0, 16-byte aligned tensors) and for that
-// kernel's own where the grid is small.  Same function, precision and range as based_parallel.hip (see there: u = (q.k + 1/c)^2 - 1/c^2 in
-// fp16, V^T in fp16 with exponents, the 1 of p kept exact), other data paths:
+// kernel's own where the grid is small.  Same function, precision and range as based_parallel.hip
+// (see there: u = (q.k + 1/c)^2 - 1/c^2 in fp16, V^T in fp16 with exponents, the 1 of p kept exact),
+// other data paths:
 //
 //   wide_pack_kernel  one work-group per 64-key block: V as an fp16 V^T block in the main kernel's
 //                     LDS layout with an exponent of its own, and its fp32 column sums;

@@ -17,8 +17,9 @@ Two chunked paths: the recurrence kernel for bf16 inputs with d = 16 and dv <= 6
 configuration), and for other head dims and fp32 inputs (d <= 64, dv <= 128) a segment-state
 path (state prefixes of 512-token segments in the feature basis, then every query's contraction
 with its segment's prefix plus the quadratic form inside the segment; fp32 throughout for fp32
-inputs).  Both are linear in the sequence
-length.  Shapes outside both are computed by the fused parallel kernel, which evaluates the same
+inputs).  Both are linear in the sequence length; bf16 calls of the latter with 16-byte rows and 513
+to 8192 tokens (12288 for d > 16) run the parallel form inside the library, which is faster there.
+Shapes outside both are computed by the fused parallel kernel, which evaluates the same
 function (numerator or normalised) on the GPU.  ``chunk_size`` is the reference's argument
 (any value >= 1); the kernel's recurrence runs 128-token chunks (``la_based_chunked_chunk_used``
 reports it), which gives the same result for every chunk size up to rounding (chunk-size
