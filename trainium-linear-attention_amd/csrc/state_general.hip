@@ -16,7 +16,7 @@
 //
 // Measured at B1 H16 N3001 d64 dv64 (us): max 5 + prep 6 + export 57, pack 11 + apply 54, where phi
 // written to memory and GEMMs took 1210 (the whole continued call 1378 -> 168, of
-// which the sequence itself takes about 25).
+// which the sequence itself takes about 40).
 //
 //   smax_kernel     partial maxima of the finite |k|, |v| of every head (their fp16 exponents)
 //   sprep_kernel    64-token chunks of k and v transposed to fp16 rows of tokens, once
