@@ -366,7 +366,7 @@ __device__ __forceinline__ void gram_update(const uint16_t* KT, f32x16& G, int g
 // 23 % busy, LDS its port 38 %): 168 MB in 47 us = 3.5 TB/s at B1 H16 N65536.  Splitting the features
 // instead (five waves on one block each, shared tables, a barrier per chunk) read every V^T operand
 // five times and took 58 us; whole calls: B1 H4 N32768 63.4 -> 57.1 us, B2 H16 N2048 34.2 -> 32.8,
-// B2 H16 N8192 51.4 -> 50.7, B1 H16 N65536 155 -> 152 (no better while two values spilled: scratch makes a
+// B2 H16 N8192 1.00 to 1.02 times as fast, B1 H16 N65536 155 -> 152 (no better while two values spilled: scratch makes a
 // launch slower by about a microsecond; hence the packed addresses, and the lane id read anew below).
 // A wave's tables of 32 tokens: rows of 80 bytes, eight of which start in eight different groups of
 // four banks (the 16-byte operand reads); the extra halves per octet of rows spread the octets that one
@@ -938,9 +938,9 @@ __device__ __forceinline__ void output_wave(LT& L, const ChunkParams& p, int bh,
   constexpr bool GRAM = W == kGramWave;
   const int tid = threadIdx.x;
   int lane = tid & 63;
-  // In the layer kernel the lane's range is hidden from the compiler (here and at the state update):
-  // with it known, address arithmetic is folded into forms that cost registers (254 -> 247) and time
-  // (B2 H16 N8192 84.7 -> 82.9 us, N3001 45.9 -> 45.5; the chunked output kernel is 1-2 % slower so).
+  // In the layer kernel the lane's range is hidden from the compiler: with it known, address
+  // arithmetic is folded into forms that cost registers (254 -> 250) and time (B2 H16 N8192
+  // 84.6 -> 83.1 us, N3001 45.9 -> 45.8; the chunked output kernel is about 1 % slower so).
   if constexpr (LAYER) asm("" : "+v"(lane));
   const int r = lane & 31, h = lane >> 5;
   const int N = p.N, dv = p.dv;
@@ -1292,9 +1292,7 @@ __device__ __forceinline__ void output_wave(LT& L, const ChunkParams& p, int bh,
     }
 
     // ---- state update with this chunk
-    int ru = r, hu = h;
-    if constexpr (LAYER) asm("" : "+v"(ru), "+v"(hu));
-    update_blocks<NB>(L.KT, vtab(L, (c0 + c) & 1), S, ra, rb, ru, hu);
+    update_blocks<NB>(L.KT, vtab(L, (c0 + c) & 1), S, ra, rb, r, h);
     if (GRAM) gram_update(L.KT, G, grow, h, 0, 1);
     // next chunk in registers (V with the current exponent), and the maxima that decide the
     // next exponent: |S| before this update, |v| and |k| of the next chunk
