@@ -86,38 +86,82 @@ def test_pre_pass_apart_and_misaligned():
         assert _check(q, k, v, y, torch.zeros(1), 0.125)[0] < 1
 
 
+def _chunked_terms(q, k, v, c):
+    """Numerator and denominator in 64 bits, and what a chunked call may be off them by: below row 512 p is
+    bf16 hi + lo (2^-17 relative), from there on r = p - 1 of earlier blocks fp16 (2^-11); q.k sums d + 1
+    products in fp32, p turns an error e of s into (1 + |s|) e; N fp32 sums."""
+    N, d = q.shape[-2], q.shape[-1]
+    s = c * q @ k.transpose(-2, -1)
+    one = torch.tril(torch.ones(N, N, dtype=torch.float64))
+    r = (s + 0.5 * s * s) * one
+    reach = c * q.abs() @ k.abs().transpose(-2, -1)
+    ep = (1.0 + s.abs()) * (d + 2) * 2.0 ** -23 * (reach + 1.0) * one + (N + 64) * 2.0 ** -23 * (r.abs() + one)
+    rel = torch.where(torch.arange(N) < 512, 2.0 ** -17, 2.0 ** -11 + 2.0 ** -13).double()[:, None]
+    ep = ep + rel * torch.where(rel > 2.0 ** -17, r.abs(), r + one)
+    return (r + one) @ v, (r + one).sum(-1, keepdim=True), ep @ v.abs(), ep.sum(-1, keepdim=True)
+
+
 @pytest.mark.parametrize("big", [1.0, 30.0, 3000.0])
-@pytest.mark.parametrize("B,H,N,d,dv", [(1, 2, 513, 64, 64), (1, 2, 700, 32, 128), (4, 128, 514, 64, 32), (1, 3, 1024, 24, 16)])
+@pytest.mark.parametrize("B,H,N,d,dv", [(1, 2, 513, 64, 64), (1, 2, 700, 32, 128), (4, 128, 514, 64, 32), (1, 3, 1024, 24, 16),
+                                        (4, 128, 1100, 8, 72), (4, 128, 800, 64, 64)])
 def test_chunked_calls_any_scores(B, H, N, d, dv, big):
-    """Chunked calls of several segments take this kernel too, with scores of any size: a query whose
-    bound on |s| passes fp16's range scales its u by 2^-2e, e from sum |q| max |k| <= 128 2^e / qscale.
-    The bound above, and u's subnormal step 2^-25 2^2e / W.  Some queries and keys are `big` times the
-    others, numerator and normalised."""
+    """Chunked calls of several segments take this kernel too, with scores of any size: some queries and
+    keys are `big` times the others; numerator and normalised."""
     import kernels as K
     q, k, v = rand_qkv(B, H, N, d, dv, seed=N + d, dtype=torch.float32, scale_qk=0.7)
     q[:, :, 5::7] *= big
     k[:, :, 3::11] *= big
     q, k, v = (x.bfloat16() for x in (q, k, v))
-    c = 1.0 / math.sqrt(d)
     qd, kd, vd = (x.cuda() for x in (q, k, v))
     y = K.based_chunked(qd, kd, vd, out_dtype=torch.float32)
     num = K.based_chunked(qd, kd, vd, normalize=False, out_dtype=torch.float32)
     heads = slice(0, 2)          # the oracle's N x N in 64 bits: two heads of the last batch
     q, k, v = (x[-1:, heads].double() for x in (q, k, v))
-    s = c * q @ k.transpose(-2, -1)
-    r, one = torch.tril(s + 0.5 * s * s), torch.tril(torch.ones(N, N, dtype=torch.float64))
-    d64, n64 = (r + one).sum(-1, keepdim=True), (r + one) @ v
-    reach = c * q.abs().sum(-1, keepdim=True) * k.abs().max()     # bound on |s|
-    # u = W r, W >= 0.18, in units of 2^2e <= (reach / c qscale / 64)^2; 1 / (c qscale) <= 1.2 by W
-    step = 2.0 ** -25 / 0.18 * (1.0 + (1.2 * reach / 64) ** 2) * one
-    rel = 2.0 ** -11 + 2.0 ** -13
-    en = (rel * r.abs() + step) @ v.abs() + (N + 64) * 2.0 ** -23 * ((r.abs() + one) @ v.abs())
-    ed = (rel * r.abs() + step).sum(-1, keepdim=True) + N * 2.0 ** -23 * (r.abs() + one).sum(-1, keepdim=True)
+    n64, d64, en, ed = _chunked_terms(q, k, v, 1.0 / math.sqrt(d))
     off = ((num[-1:, heads].double().cpu() - n64).abs() / en).max().item()
     assert off < 1, off
     y64 = n64 / (d64 + 1e-6)
     off = ((y[-1:, heads].double().cpu() - y64).abs() / ((en + y64.abs() * ed) / d64)).max().item()
     assert off < 1.01, off
+
+
+@pytest.mark.parametrize("N,d,dv", [(900, 64, 64), (1300, 16, 128), (700, 32, 32)])
+def test_chunked_calls_as_exact_as_the_segment_path(N, d, dv):
+    """Relative errors of fp32 outputs, q and k four times the benchmark's: 2.6e-6 in the first 512 rows and
+    1.6e-4 to 2e-4 after them on the segment path (with u in fp16 for all rows: 5e-5 to 1.4e-4 in the first)."""
+    import kernels as K
+    q, k, v = rand_qkv(1, 3, N, d, dv, seed=N, dtype=torch.bfloat16, scale_qk=4.0 / math.sqrt(d))
+    y = K.based_chunked(q.cuda(), k.cuda(), v.cuda(), out_dtype=torch.float32).double().cpu()
+    n64, d64, _, _ = _chunked_terms(q.double(), k.double(), v.double(), 1.0 / math.sqrt(d))
+    y64 = n64 / (d64 + 1e-6)
+    first, rest = (((y - y64)[:, :, r].norm() / y64[:, :, r].norm()).item() for r in (slice(0, 512), slice(512, N)))
+    assert first < 4e-6 and rest < 2e-4, (first, rest)
+
+
+@pytest.mark.parametrize("d,dv", [(64, 64), (32, 128), (64, 32)])
+def test_chunked_calls_are_causal(d, dv):
+    """A huge key or value changes no bit of an earlier row, in its own 64-token block or before."""
+    import kernels as K
+    N = 1090
+    q, k, v = (x.cuda() for x in rand_qkv(1, 2, N, d, dv, seed=d, dtype=torch.bfloat16, scale_qk=0.7))
+    want = K.based_chunked(q, k, v, out_dtype=torch.float32)
+    for t in (50, 500, 520, 690, 1000, 1085):
+        kb, vb = k.clone(), v.clone()
+        kb[:, :, t] *= 3e5
+        vb[:, :, t] *= 1e20
+        y = K.based_chunked(q, kb, vb, out_dtype=torch.float32)
+        assert torch.equal(y[:, :, :t], want[:, :, :t]), t
+
+
+def test_chunked_calls_small_value_columns():
+    """A column of V 2^-30 below the others, which one fp16 exponent per block could not hold."""
+    import kernels as K
+    q, k, v = rand_qkv(1, 2, 1100, 64, 64, seed=3, dtype=torch.bfloat16, scale_qk=0.7)
+    v = (v.float() * torch.where(torch.arange(64) % 8 == 3, 2.0 ** -30, 1.0)).bfloat16()
+    num = K.based_chunked(q.cuda(), k.cuda(), v.cuda(), normalize=False, out_dtype=torch.float32).double().cpu()
+    n64, _, en, _ = _chunked_terms(q.double(), k.double(), v.double(), 0.125)
+    off = ((num - n64).abs() / en).max().item()
+    assert off < 1, off
 
 
 @pytest.mark.parametrize("B,N,H,d", [(1, 65, 2, 64), (3, 200, 4, 24), (2, 257, 16, 16), (2, 2048, 32, 64), (1, 130, 3, 8)])

@@ -22,8 +22,18 @@
 // wave pairs share queries and take one 32-key half of every block each (their accumulators meet
 // in LDS at the end), so that the grid is twice as large at the same reads per MFMA.
 //
-// Chunked calls of the same shapes take these kernels too (chunked_general.hip), with scores of any
-// size (`any_range`: the pre-pass then also reads K for its largest magnitude per block).
+// Chunked calls of the same shapes take these kernels too (chunked_general.hip), with scores and V of
+// any size, and no less exact than the segment path that they replace (fp16 prefixes and features;
+// inside a 512-token segment p in 16 bits against exact V): ANY.  A work-group takes the blocks before
+// its own queries as above where that loses nothing: from row kExactRows on, |u| inside fp16 by
+// sum |q| max |k| (the pre-pass then also reads K), one V exponent and the values of
+// every block held in fp16 to 2^-14 of their column's largest.  All other blocks, its own always, run
+// `precise`: p in fp32, as bf16 hi and lo parts against the V rows themselves.  So what a row gets
+// depends on no later key or value.  Relative error of fp32 outputs, rows before / from 512, against
+// the segment path's: B1 H4 N4096 d64 dv64, q and k of the benchmark 2.6e-6 / 3.2e-6 (2.6e-6 / 1.9e-4),
+// four times as large 2.5e-6 / 4.9e-5 (2.5e-6 / 1.9e-4), sixteen times 2.4e-6 / 2.0e-4 (2.4e-6 / 2.7e-4).
+// The blocks that run `precise` cost B2 H16 N8192 d64 dv64 5 % (266 -> 282 us); all of them, for
+// scores out of range, 432 us (the segment path 423).
 //
 // Measured (pre-pass + kernel, us; the register-staged kernel and its max pass before): B2 H16 d64 dv64
 // N2048 7 + 29 (5 + 62), N8192 14 + 252 (8 + 445): 1.04 PFLOP/s, matrix cores busy 57 % of the
@@ -46,7 +56,7 @@ struct WideParams {
   uint16_t* vt;          // [BH][nb][32 MT rows][64] fp16
   float* sums;           // [BH][nb][32 MT] column sums of V
   int* eb;               // [BH][nb] V exponents
-  u32* kmx;              // optional [BH][nb]: largest finite |k| (bf16 bits); bounds |s| (any-range calls)
+  u32* kmx;              // ANY: [BH][nb]: largest finite |k| (bf16 bits), kCoarse where fp16 V^T will not do
   void* out;
   float* den;
   int BH, H, N, d, dv, nqb, nb;
@@ -67,6 +77,9 @@ __device__ __forceinline__ int kwz(int key) {
   return KS == 1 ? ((key >> 2) ^ (key >> 3)) & 1 : KS == 2 ? (key >> 2) & 3 : wswz(key);
 }
 
+constexpr u32 kCoarse = 0x80000000u;
+constexpr int kExactRows = 512;   // the first segment of the path that chunked calls took before
+
 __device__ __forceinline__ size_t head_offset(const WideParams& p, const long long (&s)[3], int bh) {
   if (p.H == p.BH) return (size_t)bh * s[1];   // one batch: no division
   const int b = bh / p.H;
@@ -76,12 +89,13 @@ __device__ __forceinline__ size_t head_offset(const WideParams& p, const long lo
 // ---------------------------------------------------------------- V^T blocks
 // Thread -> keys 2 kp, 2 kp + 1 and eight columns; column sums through LDS.  Any dv: rows past dv
 // and keys past N are zero.
-template <int MT>
+template <int MT, bool ANY>
 __global__ __launch_bounds__(256) void wide_pack_kernel(const WideParams p) {
   constexpr int DV = 32 * MT, CPR = DV / 8, IT = (32 * CPR + 255) / 256;
   __shared__ __attribute__((aligned(16))) uint16_t img[DV * BN];
   __shared__ float csum[32][DV + 1];
   __shared__ u32 vmx[4], kmxl[4];
+  __shared__ u32 lost[ANY ? DV : 1];   // a value of this column is not exact in fp16
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int bh = blockIdx.x / p.nb, blk = blockIdx.x - bh * p.nb, dv = p.dv;
   const int vrow = (int)p.vs[2];   // elements per token
@@ -105,7 +119,8 @@ __global__ __launch_bounds__(256) void wide_pack_kernel(const WideParams p) {
     }
   m = wave_max_u32(m);
   if (lane == 0) vmx[w] = m;
-  if (p.kmx != nullptr) {   // contiguous k rows, d % 8 == 0
+  if (ANY && tid < DV) lost[tid] = 0u;
+  if constexpr (ANY) {   // contiguous k rows, d % 8 == 0
     const __amdgpu_buffer_rsrc_t rk = make_rsrc(p.k + (size_t)bh * p.N * p.d, (u32)p.N * (u32)p.d * 2u);
     u32 mk = 0u;
     for (int x = tid; x < BN * p.d / 8; x += 256) {
@@ -120,8 +135,6 @@ __global__ __launch_bounds__(256) void wide_pack_kernel(const WideParams p) {
     if (lane == 0) kmxl[w] = mk;
   }
   __syncthreads();
-  if (p.kmx != nullptr && tid == 0)
-    p.kmx[(size_t)bh * p.nb + blk] = max(max(kmxl[0], kmxl[1]), max(kmxl[2], kmxl[3]));
   const int eb = vexp_step(max(max(vmx[0], vmx[1]), max(vmx[2], vmx[3])) << 16);
 #pragma unroll
   for (int x = 0; x < IT; ++x) {
@@ -135,14 +148,33 @@ __global__ __launch_bounds__(256) void wide_pack_kernel(const WideParams p) {
       const float f1 = (c & 1) ? bf16_hi_to_f32(b[x][c >> 1]) : bf16_lo_to_f32(b[x][c >> 1]);
       const int row = col + c;
       csum[kp][row] = f0 + f1;
-      *reinterpret_cast<u32*>(&img[row * BN + ((unit ^ wswz(row)) << 3) + e]) =
-          pack_f16x2(__builtin_ldexpf(f0, -eb), __builtin_ldexpf(f1, -eb));
+      const float g0 = __builtin_ldexpf(f0, -eb), g1 = __builtin_ldexpf(f1, -eb);
+      const u32 y = pack_f16x2(g0, g1);
+      if (ANY && (f16_lo_to_f32(y) != g0 || f16_hi_to_f32(y) != g1)) lost[row] = 1u;
+      *reinterpret_cast<u32*>(&img[row * BN + ((unit ^ wswz(row)) << 3) + e]) = y;
     }
   }
   __syncthreads();
   const size_t rec = (size_t)bh * p.nb + blk;
   u32x4* dst = reinterpret_cast<u32x4*>(p.vt + rec * (DV * BN));
-  for (int i = tid; i < DV * BN / 8; i += 256) dst[i] = reinterpret_cast<const u32x4*>(img)[i];
+  int coarse = eb == 128;   // infinities and NaN
+  for (int i = tid; i < DV * BN / 8; i += 256) {
+    const u32x4 x = reinterpret_cast<const u32x4*>(img)[i];
+    dst[i] = x;
+    if constexpr (ANY) {
+      // eight lanes hold a column: what fp16 drops of it, at most 2^-25, stays below 2^-14 of its largest value
+      u32 mc = 0u;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) mc = max(mc, max(x[e] & 0x7fffu, (x[e] >> 16) & 0x7fffu));
+#pragma unroll
+      for (int y = 1; y < 8; y <<= 1) mc = max(mc, (u32)__shfl_xor((int)mc, y));
+      coarse |= lost[i >> 3] != 0u && mc < 0x1000u;   // fp16 2^-11
+    }
+  }
+  if constexpr (ANY) {
+    coarse = __syncthreads_or(coarse);
+    if (tid == 0) p.kmx[rec] = max(max(kmxl[0], kmxl[1]), max(kmxl[2], kmxl[3])) | (coarse ? kCoarse : 0u);
+  }
   if (tid < DV) {
     float s = 0.f;
 #pragma unroll
@@ -155,7 +187,7 @@ __global__ __launch_bounds__(256) void wide_pack_kernel(const WideParams p) {
 // ---------------------------------------------------------------- attention
 // KS: 16-wide steps of d; MT: 32-wide tiles of dv; QT: 32-query tiles per wave; NKH: waves sharing a
 // query group (2: each takes one 32-key half of every block).  UNIT: 1/c scales to exactly 1/2.
-template <int KS, int MT, int QT, int NKH, bool UNIT>
+template <int KS, int MT, int QT, int NKH, bool UNIT, bool ANY>
 __global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
   constexpr int DV = 32 * MT, NQW = 4 / NKH, BM = 32 * QT * NQW;
   constexpr int UB = NKH;                           // blocks per step (two 32-key units per wave either way)
@@ -165,6 +197,7 @@ __global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
   constexpr int NSR = NKH == 2 ? 2 : CW <= 4 ? 4 : 3;   // steps in the ring
   __shared__ __attribute__((aligned(16))) uint16_t ring[NSR * UB][BLK];
   __shared__ float vsl[NQW][DV];
+  __shared__ u32 wst[ANY ? 4 : 1][5];
 
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), h = lane >> 5, n = lane & 31;
   const int qg = NKH == 2 ? wv >> 1 : wv, kh = NKH == 2 ? wv & 1 : 0;
@@ -178,11 +211,16 @@ __global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
   const size_t hrow = (size_t)bh * N;
 
   // ---- ring copies: unit u < UK of a block are K rows, then V^T rows (then padding, never read)
-  const int krow = (int)p.ks[2] * 2;   // bytes per token
+  const int krow = (int)p.ks[2] * 2, vrow = (int)p.vs[2] * 2;   // bytes per token
   const size_t kbase = head_offset(p, p.ks, bh);
   const u32x4 rk = buffer_rsrc(p.k + kbase, (u32)(N - 1) * (u32)krow + (u32)d * 2u);
   const u32x4 rv = buffer_rsrc(p.vt + (size_t)bh * p.nb * (DV * BN), (u32)p.nb * (u32)(DV * BN * 2));
-  int uoff[CW];
+  // ANY: blocks from jraw on come as rows of V (of DV columns in LDS) in place of the V^T block; at
+  // first on the assumption that the others may be taken as such
+  static_assert(kExactRows % 256 == 0, "whole work-groups");
+  int jraw = q0 >= kExactRows ? jb0 : 0;
+  const u32x4 rw = buffer_rsrc(p.v + head_offset(p, p.vs, bh), (u32)(N - 1) * (u32)vrow + (u32)dv * 2u);
+  int uoff[CW], woff[CW];
 #pragma unroll
   for (int x = 0; x < CW; ++x) {
     const int u = 4 * x + wv;
@@ -192,6 +230,8 @@ __global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
     } else {
       uoff[x] = u < UK + UV ? 1024 * (u - UK) + 16 * lane : kOffOutOfRange;
     }
+    const int sl = 64 * (u - UK) + lane, key = sl / (4 * MT), c = sl % (4 * MT);
+    woff[x] = u >= UK && u < UK + UV && 8 * c < dv ? key * vrow + 16 * c : kOffOutOfRange;
   }
   auto issue = [&](int s) {   // steps and blocks past the last read nothing: the counts stay equal
 #pragma unroll
@@ -202,6 +242,10 @@ __global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
       for (int x = 0; x < CW; ++x) {
         const int u = 4 * x + wv;
         const bool isk = u < UK;
+        if (ANY && !isk && j >= jraw) {
+          lds_copy16(rw, lds + 1024 * u, j < nblk && woff[x] != kOffOutOfRange ? woff[x] + j * (BN * vrow) : kOffOutOfRange);
+          continue;
+        }
         const int off = j < nblk && uoff[x] != kOffOutOfRange ? uoff[x] + j * (isk ? BN * krow : DV * BN * 2) : kOffOutOfRange;
         lds_copy16(isk ? rk : rv, lds + 1024 * u, off);
       }
@@ -223,50 +267,65 @@ __global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
       qf[qt][kk] = scale_bf16x8(x, p.qscale);
     }
   }
-  // ---- exponents of the blocks this wave attends to
+  // ---- exponents of the blocks that this wave attends to (ANY: of those before the work-group's
+  // queries)
   const int* __restrict__ ebs = p.eb + (size_t)bh * p.nb;
   int emax = -128, emin = 1 << 20;
-  u32 km = 0u;
-  if (live)
-    for (int j = lane; j <= jd; j += 64) {
+  bool mixed = false, fast = true;   // ANY: fast: blocks before jb0 as u and V^T
+  if constexpr (ANY) {
+    u32 km = 0u, bad = 0u;
+    for (int j = tid; j < jb0; j += 256) {
       const int e = ebs[j];
+      const u32 m = p.kmx[(size_t)bh * p.nb + j];
       emax = max(emax, e);
       emin = min(emin, e);
-      if (p.kmx != nullptr) km = max(km, p.kmx[(size_t)bh * p.nb + j]);
+      km = max(km, m & ~kCoarse);
+      bad |= m & kCoarse;
     }
-  emax = (int)wave_max_u32((u32)(emax + 1024)) - 1024;
-  emin = (1 << 21) - (int)wave_max_u32((u32)((1 << 21) - emin));
-  bool mixed = live && emin != emax;
-  // u in fp16 holds |s| up to about 430.  Any-range calls bound a query's |q.k| by its sum of |q| times
-  // the largest |k|, and a query whose bound is higher takes q, 1/c and W smaller by 2^-eq (u by
-  // 2^-2 eq); its wave then runs every block through `general`.
-  int eq[QT];
-#pragma unroll
-  for (int qt = 0; qt < QT; ++qt) eq[qt] = 0;
-  if (p.kmx != nullptr) {
-    const float kmax = __builtin_bit_cast(float, wave_max_u32(km) << 16);
-    bool far = false;
+    float l1 = 0.f;   // the largest sum of |q| of the wave's queries (NaN: above every number)
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt) {
-      float l1 = 0.f;
+      float y = 0.f;
 #pragma unroll
       for (int kk = 0; kk < KS; ++kk)
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          l1 += __builtin_fabsf(bf16_lo_to_f32(qf[qt][kk][e])) + __builtin_fabsf(bf16_hi_to_f32(qf[qt][kk][e]));
-      l1 += __shfl_xor(l1, 32);
-      // |b| = |q~ k + 1/c| <= 240 keeps u = b^2 - 1/c^2 below 57600
-      const float bound = l1 * kmax + p.inv_c;
-      if (!(bound <= 240.f)) {
-        int e;
-        (void)__builtin_frexpf(__builtin_fminf(bound, 3.0e38f) * (1.0f / 128.0f), &e);   // bound / 2^e <= 128; NaN and inf: the largest
-        eq[qt] = e;
-        far = true;
-#pragma unroll
-        for (int kk = 0; kk < KS; ++kk) qf[qt][kk] = scale_bf16x8(qf[qt][kk], __builtin_ldexpf(1.0f, -e));
-      }
+          y += __builtin_fabsf(bf16_lo_to_f32(qf[qt][kk][e])) + __builtin_fabsf(bf16_hi_to_f32(qf[qt][kk][e]));
+      y += __shfl_xor(y, 32);
+      l1 = __builtin_bit_cast(float, max(__builtin_bit_cast(u32, l1), __builtin_bit_cast(u32, y)));
     }
-    if (__ballot(far) != 0ull) mixed = live;
+    const u32 st[5] = {wave_max_u32((u32)(emax + 1024)), wave_max_u32((u32)((1 << 21) - emin)), wave_max_u32(km),
+                       wave_max_u32(__builtin_bit_cast(u32, l1)), wave_max_u32(bad)};
+    if (lane == 0)
+#pragma unroll
+      for (int i = 0; i < 5; ++i) wst[wv][i] = st[i];
+    __syncthreads();
+    u32 all[5];
+#pragma unroll
+    for (int i = 0; i < 5; ++i)
+      all[i] = (u32)__builtin_amdgcn_readfirstlane((int)max(max(wst[0][i], wst[1][i]), max(wst[2][i], wst[3][i])));
+    emax = (int)all[0] - 1024;
+    emin = (1 << 21) - (int)all[1];
+    // u in fp16: |b| = |q~ k + 1/c| <= 240 keeps b^2 - 1/c^2 below 57600
+    const float bound = __builtin_bit_cast(float, all[3]) * __builtin_bit_cast(float, all[2] << 16) + p.inv_c;
+    fast = __builtin_amdgcn_readfirstlane(jraw > 0 && emin == emax && all[4] == 0u && bound <= 240.f);
+    if (jraw > 0 && !fast) {   // the copies under way are of the wrong kind
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      jraw = 0;
+#pragma unroll
+      for (int s = 0; s < NSR - 1; ++s) issue(s);
+    }
+  } else {
+    if (live)
+      for (int j = lane; j <= jd; j += 64) {
+        const int e = ebs[j];
+        emax = max(emax, e);
+        emin = min(emin, e);
+      }
+    emax = (int)wave_max_u32((u32)(emax + 1024)) - 1024;
+    emin = (1 << 21) - (int)wave_max_u32((u32)((1 << 21) - emin));
+    mixed = live && emin != emax;
   }
   // ---- column sums of V over the blocks before each query group's diagonal block
   {
@@ -288,8 +347,9 @@ __global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
         float t = 0.f;
 #pragma unroll
         for (int x = 0; x < PARTS; ++x) t += psum[x * DV + c];
-        for (int j = jb0; j < min(jd, p.nb); ++j) t += p.sums[((size_t)bh * p.nb + j) * DV + c];
-        vsl[qg][c] = t;
+        if (!ANY)
+          for (int j = jb0; j < min(jd, p.nb); ++j) t += p.sums[((size_t)bh * p.nb + j) * DV + c];
+        vsl[qg][c] = fast ? t : 0.f;   // `precise` counts the 1 of p itself
       }
     __syncthreads();   // psum read before the ring takes its place
   }
@@ -303,7 +363,7 @@ __global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
     for (int mt = 0; mt < MT; ++mt) acc[qt][mt] = splat16(0.f);
   }
   const float inv_c = UNIT ? 0.5f : p.inv_c, inv_c2 = UNIT ? 0.25f : p.inv_c2;
-  constexpr u32 kOnes = 0x3c003c00u;   // packed fp16 (1, 1)
+  constexpr u32 kOnes = 0x3c003c00u, kOnesBf = 0x3f803f80u;   // packed (1, 1) in fp16, bf16
 
   auto kfrag = [&](const uint16_t* st, int ks, int kk) {
     const int key = 32 * ks + n;
@@ -381,14 +441,8 @@ __global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
     for (int qt = 0; qt < QT; ++qt) {
       const int qbase = wq0 + 32 * qt, query = qbase + n;
       act[qt] = kb <= qbase + 31 && qbase < N;
-      const float ic = __builtin_ldexpf(inv_c, -eq[qt]), ic2 = __builtin_ldexpf(inv_c2, -2 * eq[qt]);
-      u32 whi = p.ones_hi, wlo = p.ones_lo;
-      if (eq[qt] != 0) {
-        const float wq = __builtin_ldexpf(1.0f / p.fscale, -2 * eq[qt]);
-        whi = pack_f16x2(wq, wq);
-        wlo = pack_f16x2(wq - f16_lo_to_f32(whi), wq - f16_lo_to_f32(whi));
-      }
-      f32x16 b = splat16(ic);
+      const u32 whi = p.ones_hi, wlo = p.ones_lo;
+      f32x16 b = splat16(inv_c);
 #pragma unroll
       for (int kk = 0; kk < KS; ++kk) b = mfma32x32x16(kf[kk], qf[qt][kk], b);
 #pragma unroll
@@ -396,7 +450,7 @@ __global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
           const int i = 8 * m + 2 * c, k0 = kb + c32_row(i, h);   // keys k0, k0 + 1
-          const float u0 = __builtin_fmaf(b[i], b[i], -ic2), u1 = __builtin_fmaf(b[i + 1], b[i + 1], -ic2);
+          const float u0 = __builtin_fmaf(b[i], b[i], -inv_c2), u1 = __builtin_fmaf(b[i + 1], b[i + 1], -inv_c2);
           const bool in0 = k0 <= query, in1 = k0 + 1 <= query;
           x[0][qt][m][c] = pack_f16x2(in0 ? u0 : 0.f, in1 ? u1 : 0.f);
           x[1][qt][m][c] = (in0 ? whi & 0xffffu : 0u) | (in1 ? whi & 0xffff0000u : 0u);
@@ -404,7 +458,58 @@ __global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
           if (act[qt]) rsum[qt] = dot2_f16(x[0][qt][m][c], kOnes, rsum[qt]);
         }
     }
-    Pscaled(st, ks, x, !diag ? 1 : p.ones_lo != 0u || p.kmx != nullptr ? 3 : 2, act, e);
+    Pscaled(st, ks, x, !diag ? 1 : p.ones_lo != 0u ? 3 : 2, act, e);
+  };
+  // ANY: W p = b^2 + 1/c^2 in fp32, carried as bf16 hi + lo (16 bits) against the rows of V (exact) that
+  // the stage holds; the row sums take the same two parts, so that a row's rounding cancels in the quotient
+  auto weights = [&](const f32x16& b, int kb, int query, bool masked, float& sum, u32x4 (&hi)[2], u32x4 (&lo)[2]) {
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int i = 8 * m + 2 * c, k0 = kb + c32_row(i, h);   // keys k0, k0 + 1
+        float w0 = __builtin_fmaf(b[i], b[i], inv_c2), w1 = __builtin_fmaf(b[i + 1], b[i + 1], inv_c2);
+        if (masked) {
+          w0 = k0 <= query ? w0 : 0.f;
+          w1 = k0 + 1 <= query ? w1 : 0.f;
+        }
+        hi[m][c] = pack_bf16x2(w0, w1);
+        lo[m][c] = pack_bf16x2(w0 - bf16_lo_to_f32(hi[m][c]), w1 - bf16_hi_to_f32(hi[m][c]));
+        sum = dot2_bf16(lo[m][c], kOnesBf, dot2_bf16(hi[m][c], kOnesBf, sum));
+      }
+  };
+  // A operand of P.V from the rows of V: column 32 mt + n, keys 16 m + 4 h + {0..3, 8..11}
+  auto vrows = [&](const uint16_t* st, int ks, int m, int mt) {
+    const uint16_t* x = st + UK * 512 + (32 * ks + 4 * h + 16 * m) * DV + n + 32 * mt;
+    return (u32x4){(u32)x[0] | ((u32)x[DV] << 16), (u32)x[2 * DV] | ((u32)x[3 * DV] << 16),
+                   (u32)x[8 * DV] | ((u32)x[9 * DV] << 16), (u32)x[10 * DV] | ((u32)x[11 * DV] << 16)};
+  };
+  auto precise = [&](const uint16_t* st, int kb, int ks, auto masked_tag) {
+    constexpr bool MASKED = decltype(masked_tag)::value;
+    u32x4 kf[KS], vf[MT][2];
+#pragma unroll
+    for (int kk = 0; kk < KS; ++kk) kf[kk] = kfrag(st, ks, kk);
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int m = 0; m < 2; ++m) vf[mt][m] = vrows(st, ks, m, mt);
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) {
+      const int qbase = wq0 + 32 * qt;
+      if (MASKED && kb > qbase + 31) continue;   // no weight for any query (an infinite V there would count)
+      f32x16 b = splat16(inv_c);
+#pragma unroll
+      for (int kk = 0; kk < KS; ++kk) b = mfma32x32x16(kf[kk], qf[qt][kk], b);
+      u32x4 hi[2], lo[2];
+      weights(b, kb, qbase + n, MASKED && kb + 31 > qbase, rsum[qt], hi, lo);
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+          acc[qt][mt] = mfma32x32x16(vf[mt][m], hi[m], acc[qt][mt]);
+          acc[qt][mt] = mfma32x32x16(vf[mt][m], lo[m], acc[qt][mt]);
+        }
+    }
   };
 
   // step s of this wave landed (NSR - 2 later ones may be in flight), then every wave's; every wave is
@@ -419,7 +524,7 @@ __global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
   // Steps before the wave's diagonal block in a loop of their own: as one branch of a common loop the
   // accumulators were copied at its end (32 v_mov_b64 per step).  The waves leave it at different steps
   // and meet at the same count of barriers.
-  const int nfull = !live || mixed ? 0 : min(jd / UB, nstep);
+  const int nfull = ANY ? jraw / UB : !live || mixed ? 0 : min(jd / UB, nstep);
   for (int s = 0; s < nfull; ++s) {
     begin(s);
     const uint16_t* s0 = &ring[(s % NSR) * UB][0];
@@ -434,13 +539,37 @@ __global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
     E(b1, p1);
     P(s1, k1, p1);
   }
+  if (ANY && jraw > 0) {   // acc in units of 1 from here on
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt)
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[qt][mt][r] = __builtin_ldexpf(acc[qt][mt][r], emax);
+  }
+  const int npre = ANY && live ? max(nfull, min(jd / UB, nstep)) : nfull;
+  if constexpr (ANY) {
 #pragma unroll 1
-  for (int s = nfull; s < nstep; ++s) {
+    for (int s = nfull; s < npre; ++s) {
+      begin(s);
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+        precise(&ring[(s % NSR) * UB + (NKH == 2 ? t : 0)][0], 0, NKH == 2 ? kh : t, std::false_type{});
+    }
+  }
+#pragma unroll 1
+  for (int s = npre; s < nstep; ++s) {
     begin(s);
 #pragma unroll 1
     for (int t = 0; t < 2; ++t) {
       const int j = UB * s + (NKH == 2 ? t : 0), ks = NKH == 2 ? kh : t;
-      if (live && j <= jd && BN * j + 32 * ks <= wq0 + 32 * QT - 1) general(&ring[(s % NSR) * UB + (NKH == 2 ? t : 0)][0], j, ks);
+      const uint16_t* st = &ring[(s % NSR) * UB + (NKH == 2 ? t : 0)][0];
+      if (live && j <= jd && BN * j + 32 * ks <= wq0 + 32 * QT - 1) {
+        if constexpr (ANY)
+          precise(st, BN * j + 32 * ks, ks, std::true_type{});
+        else
+          general(st, j, ks);
+      }
     }
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no copy in flight into the ring
@@ -452,7 +581,6 @@ __global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
   const int e0 = NKH == 2 ? kh : 0;
   f32x16 fin[QE][MT];
   float rs[QE];
-  int ef[QE];   // the queries' exponents
   if constexpr (NKH == 2) {
     float* mine = reinterpret_cast<float*>(&ring[0][0]) + wv * ((16 * MT + 1) * 64) + lane;
     float* other = reinterpret_cast<float*>(&ring[0][0]) + (wv ^ 1) * ((16 * MT + 1) * 64) + lane;
@@ -467,13 +595,11 @@ __global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) fin[0][mt][r] = (kh ? acc[1][mt][r] : acc[0][mt][r]) + other[(16 * mt + r) * 64];
     rs[0] = (kh ? rsum[1] : rsum[0]) + other[16 * MT * 64];
-    ef[0] = kh ? eq[1] : eq[0];
     __syncthreads();   // read before the output tiles take their place
   } else {
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt) {
       rs[qt] = rsum[qt];
-      ef[qt] = eq[qt];
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) fin[qt][mt] = acc[qt][mt];
     }
@@ -481,8 +607,9 @@ __global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
   if (!live) return;
 
   // ---- out = (acc 2^E / W + column sums) / (t + 1 + row sum / W + eps), 32 rows x 64 columns at a
-  // time through this wave's own LDS, so that stores write whole lines
-  const float fscale = p.fscale, afs = fscale * __builtin_ldexpf(1.0f, emax);
+  // time through this wave's own LDS, so that stores write whole lines (ANY: E = 0, and jraw 64 in place
+  // of t + 1)
+  const float fscale = p.fscale, afs = ANY ? fscale : fscale * __builtin_ldexpf(1.0f, emax);
   auto store = [&](auto f32_tag) {
     constexpr bool F32 = decltype(f32_tag)::value;
     constexpr int CT = MT == 1 ? 1 : 2, EB = F32 ? 4 : 2, RB = 32 * CT * EB, RS = RB + 16, CPR = RB / 16;
@@ -494,10 +621,9 @@ __global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
     for (int qe = 0; qe < QE; ++qe) {
       const int qbase = wq0 + 32 * (e0 + qe), query = qbase + n;
       const float r2 = rs[qe] + __shfl_xor(rs[qe], 32);
-      const float den = (float)(query + 1) + __builtin_ldexpf(fscale * r2, 2 * ef[qe]);
+      const float den = (float)(ANY ? BN * jraw : query + 1) + fscale * r2;
       const float inv = p.normalize ? 1.0f / (den + p.eps) : 1.0f;
       if (p.den != nullptr && h == 0 && query < N) p.den[hrow + query] = den;
-      const float aq = __builtin_ldexpf(afs, 2 * ef[qe]);
 #pragma unroll
       for (int ct = 0; ct < MT; ct += CT) {
 #pragma unroll
@@ -507,7 +633,7 @@ __global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
             float y[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-              y[e] = (aq * fin[qe][ct + mt][4 * g + e] + vsl[qg][32 * (ct + mt) + 8 * g + 4 * h + e]) * inv;
+              y[e] = (afs * fin[qe][ct + mt][4 * g + e] + vsl[qg][32 * (ct + mt) + 8 * g + 4 * h + e]) * inv;
             char* dst = tile + n * RS + (32 * mt + 8 * g + 4 * h) * EB;
             if (F32)
               *reinterpret_cast<f32x4*>(dst) = (f32x4){y[0], y[1], y[2], y[3]};
@@ -537,17 +663,23 @@ int launch_main(const WideParams& pp, hipStream_t stream) {
   constexpr int BM = 128 * QT / NKH;
   p.nqb = (p.N + BM - 1) / BM;
   const dim3 grid((unsigned)(p.nqb * p.BH)), block(256);
-  if (p.inv_c == 0.5f && p.inv_c2 == 0.25f)
-    hipLaunchKernelGGL((wide_kernel<KS, MT, QT, NKH, true>), grid, block, 0, stream, p);
+  if (p.kmx != nullptr)
+    hipLaunchKernelGGL((wide_kernel<KS, MT, QT, NKH, false, true>), grid, block, 0, stream, p);
+  else if (p.inv_c == 0.5f && p.inv_c2 == 0.25f)
+    hipLaunchKernelGGL((wide_kernel<KS, MT, QT, NKH, true, false>), grid, block, 0, stream, p);
   else
-    hipLaunchKernelGGL((wide_kernel<KS, MT, QT, NKH, false>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((wide_kernel<KS, MT, QT, NKH, false, false>), grid, block, 0, stream, p);
   return (int)hipGetLastError();
 }
 
 template <int KS, int MT>
 int launch_wide(const WideParams& p, int stages, hipStream_t stream) {
   if (stages & 1) {
-    hipLaunchKernelGGL((wide_pack_kernel<MT>), dim3((unsigned)(p.BH * p.nb)), dim3(256), 0, stream, p);
+    const dim3 pgrid((unsigned)(p.BH * p.nb));
+    if (p.kmx != nullptr)
+      hipLaunchKernelGGL((wide_pack_kernel<MT, true>), pgrid, dim3(256), 0, stream, p);
+    else
+      hipLaunchKernelGGL((wide_pack_kernel<MT, false>), pgrid, dim3(256), 0, stream, p);
     const int e = (int)hipGetLastError();
     if (e != 0) return e;
   }
