@@ -60,6 +60,38 @@ def test_v_exponents(dv):
     assert off < 1 and offd < 1, (off, offd)
 
 
+@pytest.mark.parametrize("B,H,d,dv", [(2, 2, 64, 64), (1, 3, 16, 128), (4, 128, 32, 32), (4, 128, 64, 64)])
+@pytest.mark.parametrize("std", [0.13, 2.0 ** -9])
+def test_v_exponents_a_step_apart(B, H, d, dv, std):
+    """V whose blocks lie on both sides of a step of their exponents (largest values 0.3 to 0.7), and 2^8
+    below it every third block: lower blocks take u by 2^-8, rounded at 2^-25 (2^-16 of W = 0.18 to 0.71, the
+    weight of the 1 of p), and by 2^-16 they multiply apart.  Parallel and chunked calls."""
+    import kernels as K
+    N = 4500 if B * H < 8 else 700          # more than 64 blocks
+    q, k, v = rand_qkv(B, H, N, d, dv, seed=dv, dtype=torch.bfloat16, scale_qk=0.7)
+    v = v.float() * std
+    v[:, :, (torch.arange(N) // 64) % 3 == 1] *= 0.13 / 2.0 ** 7
+    v = v.bfloat16()
+    qd, kd, vd = (x.cuda() for x in (q, k, v))
+    y, den = K.based_parallel(qd, kd, vd, scale=0.09, out_dtype=torch.float32, return_den=True)
+    num = K.based_chunked(qd, kd, vd, scale=0.09, normalize=False, out_dtype=torch.float32)
+    y, den, num = (x[-1:, -2:].double().cpu() for x in (y, den, num))
+    q, k, v = (x[-1:, -2:].double() for x in (q, k, v))
+    n64, d64, en, ed = _chunked_terms(q, k, v, 0.09)
+    one = torch.tril(torch.ones(N, N, dtype=torch.float64))
+    r = (0.09 * q @ k.transpose(-2, -1)) * one
+    r = r + 0.5 * r * r
+    step = 2.0 ** -15 * one + (2.0 ** -11 + 2.0 ** -13) * r.abs()     # fp16 u in every row, or by 2^-8
+    en = en + step @ v.abs() + (N + 64) * 2.0 ** -24 * ((r.abs() + one) @ v.abs())
+    ed = ed + step.sum(-1, keepdim=True)
+    off = ((num - n64).abs() / en).max().item()
+    assert off < 1, off
+    y64 = n64 / (d64 + 1e-6)
+    off = ((y - y64).abs() / ((en + y64.abs() * ed) / d64)).max().item()
+    offd = ((den[..., None] - d64).abs() / ed).max().item()
+    assert off < 1.01 and offd < 1, (off, offd)
+
+
 def test_pre_pass_apart_and_misaligned():
     """The two halves apart equal the whole call; an output that is not 16-byte aligned takes the
     register-staged kernel, after the same pre-pass too."""

@@ -13,7 +13,8 @@
 // There is no scan between them: a work-group adds the column sums of the blocks before its own
 // queries itself (DV floats per block, against 2 (d + dv) 64 bytes of K and V that it reads of each),
 // and a wave takes the largest exponent of the blocks it attends to; a block with a smaller one
-// (rare) multiplies into cleared accumulators that are added in fp32 with the power of two.
+// takes u with that power of two if it is one step (2^-8), else (rare) multiplies into cleared
+// accumulators that are added in fp32 with it.
 //
 // What bounds it: matrix cores and LDS reads.  A wave owns 64 queries (two 32-wide tiles), so a K
 // or V^T fragment read (1 KB, 16 bytes a lane) feeds two MFMAs: d = dv = 64 reads 16 KB per 32 MFMAs
@@ -26,7 +27,7 @@
 // any size, and no less exact than the segment path that they replace (fp16 prefixes and features;
 // inside a 512-token segment p in 16 bits against exact V): ANY.  A work-group takes the blocks before
 // its own queries as above where that loses nothing: from row kExactRows on, |u| inside fp16 by
-// sum |q| max |k| (the pre-pass then also reads K), one V exponent and the values of
+// sum |q| max |k| (the pre-pass then also reads K), V exponents at most a step apart and the values of
 // every block held in fp16 to 2^-14 of their column's largest.  All other blocks, its own always, run
 // `precise`: p in fp32, as bf16 hi and lo parts against the V rows themselves.  So what a row gets
 // depends on no later key or value.  Relative error of fp32 outputs, rows before / from 512, against
@@ -188,7 +189,7 @@ __global__ __launch_bounds__(256) void wide_pack_kernel(const WideParams p) {
 // KS: 16-wide steps of d; MT: 32-wide tiles of dv; QT: 32-query tiles per wave; NKH: waves sharing a
 // query group (2: each takes one 32-key half of every block).  UNIT: 1/c scales to exactly 1/2.
 template <int KS, int MT, int QT, int NKH, bool UNIT, bool ANY>
-__global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
+__global__ __launch_bounds__(256, KS == 1 && MT == 1 ? 3 : 2) void wide_kernel(const WideParams p) {
   constexpr int DV = 32 * MT, NQW = 4 / NKH, BM = 32 * QT * NQW;
   constexpr int UB = NKH;                           // blocks per step (two 32-key units per wave either way)
   constexpr int UK = 2 * KS, UV = 4 * MT;           // 1 KB copy units of a block
@@ -268,17 +269,19 @@ __global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
     }
   }
   // ---- exponents of the blocks that this wave attends to (ANY: of those before the work-group's
-  // queries)
+  // queries); all-zero blocks (-128) go with any
   const int* __restrict__ ebs = p.eb + (size_t)bh * p.nb;
   int emax = -128, emin = 1 << 20;
-  bool mixed = false, fast = true;   // ANY: fast: blocks before jb0 as u and V^T
+  // near: two exponents a step of 8 apart, whose lower blocks take u by 2^-8 (V near the edge of a step has
+  // both in most heads); mixed: more.  ANY: fast: blocks before jb0 as u and V^T
+  bool near = false, mixed = false, fast = true;
   if constexpr (ANY) {
     u32 km = 0u, bad = 0u;
     for (int j = tid; j < jb0; j += 256) {
       const int e = ebs[j];
       const u32 m = p.kmx[(size_t)bh * p.nb + j];
       emax = max(emax, e);
-      emin = min(emin, e);
+      emin = min(emin, e == -128 ? emin : e);
       km = max(km, m & ~kCoarse);
       bad |= m & kCoarse;
     }
@@ -308,7 +311,8 @@ __global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
     emin = (1 << 21) - (int)all[1];
     // u in fp16: |b| = |q~ k + 1/c| <= 240 keeps b^2 - 1/c^2 below 57600
     const float bound = __builtin_bit_cast(float, all[3]) * __builtin_bit_cast(float, all[2] << 16) + p.inv_c;
-    fast = __builtin_amdgcn_readfirstlane(jraw > 0 && emin == emax && all[4] == 0u && bound <= 240.f);
+    fast = __builtin_amdgcn_readfirstlane(jraw > 0 && emin >= emax - 8 && all[4] == 0u && bound <= 240.f);
+    near = emin < emax;
     if (jraw > 0 && !fast) {   // the copies under way are of the wrong kind
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
@@ -321,11 +325,12 @@ __global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
       for (int j = lane; j <= jd; j += 64) {
         const int e = ebs[j];
         emax = max(emax, e);
-        emin = min(emin, e);
+        emin = min(emin, e == -128 ? emin : e);
       }
     emax = (int)wave_max_u32((u32)(emax + 1024)) - 1024;
     emin = (1 << 21) - (int)wave_max_u32((u32)((1 << 21) - emin));
-    mixed = live && emin != emax;
+    near = emin < emax;
+    mixed = live && emin < emax - 8;
   }
   // ---- column sums of V over the blocks before each query group's diagonal block
   {
@@ -386,15 +391,20 @@ __global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
       for (int kk = 0; kk < KS; ++kk) b[qt] = mfma32x32x16(kf[kk], qf[qt][kk], b[qt]);
     }
   };
-  auto E = [&](const f32x16 (&b)[QT], u32x4 (&pf)[QT][2]) {
+  // NEAR: low blocks (an exponent 8 below the wave's) take u 2^-8, whose rounding at 2^-25 is 2^-16 of the 1 of p
+  auto E = [&](auto near_tag, bool low, const f32x16 (&b)[QT], u32x4 (&pf)[QT][2]) {
+    constexpr bool NEAR = decltype(near_tag)::value;
+    const float f = low ? 0.0625f : 1.0f, cc = low ? -0.00390625f * inv_c2 : -inv_c2;
+    const u32 ones = low ? 0x5c005c00u : kOnes;   // fp16 2^8
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt)
 #pragma unroll
       for (int m = 0; m < 2; ++m)
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-          pf[qt][m][c] = sq_plus_f16x2(b[qt][8 * m + 2 * c], b[qt][8 * m + 2 * c + 1], -inv_c2);
-          rsum[qt] = dot2_f16(pf[qt][m][c], kOnes, rsum[qt]);
+          const float b0 = b[qt][8 * m + 2 * c], b1 = b[qt][8 * m + 2 * c + 1];
+          pf[qt][m][c] = NEAR ? sq_plus_f16x2(b0 * f, b1 * f, cc) : sq_plus_f16x2(b0, b1, -inv_c2);
+          rsum[qt] = dot2_f16(pf[qt][m][c], NEAR ? ones : kOnes, rsum[qt]);
         }
   };
   auto P = [&](const uint16_t* st, int ks, const u32x4 (&pf)[QT][2]) {
@@ -430,7 +440,7 @@ __global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
   };
   // a unit of the wave's diagonal block, or a full unit of a block with a smaller V exponent
   auto general = [&](const uint16_t* st, int j, int ks) {
-    const int kb = BN * j + 32 * ks, e = mixed ? max(ebs[j] - emax, -126) : 0;
+    const int kb = BN * j + 32 * ks, e = near ? max(ebs[j] - emax, -126) : 0;
     u32x4 x[3][QT][2];   // u, then the mask times W's hi and lo parts (the exact 1 of p)
     bool act[QT];
     u32x4 kf[KS];
@@ -525,8 +535,13 @@ __global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
   // accumulators were copied at its end (32 v_mov_b64 per step).  The waves leave it at different steps
   // and meet at the same count of barriers.
   const int nfull = ANY ? jraw / UB : !live || mixed ? 0 : min(jd / UB, nstep);
-  for (int s = 0; s < nfull; ++s) {
+  unsigned long long low = 0ull;
+  auto full = [&](auto near_tag, int s) {
+    constexpr bool NEAR = decltype(near_tag)::value;
     begin(s);
+    // the low blocks of 64 at a time: a load per block would wait for the copies in flight
+    if (NEAR && (UB * s & 63) == 0) low = __ballot(ebs[min(UB * s + lane, p.nb - 1)] < emax);
+    const bool l0 = NEAR && (low >> (UB * s & 63) & 1), l1 = NEAR && (low >> ((UB * s & 63) + UB - 1) & 1);
     const uint16_t* s0 = &ring[(s % NSR) * UB][0];
     const uint16_t* s1 = NKH == 2 ? &ring[(s % NSR) * UB + 1][0] : s0;
     const int k0 = NKH == 2 ? kh : 0, k1 = NKH == 2 ? kh : 1;
@@ -534,11 +549,15 @@ __global__ __launch_bounds__(256, 2) void wide_kernel(const WideParams p) {
     u32x4 p0[QT][2], p1[QT][2];
     S(s0, k0, b0);
     S(s1, k1, b1);
-    E(b0, p0);
+    E(near_tag, l0, b0, p0);
     P(s0, k0, p0);
-    E(b1, p1);
+    E(near_tag, l1, b1, p1);
     P(s1, k1, p1);
-  }
+  };
+  if (near)
+    for (int s = 0; s < nfull; ++s) full(std::true_type{}, s);
+  else
+    for (int s = 0; s < nfull; ++s) full(std::false_type{}, s);
   if (ANY && jraw > 0) {   // acc in units of 1 from here on
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt)
