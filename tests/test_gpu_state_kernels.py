@@ -120,3 +120,52 @@ def test_scales(kscale, vscale):
     y, m = (pq @ s64[..., :dv]) / z, (pq.abs() @ s64.abs()[..., :dv]) / z
     rel = 2 * ((ph.shape[-2] / 8 + 16) * 2.0 ** -24 + 2.0 ** -21)
     assert float(((out.cpu().double() - y).abs() - rel * m).max()) <= 1e-36
+
+
+def _need_gib(n):
+    if torch.cuda.mem_get_info()[0] < n * 2 ** 30:
+        pytest.skip(f"needs {n} GiB of device memory")
+
+
+def test_export_of_a_sequence_past_2_32_bytes_of_chunks():
+    """One part of 11.3 M tokens, 24 KB of converted rows per 64: the last tokens' offsets pass 2^32.  Zeros
+    but for the first and the last tokens, whose state alone is the reference."""
+    _need_gib(120)
+    B, H, N, d, dv, n1 = 1, 8, 11_300_000, 64, 128, 640
+    k = torch.zeros(B, H, N, d, dtype=torch.bfloat16, device="cuda")
+    v = torch.zeros(B, H, N, dv, dtype=torch.bfloat16, device="cuda")
+    _, k1, v1 = (x.cuda() for x in _inputs(B, H, 2 * n1, d, dv))
+    for x, x1 in ((k, k1), (v, v1)):
+        x[:, :, :n1] = x1[:, :, :n1]
+        x[:, :, N - n1:] = x1[:, :, n1:]
+    out = []
+    for kk, vv, n in ((k, v, N), (k1, v1, 2 * n1)):
+        ws, nb = _ws(B, H, n, d, dv)
+        st = torch.empty(B, H, 2145, dv + 1, device="cuda")
+        _call("la_based_state_export", kk.data_ptr(), vv.data_ptr(), 1, None, st.data_ptr(), B, H, n, d, dv, 0.125,
+              ws.data_ptr(), nb)
+        out.append(st)
+        del ws
+    assert (out[0][:, :, 0, dv] == N).all()
+    out[1][:, :, 0, dv] = N
+    assert ((out[0] - out[1]).norm() / out[1][:, :, 1:].norm()).item() < 1e-5
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_chunked_sequence_past_2_32_bytes(dtype):
+    """The segment states of 10.9 M tokens (25 KB of converted rows per 64; fp32 rows of v past 2^32 bytes):
+    the last row's numerator against the 512 tokens that are not zero.  In bf16 the fp16 prefix holds them with
+    one exponent beside the count of all tokens: 5 % off at this length, 2e-4 at 20000 (resources that wrapped
+    gave zeros, 100 %)."""
+    _need_gib(120)
+    import kernels as K
+    N, d, dv, n1, at = 10_900_000, 64, 128, 512, 10_800_000
+    q = torch.zeros(1, 1, N, d, dtype=dtype, device="cuda")
+    k, v = torch.zeros_like(q), torch.zeros(1, 1, N, dv, dtype=dtype, device="cuda")
+    q1, k1, v1 = (x.to(dtype).cuda() for x in rand_qkv(1, 1, n1, d, dv, seed=1, dtype=torch.bfloat16, scale_qk=0.7))
+    k[:, :, at:at + n1], v[:, :, at:at + n1], q[:, :, N - 1] = k1, v1, q1[:, :, 0]
+    num = K.based_chunked(q, k, v, normalize=False, out_dtype=torch.float32)[0, 0, N - 1].double().cpu()
+    s = (k1[0, 0].double() @ q1[0, 0, 0].double()).cpu() / 8
+    p = 1 + s + 0.5 * s * s
+    want = p @ v1[0, 0].double().cpu()
+    assert ((num - want).norm() / want.norm()).item() < (0.1 if dtype == torch.bfloat16 else 1e-6)

@@ -81,3 +81,44 @@ def test_map_causal_block_is_a_bijection(tmp_path):
     out = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
     print(out.stdout.strip())
     assert out.returncode == 0 and out.stdout.startswith("OK"), out.stdout + out.stderr
+
+
+WINDOWS = r"""
+#include <cstdio>
+#include "la_internal.hpp"
+
+int main() {
+  // every chunk of a head's converted chunks at the longest sequences the entry points accept
+  const long long chunks[] = {1, 2, 3, 87383, 174763, 262144};
+  for (uint32_t bytes : {4096u, 16384u, 24576u, 25600u})
+    for (long long n : chunks)
+      for (int most : {1, 2})
+        for (long long c = 0; c < n + 3; c += n > 10 ? (c + 70000 < n ? 69999 : 1) : 1) {
+          const la::RecordWindow w = la::record_window(c, n, most, bytes);
+          const long long have = c >= n ? 0 : n - c < most ? n - c : most;
+          const bool in = have == 0 || w.offset == (size_t)c * bytes;
+          if (!in || w.bytes != have * bytes || w.offset + w.bytes > (size_t)n * bytes) {
+            printf("FAIL n=%lld c=%lld most=%d bytes=%u -> (%zu, %u)\n", n, c, most, bytes, w.offset, w.bytes);
+            return 1;
+          }
+        }
+  printf("OK\n");
+  return 0;
+}
+"""
+
+
+def test_record_windows_at_any_length(tmp_path):
+    """The buffer resources of the state kernels' copy steps (record_window): exact 64-bit offsets, a size of
+    the step's own records, nothing past the last."""
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not os.path.exists(hipcc):
+        pytest.skip("hipcc not available")
+    src = tmp_path / "windows.hip"
+    src.write_text(WINDOWS)
+    exe = tmp_path / "windows"
+    r = subprocess.run([hipcc, "-O1", "-std=c++17", "--offload-arch=gfx950", "-I", CSRC, str(src), "-o", str(exe)],
+                       capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0 and r.stdout.startswith("OK"), r.stdout

@@ -326,14 +326,15 @@ __global__ __launch_bounds__(64 * (8 / TW), TW == 1 ? 4 : 1) void gstate_kernel(
 
   constexpr int UW = (CK::UNITS + NWV - 1) / NWV;   // most copy units per wave and chunk
   const int my_units = CK::UNITS / NWV + (w < CK::UNITS % NWV ? 1 : 0);
-  const u32x4 rsrc = buffer_rsrc(src, (u32)((size_t)nch * CK::HALVES * 2));
   auto issue = [&](int c) {
     if (c >= c1) return;
     const u32 base = lds_addr(&ring[c % NS][0]);
+    const RecordWindow win = record_window(c, nch, 1, CK::HALVES * 2);
+    const u32x4 rsrc = buffer_rsrc(reinterpret_cast<const char*>(src) + win.offset, win.bytes);
 #pragma unroll
     for (int x = 0; x < UW; ++x) {
       const int u = w + NWV * x;
-      if (u < CK::UNITS) lds_copy16(rsrc, base + 1024 * u, c * (CK::HALVES * 2) + 1024 * u + 16 * lane);
+      if (u < CK::UNITS) lds_copy16(rsrc, base + 1024 * u, 1024 * u + 16 * lane);
     }
   };
   __syncthreads();

@@ -120,17 +120,21 @@ __global__ __launch_bounds__(256) void g32_state_kernel(const G32Params p) {
   const int cps = GL / GC32;
   const int c0 = part * p.spp * cps, c1 = min((part + 1) * p.spp, p.nseg - 1) * cps;   // this part's chunks
   constexpr int PER = 2 * DVT * 16 + 2;   // a thread's sums: accumulators, then z partials
-  const u32x4 rk = buffer_rsrc(p.k + (size_t)bh * N * d, (u32)((size_t)N * d * 4));
-  const u32x4 rv = buffer_rsrc(p.v + (size_t)bh * N * dv, (u32)((size_t)N * dv * 4));
+  const char* khead = reinterpret_cast<const char*>(p.k + (size_t)bh * N * d);
+  const char* vhead = reinterpret_cast<const char*>(p.v + (size_t)bh * N * dv);
   const int my_units = (ku + vu) / 4 + (w < (ku + vu) % 4 ? 1 : 0);
   auto issue = [&](int c) {
     if (c >= c1) return;
     const u32 base = lds_addr(&ring[c % NS][0]);
+    // the chunk's rows and what follows them in its last copy
+    const RecordWindow wk = record_window((long long)c * GC32, N, 2 * GC32 + 1024, (u32)d * 4);
+    const RecordWindow wv = record_window((long long)c * GC32, N, 2 * GC32 + 1024, (u32)dv * 4);
+    const u32x4 rk = buffer_rsrc(khead + wk.offset, wk.bytes), rv = buffer_rsrc(vhead + wv.offset, wv.bytes);
     for (int u = w; u < ku + vu; u += 4) {
       if (u < ku)
-        lds_copy16(rk, base + 1024 * u, c * (GC32 * d * 4) + 1024 * u + 16 * lane);
+        lds_copy16(rk, base + 1024 * u, 1024 * u + 16 * lane);
       else
-        lds_copy16(rv, base + 4 * voff_f + 1024 * (u - ku), c * (GC32 * dv * 4) + 1024 * (u - ku) + 16 * lane);
+        lds_copy16(rv, base + 4 * voff_f + 1024 * (u - ku), 1024 * (u - ku) + 16 * lane);
     }
   };
 

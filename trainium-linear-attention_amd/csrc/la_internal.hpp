@@ -180,4 +180,16 @@ __host__ __device__ __forceinline__ void map_causal_block(int wg, int BH, int nq
   }
 }
 
+// Records first .. first + most - 1 of `end` consecutive ones of `record` bytes, none past the last: the
+// buffer resource of one copy step (base offset, size).  A resource over all of a head's records would
+// need offsets past 2^31 (its size past 2^32) at 5.6 (11.2) million tokens of 24 KB per 64.
+struct RecordWindow {
+  size_t offset;
+  uint32_t bytes;
+};
+__host__ __device__ __forceinline__ RecordWindow record_window(long long first, long long end, int most, uint32_t record) {
+  const long long left = end - first, n = left < 0 ? 0 : left < most ? left : most;
+  return {(size_t)(n > 0 ? first : 0) * record, (uint32_t)n * record};
+}
+
 }  // namespace la

@@ -195,18 +195,20 @@ __global__ __launch_bounds__(512, 2) void sexport_kernel(const ExportParams p) {
   const int ek = export_ek(p, bh), ev = export_ev(p, bh);
   const int nch = (N + TC - 1) / TC, c0 = part * p.cpp, c1 = min(c0 + p.cpp, nch), nst = (c1 - c0 + 1) / 2;
   const int cbytes = (32 * DT + 32 * p.nct) * TC * 2;
-  // chunks c0 .. c1 - 1; a missing second chunk of the last stage lies past the resource and reads
+  // chunks c0 .. c1 - 1, a resource for each stage of two; a missing second chunk lies past it and reads
   // as zeros, which add nothing
-  const u32x4 rk = buffer_rsrc(p.kv + ((size_t)bh * nch + c0) * (cbytes / 2), (u32)(c1 - c0) * (u32)cbytes);
+  const char* kv = reinterpret_cast<const char*>(p.kv) + (size_t)bh * nch * cbytes;
   // wave wv copies 1 KB units wv, wv + 8, ...: per chunk the k rows, then this column tile's v
   // rows; stages past the last read nothing, so that every wave's count of copies is the same
   auto issue = [&](int s) {
     const u32 lds = lds_addr(&ring[s % NS][0]);
+    const RecordWindow win = record_window(c0 + 2LL * s, c1, 2, (u32)cbytes);
+    const u32x4 rk = buffer_rsrc(kv + win.offset, win.bytes);
 #pragma unroll
     for (int x = 0; x < CW; ++x) {
       const int u = 8 * x + wv, sub = u >= 4 * CW ? 1 : 0, r = u - 4 * CW * sub;
       lds_copy16(rk, lds + 1024 * u,
-                 s < nst ? (2 * s + sub) * cbytes + 1024 * (r < 4 * DT ? r : r + 4 * ct) + 16 * lane : kOffOutOfRange);
+                 sub * cbytes + 1024 * (r < 4 * DT ? r : r + 4 * ct) + 16 * lane);
     }
   };
   const int i0 = 4 * g + w, i1 = i0 + 16 * DT;
