@@ -97,7 +97,7 @@ def test_apply(B, H, N, d, dv, normalize):
 
 @pytest.mark.parametrize("kscale,vscale", [(1e-12, 1e-20), (1e3, 1e20), (0.0, 1.0), (1.0, 0.0), (64.0, 2.0 ** -100)])
 def test_scales(kscale, vscale):
-    """Powers far from one (fp16 operands carry exponents of their own) and zeros."""
+    """Powers far from one and zeros."""
     B, H, N, d, dv = 1, 2, 200, 64, 64
     q, k, v = _inputs(B, H, N, d, dv, kscale, vscale)
     scale = 1.0 / math.sqrt(d)
@@ -120,6 +120,56 @@ def test_scales(kscale, vscale):
     y, m = (pq @ s64[..., :dv]) / z, (pq.abs() @ s64.abs()[..., :dv]) / z
     rel = 2 * ((ph.shape[-2] / 8 + 16) * 2.0 ** -24 + 2.0 ** -21)
     assert float(((out.cpu().double() - y).abs() - rel * m).max()) <= 1e-36
+
+
+def _export(k, v, scale=0.125):
+    B, H, N, d = k.shape
+    dv = v.shape[-1]
+    ws, n = _ws(B, H, N, d, dv)
+    st = torch.full((B, H, 1 + d + d * (d + 1) // 2, dv + 1), float("nan"), device="cuda")
+    kd, vd = k.cuda(), v.cuda()
+    _call("la_based_state_export", kd.data_ptr(), vd.data_ptr(), 1, None, st.data_ptr(), B, H, N, d, dv, scale,
+          ws.data_ptr(), n)
+    return st.cpu().double()
+
+
+@pytest.mark.parametrize("big", [1e3, 1e5, 1e12])
+@pytest.mark.parametrize("what", ["channel", "token", "sink", "column"])
+@pytest.mark.parametrize("d,dv", [(64, 64), (32, 40)])
+def test_export_of_uneven_inputs(d, dv, what, big):
+    """One key channel, one token's keys (with its values, or with zeros as of an attention sink) or one
+    value column far above the rest: every entry still within the bound of its own terms."""
+    _, k, v = (x.float() for x in _inputs(1, 2, 1100, d, dv))
+    if what == "channel":
+        k[..., d // 3] *= big
+    elif what == "column":
+        v[..., dv // 3] *= big
+    else:
+        k[:, :, 500] *= big
+        v[:, :, 500] *= what == "token"
+    k, v = k.bfloat16(), v.bfloat16()
+    vx = torch.cat([v.double(), torch.ones(1, 2, 1100, 1, dtype=torch.float64)], -1)
+    ph = _phi(k, 0.125).transpose(-2, -1)
+    off = ((_export(k, v) - ph @ vx).abs() / (ph.abs() @ vx.abs())).max().item()
+    assert off < (1100 / 8 + 16) * 2.0 ** -24, off
+
+
+def test_export_of_infinite_keys():
+    """The rows of an infinite key are infinite (its K-sums too), of the sign of their products, and so are
+    sums that overflow (another head); the others as without it."""
+    _, k, v = _inputs(1, 2, 300, 64, 64)
+    k[0, 0, 70, 5] = float("inf")
+    k[0, 1, 200], v[0, 1, 200] = 1.0, 64.0
+    k[0, 1, 200, 9] = 3e38
+    got = _export(k, v)
+    vx = torch.cat([v.double(), torch.ones(1, 2, 300, 1, dtype=torch.float64)], -1)
+    ph = _phi(k, 0.125).transpose(-2, -1)
+    want, m = ph @ vx, ph.abs() @ vx.abs()
+    inf = want.abs() > 2e38
+    assert inf[0, 0].any() and inf[0, 1].any() and not want.isnan().any()
+    big = got.abs() > 2e38
+    assert torch.equal(big, inf) and torch.equal(got[big].sign(), want[inf].sign())
+    assert ((got - want).abs()[~inf] / m[~inf]).max().item() < (300 / 8 + 16) * 2.0 ** -24
 
 
 def _need_gib(n):

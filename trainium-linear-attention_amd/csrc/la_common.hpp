@@ -71,11 +71,6 @@ __device__ __forceinline__ u32 pk_fma_f16(u32 a, u32 b, u32 c) {
   return __builtin_bit_cast(u32, __builtin_elementwise_fma(__builtin_bit_cast(f16x2, a), __builtin_bit_cast(f16x2, b),
                                                            __builtin_bit_cast(f16x2, c)));
 }
-// Packed fp16 a*b - c, one rounding per half (the negation is the instruction's own modifier).
-__device__ __forceinline__ u32 pk_fms_f16(u32 a, u32 b, u32 c) {
-  return __builtin_bit_cast(u32, __builtin_elementwise_fma(__builtin_bit_cast(f16x2, a), __builtin_bit_cast(f16x2, b),
-                                                           -__builtin_bit_cast(f16x2, c)));
-}
 __device__ __forceinline__ u32 pk_mul_f16(u32 a, u32 b) {
   return __builtin_bit_cast(u32, __builtin_bit_cast(f16x2, a) * __builtin_bit_cast(f16x2, b));
 }

@@ -5,26 +5,26 @@
 // phi is never written to memory: the quadratic features factor as x_i x_j, so every contraction
 // over them is a product over j (matrix cores) for each i.
 //
-// Precision.  Both directions stand in for fp32 products of phi with V or with the state, so
-// every operand keeps its bits: bf16 k, v and q are exact in fp16 after a power of two; a product
-// k_i k_j has at most 16 significant bits and is carried as fp16 hi + lo (v_pk_mul_f16, then
-// v_pk_fma_f16 for its exact remainder); a state entry is carried as fp16 hi + lo (22 bits) with
-// one exponent per feature row i.  Sums are fp32.  Relative error (2-norm) against 64 bits, against
-// fp32 phi and fp32 GEMMs on the same inputs: quadratic state rows at B1 H4 N3001 d64 dv64 1.8e-7
-// (9.0e-7), B1 H2 N40000 d32 dv64 3.8e-7 (2.3e-6); the first 64 outputs after a state of 500 tokens
+// Precision.  Both directions stand in for fp32 products of phi with V or with the state, so every
+// operand keeps its bits.  Export: a product k_i v has at most 16 significant bits and is carried as
+// bf16 hi + lo, exactly and over the whole range of fp32, against the bf16 rows of k: no channel,
+// column or token takes bits from another.  Import: a state entry is carried as fp16 hi + lo (22 bits)
+// with one exponent per feature row i, q exact in fp16 after a power of two.  Sums are fp32.  Relative
+// error (2-norm) against 64 bits, against fp32 phi and fp32 GEMMs on the same inputs: quadratic state
+// rows at B1 H4 N3001 d64 dv64 1.1e-7 (9.0e-7); the first 64 outputs after a state of 500 tokens
 // 6.7e-7 (1.5e-6).
 //
-// Measured at B1 H16 N3001 d64 dv64 (us): max 5 + prep 6 + export 57, pack 11 + apply 54, where phi
-// written to memory and GEMMs took 1210 (the whole continued call 1378 -> 168, of
-// which the sequence itself takes about 40).
+// Measured at B1 H16 N3001 d64 dv64 (us): prep 8 + export 66, pack 11 + apply 54, where
+// phi written to memory and GEMMs took 1210.
 //
-//   smax_kernel     partial maxima of the finite |k|, |v| of every head (their fp16 exponents)
-//   sprep_kernel    64-token chunks of k and v transposed to fp16 rows of tokens, once
+//   sprep_kernel    64-token chunks of k and v transposed to rows of tokens, once
 //   sexport_kernel  state rows from those: work-group = (head, 32 value columns, four i0), the
 //                   chunks through an LDS ring; parts of the sequence where heads are few, added
 //                   by scombine_kernel in order (no atomics)
 //   spack_kernel    a state's rows as fp16 hi / lo MFMA fragments, 1 KB each, i-major
 //   sapply_kernel   phi(a q) [S | z] added to a numerator and denominator, and the division
+#include <type_traits>
+
 #include "../../include/based_la.h"
 #include "../../include/based_la_ext.h"
 #include "la_common.hpp"
@@ -34,7 +34,6 @@
 namespace la {
 namespace {
 
-constexpr int kMxParts = 32;    // partial maxima per head (smax_kernel)
 constexpr int TC = 64;          // tokens per chunk of the export (a transposed row: 128 bytes)
 // The eight 16-byte units of transposed row r sit at unit ^ tswz(r): a fragment read (one unit of
 // 32 rows) touches all 64 banks once per 16-lane pass, and the transposing 8-byte writes (rows
@@ -50,48 +49,11 @@ struct ExportParams {
   const uint16_t* v;
   const float* state_in;
   float* dst;             // state_out, or the parts [S][BH][F][dv + 1]
-  u32* mx;                // [BH][2][kMxParts]
-  uint16_t* kv;           // [BH][chunks][32 DT k rows, 32 nct v rows][TC] fp16
+  u32* far;               // [BH][chunks]: not 0 where a product k_i v may be infinite
+  uint16_t* kv;           // [BH][chunks][32 DT k rows, 32 nct v rows][TC] bf16
   int BH, N, d, dv, nct, ngrp, parts, cpp;   // column tiles, i0 groups, parts of cpp 64-token chunks
   float c_lin, c_diag, c_off;                // a / d^(1/4), a^2 / sqrt(2 d), a^2 / sqrt(d)
 };
-
-// Work-group (s, head): the largest finite |k| and |v| (bf16 bits) of its share of the tokens.
-__global__ __launch_bounds__(256) void smax_kernel(const ExportParams p) {
-  __shared__ u32 wm[2][4];
-  const int tid = threadIdx.x, s = blockIdx.x % kMxParts, bh = blockIdx.x / kMxParts;
-  const int per = (p.N + kMxParts - 1) / kMxParts;
-  const int r0 = min(p.N, s * per), r1 = min(p.N, r0 + per);
-  const auto fin = [](u32 x) { return x < 0x7f80u ? x : 0u; };
-#pragma unroll
-  for (int a = 0; a < 2; ++a) {
-    const int w = a ? p.dv : p.d;
-    const uint16_t* base = (a ? p.v : p.k) + ((size_t)bh * p.N + r0) * w;
-    const long long n = (long long)(r1 - r0) * w;
-    u32 m = 0u;
-    long long i0 = 0;
-    if ((reinterpret_cast<uintptr_t>(base) & 15) == 0) {
-      const u32x4* b4 = reinterpret_cast<const u32x4*>(base);
-      for (long long i = tid; i < n / 8; i += 256) {
-        const u32x4 x = b4[i];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) m = max(m, max(fin(x[e] & 0x7fffu), fin((x[e] >> 16) & 0x7fffu)));
-      }
-      i0 = n / 8 * 8;
-    }
-    for (long long i = i0 + tid; i < n; i += 256) m = max(m, fin(base[i] & 0x7fffu));
-    m = wave_max_u32(m);
-    if ((tid & 63) == 0) wm[a][tid >> 6] = m;
-  }
-  __syncthreads();
-  if (tid < 2) p.mx[((size_t)bh * 2 + tid) * kMxParts + s] = max(max(wm[tid][0], wm[tid][1]), max(wm[tid][2], wm[tid][3]));
-}
-
-// floor(log2) of the largest of a head's partial maxima (bf16 bits), 0 for an all-zero head.
-__device__ __forceinline__ int head_exp(const u32* mx) {
-  const u32 m = wave_max_u32(mx[threadIdx.x & (kMxParts - 1)]);
-  return m == 0u ? 0 : (int)((m << 16) >> 23) - 127;   // bf16 subnormals: -127
-}
 
 // One 4-token x 4-column group of a bf16 array [rows][w]: rows row0 .. row0 + 3 (zero past N),
 // columns col .. col + 3 (zero past w).
@@ -112,29 +74,24 @@ __device__ __forceinline__ void load44(const uint16_t* __restrict__ g, int row0,
     }
   }
 }
-// The group transposed into rows row .. row + 3 at tokens t0 .. t0 + 3, as fp16(x 2^-e).
-__device__ __forceinline__ void store44(uint16_t* dst, int row, int t0, const u32x2 (&x)[4], int e) {
+// The group transposed into rows row .. row + 3 at tokens t0 .. t0 + 3.  Returns its largest magnitude (bf16 bits).
+__device__ __forceinline__ u32 store44(uint16_t* dst, int row, int t0, const u32x2 (&x)[4]) {
+  u32 m = 0u;
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
-    float f[4];
+    u32 y[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const u32 w = x[i][c >> 1];
-      f[i] = __builtin_ldexpf((c & 1) ? bf16_hi_to_f32(w) : bf16_lo_to_f32(w), -e);
+      y[i] = (c & 1) ? x[i][c >> 1] >> 16 : x[i][c >> 1] & 0xffffu;
+      m = max(m, y[i] & 0x7fffu);
     }
     *reinterpret_cast<u32x2*>(dst + (row + c) * TC + (((t0 >> 3) ^ tswz(row + c)) << 3) + (t0 & 4)) =
-        (u32x2){pack_f16x2(f[0], f[1]), pack_f16x2(f[2], f[3])};
+        (u32x2){y[0] | (y[1] << 16), y[2] | (y[3] << 16)};
   }
+  return m;
 }
 
-// One work-group per (chunk, head).  k 2^-ek in [-128, 128): every product of two is below 2^14
-// and exact in hi + lo down to 2^-38 of that; v 2^-ev below 2^15.
-__device__ __forceinline__ int export_ek(const ExportParams& p, int bh) {
-  return head_exp(p.mx + (size_t)bh * 2 * kMxParts) - 6;
-}
-__device__ __forceinline__ int export_ev(const ExportParams& p, int bh) {
-  return head_exp(p.mx + ((size_t)bh * 2 + 1) * kMxParts) - 14;
-}
+// One work-group per (chunk, head).
 template <int DT, bool VEC>
 __global__ __launch_bounds__(256) void sprep_kernel(const ExportParams p) {
   __shared__ __attribute__((aligned(16))) uint16_t img[(32 * DT + 128) * TC];
@@ -150,13 +107,25 @@ __global__ __launch_bounds__(256) void sprep_kernel(const ExportParams p) {
 #pragma unroll
   for (int x = 0; x < 2; ++x)
     if (tid + 256 * x < ngr) load44<VEC>(vg, TC * c + 4 * ((tid + 256 * x) / vg4), 4 * ((tid + 256 * x) % vg4), N, dv, vx[x]);
-  const int ek = export_ek(p, bh), ev = export_ev(p, bh);
-  if (kst) store44(img, kcol, kt0, kx, ek);
+  __shared__ u32 wm[2][4];
+  u32 mk = 0u, mv = 0u;
+  if (kst) mk = store44(img, kcol, kt0, kx);
 #pragma unroll
   for (int x = 0; x < 2; ++x)
     if (tid + 256 * x < ngr)
-      store44(img, 32 * DT + 4 * ((tid + 256 * x) % vg4), 4 * ((tid + 256 * x) / vg4), vx[x], ev);
+      mv = max(mv, store44(img, 32 * DT + 4 * ((tid + 256 * x) % vg4), 4 * ((tid + 256 * x) / vg4), vx[x]));
+  mk = wave_max_u32(mk);
+  mv = wave_max_u32(mv);
+  if ((tid & 63) == 0) {
+    wm[0][tid >> 6] = mk;
+    wm[1][tid >> 6] = mv;
+  }
   __syncthreads();
+  if (tid == 0) {   // exponents of the largest |k| and |v|: their sum bounds the products below 2^128, or does not
+    mk = max(max(wm[0][0], wm[0][1]), max(wm[0][2], wm[0][3])) >> 7;
+    mv = max(max(wm[1][0], wm[1][1]), max(wm[1][2], wm[1][3])) >> 7;
+    p.far[(size_t)bh * nch + c] = mk == 255u || mv == 255u || mk + mv > 2u * 127u + 125u ? 1u : 0u;
+  }
   const int units = (32 * DT + 32 * p.nct) * TC / 8;
   u32x4* dst = reinterpret_cast<u32x4*>(p.kv + ((size_t)bh * nch + c) * ((32 * DT + 32 * p.nct) * TC));
   for (int x = tid; x < units; x += 256) dst[x] = reinterpret_cast<const u32x4*>(img)[x];
@@ -164,21 +133,21 @@ __global__ __launch_bounds__(256) void sprep_kernel(const ExportParams p) {
 
 // ---------------------------------------------------------------- export
 // DT 32-wide tiles of j (d <= 32 DT).  The quadratic work-groups: wave w takes i0 = 4 g + w and
-// i1 = i0 + 16 DT; A = the rows k_i k_j over tokens (formed in registers: 8 VALU per fragment,
-// two MFMAs each), B = V^T's rows as columns, so C[j][column] is the state row (i, j).  Only tiles
-// with j >= i are formed: i0 both (DT = 2) or the one, i1 the last.  The last work-group of a
-// (head, column tile) takes the linear rows, the constant row and, in column tile 0, the K-sums
-// (the Gram matrix of [k | 1]).
-// What bounds it: matrix cores (six MFMAs against 3 x 8 VALU and 5 LDS reads per K step and wave).
+// i1 = i0 + 16 DT; A = the k rows j over tokens, B = the products k_i v of a value column (formed in
+// registers: 44 VALU per fragment for the six MFMAs of two), so C[j][column] is the state row (i, j).
+// Only tiles with j >= i are formed: i0 both (DT = 2) or the one, i1 the last.  The last work-group of
+// a (head, column tile) takes the linear rows, the constant row and, in column tile 0, the K-sums (the
+// Gram matrix of [k | 1]).
+// What bounds it: VALU (88 per K step and wave against six MFMAs and five LDS reads).  The products as
+// fp16 hi + lo with one exponent of k and of v per head, two packed VALU per pair, took 57 us (and 11
+// for maxima and rows against 8) and lost the bits of every channel far below the head's largest.
 // 32 columns per work-group rather than dv: at 16 heads, d = 64 that makes 288 work-groups for
-// 256 CUs without splitting the sequence, whose parts would cost a pass over fp32 partials.  With
-// one work-group per CU four waves leave each SIMD one, whose LDS and MFMA latencies nothing
-// covers (72 us at B1 H16 N3001 d64 dv64, 97 with k and v converted by every work-group instead of
-// once by sprep_kernel), so eight waves share the tokens: waves 0-3 the even chunks, waves 4-7 the
-// odd ones with the same rows, added through LDS at the end (57 us; 42 of them the loop, against 18
-// for its MFMAs alone: 160 KB of LDS reads per 128-token stage come close to them).
+// 256 CUs without splitting the sequence, whose parts would cost a pass over fp32 partials; two fit a
+// CU (128 VGPRs; with 147 and one per CU the last 32 ran a second round: 90 us for 66).  Eight waves
+// share the tokens, for the LDS and MFMA latencies that four leave open: waves 0-3 the even chunks,
+// waves 4-7 the odd ones with the same rows, added through LDS at the end.
 template <int DT>
-__global__ __launch_bounds__(512, 2) void sexport_kernel(const ExportParams p) {
+__global__ __launch_bounds__(512, 4) void sexport_kernel(const ExportParams p) {
   constexpr int NS = 3, CW = DT + 1;           // ring stages (two chunks each); 1 KB copies per wave and stage
   constexpr int CH = 32 * CW * TC;             // halves per chunk in a stage
   __shared__ __attribute__((aligned(16))) uint16_t ring[NS][2 * CH];
@@ -192,7 +161,6 @@ __global__ __launch_bounds__(512, 2) void sexport_kernel(const ExportParams p) {
   const int g = id % (p.ngrp + 1), part = id / (p.ngrp + 1);
   const bool linear = g == p.ngrp;
   const int N = p.N, d = p.d, dv = p.dv;
-  const int ek = export_ek(p, bh), ev = export_ev(p, bh);
   const int nch = (N + TC - 1) / TC, c0 = part * p.cpp, c1 = min(c0 + p.cpp, nch), nst = (c1 - c0 + 1) / 2;
   const int cbytes = (32 * DT + 32 * p.nct) * TC * 2;
   // chunks c0 .. c1 - 1, a resource for each stage of two; a missing second chunk lies past it and reads
@@ -212,8 +180,6 @@ __global__ __launch_bounds__(512, 2) void sexport_kernel(const ExportParams p) {
     }
   };
   const int i0 = 4 * g + w, i1 = i0 + 16 * DT;
-  // the exponents' loads returned before the waits below count this wave's copies
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   f32x16 acc[3];
 #pragma unroll
   for (int x = 0; x < 3; ++x) acc[x] = splat16(0.f);
@@ -231,39 +197,56 @@ __global__ __launch_bounds__(512, 2) void sexport_kernel(const ExportParams p) {
     issue(s + NS - 1);
     return static_cast<const uint16_t*>(&ring[s % NS][half * CH]);
   };
-  if (!linear) {
-    for (int s = 0; s < nst; ++s) {
-      const uint16_t* kt = next(s);
-      const uint16_t* vt = kt + 32 * DT * TC;
+  // Products of a K step.  FAR: the remainder of an infinite one (inf - inf), or none beside an infinite
+  // k_j (0 inf), is a tiny number of the product's sign.
+  constexpr float tiny = 0x1p-126f;
+  auto step = [&](auto far_tag, const uint16_t* kt, const uint16_t* vt, int u) {
+    constexpr bool FAR = decltype(far_tag)::value;
+    u32x4 kf[DT];
 #pragma unroll
-      for (int ks = 0; ks < TC / 16; ++ks) {
-        const int u = 2 * ks + h;
-        u32x4 kf[DT];
+    for (int jt = 0; jt < DT; ++jt) kf[jt] = frag(kt, 32 * jt + n, u);
+    const u32x4 vf = frag(vt, n, u);
+    // the rows i of this half's eight tokens, the same for its 32 lanes
+    const u32x4 ki[2] = {frag(kt, i0, u), frag(kt, i1, u)};
+    u32x4 hi[2], lo[2];
 #pragma unroll
-        for (int jt = 0; jt < DT; ++jt) kf[jt] = frag(kt, 32 * jt + n, u);
-        const u32x4 vf = frag(vt, n, u);
-        // the row i of this half's eight tokens, the same for its 32 lanes
-        const u32x4 ki0 = frag(kt, i0, u), ki1 = frag(kt, i1, u);
-        u32x4 hi[DT + 1], lo[DT + 1];
+    for (int x = 0; x < 2; ++x)
 #pragma unroll
-        for (int x = 0; x < DT + 1; ++x) {
-          const u32x4& ki = x < DT ? ki0 : ki1;
-          const u32x4& kj = kf[x < DT ? x : DT - 1];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            hi[x][e] = pk_mul_f16(ki[e], kj[e]);
-            lo[x][e] = pk_fms_f16(ki[e], kj[e], hi[x][e]);
-          }
+      for (int e = 0; e < 4; ++e) {
+        // 16 significant bits: the upper half of the word holds eight of them, its remainder is a bf16 too
+        const float p0 = bf16_lo_to_f32(ki[x][e]) * bf16_lo_to_f32(vf[e]), p1 = bf16_hi_to_f32(ki[x][e]) * bf16_hi_to_f32(vf[e]);
+        const u32 b0 = __builtin_bit_cast(u32, p0), b1 = __builtin_bit_cast(u32, p1);
+        float r0 = p0 - bf16_hi_to_f32(b0), r1 = p1 - bf16_hi_to_f32(b1);
+        if (FAR) {
+          if (r0 == 0.f || __builtin_isinf(p0)) r0 = p0 == 0.f ? 0.f : __builtin_copysignf(tiny, p0);
+          if (r1 == 0.f || __builtin_isinf(p1)) r1 = p1 == 0.f ? 0.f : __builtin_copysignf(tiny, p1);
         }
-#pragma unroll
-        for (int x = 0; x < DT + 1; ++x) acc[x] = mfma32x32x16_f16(hi[x], vf, acc[x]);
-#pragma unroll
-        for (int x = 0; x < DT + 1; ++x) acc[x] = mfma32x32x16_f16(lo[x], vf, acc[x]);
+        hi[x][e] = __builtin_amdgcn_perm(b1, b0, 0x07060302u);
+        lo[x][e] = __builtin_amdgcn_perm(__builtin_bit_cast(u32, r1), __builtin_bit_cast(u32, r0), 0x07060302u);
       }
-    }
+#pragma unroll
+    for (int x = 0; x < DT + 1; ++x) acc[x] = mfma32x32x16(kf[x < DT ? x : DT - 1], hi[x < DT ? 0 : 1], acc[x]);
+#pragma unroll
+    for (int x = 0; x < DT + 1; ++x) acc[x] = mfma32x32x16(kf[x < DT ? x : DT - 1], lo[x < DT ? 0 : 1], acc[x]);
+  };
+  if (!linear) {
+    // one rule for the part: as a branch inside one loop the accumulators were copied between the two
+    int far = 0;
+    for (int c = c0 + tid; c < c1; c += 512) far |= p.far[(size_t)bh * nch + c] != 0u;
+    auto run = [&](auto far_tag) {
+      for (int s = 0; s < nst; ++s) {
+        const uint16_t* kt = next(s);
+#pragma unroll 2
+        for (int ks = 0; ks < TC / 16; ++ks) step(far_tag, kt, kt + 32 * DT * TC, 2 * ks + h);
+      }
+    };
+    if (__syncthreads_or(far))
+      run(std::true_type{});
+    else
+      run(std::false_type{});
   } else {
     // A operands a[x], B operands b[x] of this wave's products
-    const u32x4 one = {0x3c003c00u, 0x3c003c00u, 0x3c003c00u, 0x3c003c00u};   // fp16 1
+    const u32x4 one = {0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};   // bf16 1
     for (int s = 0; s < nst; ++s) {
       const uint16_t* kt = next(s);
       const uint16_t* vt = kt + 32 * DT * TC;
@@ -273,10 +256,10 @@ __global__ __launch_bounds__(512, 2) void sexport_kernel(const ExportParams p) {
         const u32x4 kf0 = frag(kt, n, u), kf1 = frag(kt, 32 * (DT - 1) + n, u), vf = frag(vt, n, u);
         const u32x4 a0 = w == 1 ? one : kf0, b0 = w <= 1 ? vf : w == 2 ? kf0 : one;
         const u32x4 a1 = w == 2 ? kf0 : kf1, b1 = w <= 1 ? vf : w == 2 ? kf1 : one;
-        acc[0] = mfma32x32x16_f16(a0, b0, acc[0]);
+        acc[0] = mfma32x32x16(a0, b0, acc[0]);
         if (DT == 2) {
-          acc[1] = mfma32x32x16_f16(a1, b1, acc[1]);
-          acc[2] = mfma32x32x16_f16(kf1, kf1, acc[2]);
+          acc[1] = mfma32x32x16(a1, b1, acc[1]);
+          acc[2] = mfma32x32x16(kf1, kf1, acc[2]);
         }
       }
     }
@@ -316,10 +299,9 @@ __global__ __launch_bounds__(512, 2) void sexport_kernel(const ExportParams p) {
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
         const int x = x0 + 16 * t;   // row x & 31 of tile (x >> 5) % 3 of wave x / 96
-        int e = 0;
         float f = 0.f;
-        o[t] = x < 4 * 3 * 32 ? where(x / 96, (x >> 5) % 3, x & 31, f, e) : -1;
-        y[t] = __builtin_ldexpf(sum[(x < 4 * 3 * 32 ? x : 0) * 32 + n] * f, e);
+        o[t] = x < 4 * 3 * 32 ? where(x / 96, (x >> 5) % 3, x & 31, f) : -1;
+        y[t] = sum[(x < 4 * 3 * 32 ? x : 0) * 32 + n] * f;
         old[t] = sin != nullptr && o[t] >= 0 ? sin[o[t]] : 0.f;
       }
 #pragma unroll
@@ -333,8 +315,7 @@ __global__ __launch_bounds__(512, 2) void sexport_kernel(const ExportParams p) {
     return j < i || j >= d ? -1 : (j == i ? 1 + d + i : off_row(d, i) + j - i - 1) * ld + c;
   };
   if (!linear) {
-    copy_out([&](int ww, int x, int r, float& f, int& e) {
-      e = 2 * ek + ev;
+    copy_out([&](int ww, int x, int r, float& f) {
       if (x >= NTILE || col >= dv) return -1;
       return quad(4 * g + ww + (x < DT ? 0 : 16 * DT), 32 * (x < DT ? x : DT - 1) + r, col, f);
     });
@@ -342,23 +323,18 @@ __global__ __launch_bounds__(512, 2) void sexport_kernel(const ExportParams p) {
   }
   // wave 0: k V; wave 1: the sum of V in every row of tile 0; column tile 0, wave 2: the Gram tiles
   // (0, 0), (0, 1), (1, 1); wave 3: the sums of k in every column
-  copy_out([&](int ww, int x, int r, float& f, int& e) {
+  copy_out([&](int ww, int x, int r, float& f) {
     const int j = 32 * x + r;
     if (ww == 0 || (ww == 3 && ct == 0 && n == 0)) {
       f = p.c_lin;
-      e = ww == 0 ? ek + ev : ek;
       const int c = ww == 0 ? col : dv;
       return x < DT && j < d && (ww == 3 || c < dv) ? (1 + j) * ld + c : -1;
     }
     if (ww == 1) {
       f = 1.0f;
-      e = ev;
       return x == 0 && r == 0 && col < dv ? col : -1;
     }
-    if (ww == 2 && ct == 0 && (DT == 2 || x == 0)) {
-      e = 2 * ek;
-      return quad((x == 2 ? 32 : 0) + r, (x >= 1 ? 32 : 0) + n, dv, f);
-    }
+    if (ww == 2 && ct == 0 && (DT == 2 || x == 0)) return quad((x == 2 ? 32 : 0) + r, (x >= 1 ? 32 : 0) + n, dv, f);
     return -1;
   });
   if (ct == 0 && tid == 0)
@@ -738,7 +714,7 @@ struct ExportLayout {
 };
 ExportLayout export_layout(int BH, int N, int d, int dv, const ExportParams& p) {
   ExportLayout L{};
-  L.kv = up256((size_t)BH * 2 * kMxParts * 4);
+  L.kv = up256((size_t)BH * ((N + TC - 1) / TC) * 4);
   L.parts = L.kv + up256((size_t)BH * ((N + TC - 1) / TC) * (32 * (d <= 32 ? 1 : 2) + 32 * p.nct) * TC * 2);
   L.total = L.parts + (p.parts > 1 ? (size_t)p.parts * BH * feat(d) * (dv + 1) * 4 : 0);
   return L;
@@ -831,7 +807,7 @@ int la_based_state_export(const void* k, const void* v, int in_dtype, const floa
   p.k = static_cast<const uint16_t*>(k);
   p.v = static_cast<const uint16_t*>(v);
   p.state_in = state_in_or_null;
-  p.mx = static_cast<u32*>(workspace);
+  p.far = static_cast<u32*>(workspace);
   const ExportLayout L = export_layout(B * H, N, d, dv, p);
   p.kv = reinterpret_cast<uint16_t*>(static_cast<char*>(workspace) + L.kv);
   float* parts = reinterpret_cast<float*>(static_cast<char*>(workspace) + L.parts);
@@ -843,9 +819,6 @@ int la_based_state_export(const void* k, const void* v, int in_dtype, const floa
   p.c_lin = (float)__builtin_sqrt(a2 / sd);
   p.c_diag = (float)(a2 / (sd * 1.4142135623730951));
   p.c_off = (float)(a2 / sd);
-  hipLaunchKernelGGL(smax_kernel, dim3(kMxParts * (unsigned)p.BH), dim3(256), 0, stream, p);
-  int e = (int)hipGetLastError();
-  if (e != 0) return e;
   const dim3 pgrid((unsigned)((N + TC - 1) / TC) * (unsigned)p.BH);
   const dim3 grid((unsigned)((long long)p.BH * p.nct * (p.ngrp + 1) * p.parts));
   const bool vec = d % 4 == 0 && dv % 4 == 0 && aligned(k, 8) && aligned(v, 8);
@@ -862,7 +835,7 @@ int la_based_state_export(const void* k, const void* v, int in_dtype, const floa
       hipLaunchKernelGGL((sprep_kernel<2, false>), pgrid, dim3(256), 0, stream, p);
     hipLaunchKernelGGL((sexport_kernel<2>), grid, dim3(512), 0, stream, p);
   }
-  e = (int)hipGetLastError();
+  const int e = (int)hipGetLastError();
   if (e != 0 || p.parts == 1) return e;
   const long long n = (long long)p.BH * feat(d) * (dv + 1);
   hipLaunchKernelGGL(scombine_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, parts, state_in_or_null,
