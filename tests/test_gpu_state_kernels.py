@@ -1,8 +1,7 @@
 """The state kernels of the segment-state shapes (la_based_state_export, la_based_state_apply) at the
-edges of their tiles, against 64 bits.  Bounds: every output is a fp32 sum of exact products (export)
-or of products with 22-bit state entries (apply), so it is off by at most (steps 2^-24 + 2^-21) times
-the sum of the magnitudes of its terms, steps the additions in a row (two MFMAs for each 16 tokens,
-and the parts; two for each 16 features)."""
+edges of their tiles, against 64 bits.  Bounds: every output is a fp32 sum of exact products, so it is off
+by at most steps 2^-24 times the sum of the magnitudes of its terms, steps the additions in a row (two
+MFMAs for each 16 tokens, and the parts; three for each 16 features)."""
 
 import math
 
@@ -170,6 +169,56 @@ def test_export_of_infinite_keys():
     big = got.abs() > 2e38
     assert torch.equal(big, inf) and torch.equal(got[big].sign(), want[inf].sign())
     assert ((got - want).abs()[~inf] / m[~inf]).max().item() < (300 / 8 + 16) * 2.0 ** -24
+
+
+def _apply(q, st, num, den, scale, eps, normalize):
+    B, H, N, d = q.shape
+    dv = num.shape[-1]
+    ws, n = _ws(B, H, N, d, dv)
+    qd, sd, nd, dd = (x.cuda() for x in (q, st, num, den))
+    out = torch.full((B, H, N, dv), float("nan"), device="cuda")
+    _call("la_based_state_apply", qd.data_ptr(), 1, sd.data_ptr(), nd.data_ptr(), dd.data_ptr(), out.data_ptr(), 0, B, H,
+          N, d, dv, scale, eps, normalize, ws.data_ptr(), n)
+    return out.cpu().double()
+
+
+@pytest.mark.parametrize("N,d,dv", [(300, 64, 64), (130, 32, 128), (70, 16, 24)])
+@pytest.mark.parametrize("what", ["columns", "entries", "queries"])
+def test_apply_of_uneven_inputs(N, d, dv, what):
+    """Value columns 2^-28 below the others, entries of the state of any power, one query channel far above
+    the rest: every output within the bound of its own terms (exact entries: no 2^-21)."""
+    q, _, _ = _inputs(1, 2, N, d, dv)
+    F = 1 + d + d * (d + 1) // 2
+    g = torch.Generator().manual_seed(N + len(what))
+    st = torch.randn(1, 2, F, dv + 1, generator=g)
+    if what == "columns":
+        st[..., 2:dv:8] *= 2.0 ** -28
+    elif what == "entries":
+        st = torch.ldexp(st, torch.randint(-40, 40, st.shape, generator=g))
+    else:
+        q[..., d // 3] *= 3e4
+    num, den = torch.zeros(1, 2, N, dv), torch.zeros(1, 2, N)
+    ph = _phi(q, 0.8 / math.sqrt(d))
+    want, mag = ph @ st[..., :dv].double(), ph.abs() @ st[..., :dv].abs().double()
+    off = ((_apply(q, st, num, den, 0.8 / math.sqrt(d), 0.0, 0) - want).abs() / mag).max().item()
+    assert off < (F / 8 + 16) * 2.0 ** -24, off
+
+
+def test_apply_of_infinite_entries():
+    """Infinite entries of the state make their column's numerators infinite, of the sign of the feature."""
+    q, _, _ = _inputs(1, 1, 200, 64, 64)
+    st = torch.randn(1, 1, 2145, 65, generator=torch.Generator().manual_seed(3))
+    rows = (3, 70, 1000)        # a linear, a square and an off-diagonal feature
+    for f, c in zip(rows, (0, 5, 40)):
+        st[0, 0, f, c] = float("inf")
+    num, den = torch.zeros(1, 1, 200, 64), torch.zeros(1, 1, 200)
+    ph = _phi(q, 0.125)
+    assert (ph != 0).all()
+    got = _apply(q, st, num, den, 0.125, 0.0, 0)
+    want, mag = ph @ st[..., :64].double(), ph.abs() @ st[..., :64].abs().double()
+    inf = want.isinf()
+    assert inf[..., [0, 5, 40]].all() and torch.equal(got[inf], want[inf])
+    assert ((got - want).abs()[~inf] / mag[~inf]).max().item() < (2145 / 8 + 16) * 2.0 ** -24
 
 
 def _need_gib(n):

@@ -8,20 +8,20 @@
 // Precision.  Both directions stand in for fp32 products of phi with V or with the state, so every
 // operand keeps its bits.  Export: a product k_i v has at most 16 significant bits and is carried as
 // bf16 hi + lo, exactly and over the whole range of fp32, against the bf16 rows of k: no channel,
-// column or token takes bits from another.  Import: a state entry is carried as fp16 hi + lo (22 bits)
-// with one exponent per feature row i, q exact in fp16 after a power of two.  Sums are fp32.  Relative
-// error (2-norm) against 64 bits, against fp32 phi and fp32 GEMMs on the same inputs: quadratic state
-// rows at B1 H4 N3001 d64 dv64 1.1e-7 (9.0e-7); the first 64 outputs after a state of 500 tokens
-// 6.7e-7 (1.5e-6).
+// column or token takes bits from another.  Import: a state entry is carried as three bf16 parts
+// (24 bits, exactly) against the bf16 rows of q.  Sums are fp32.  Relative error (2-norm) against 64
+// bits, against fp32 phi and fp32 GEMMs on the same inputs: quadratic state rows at B1 H4 N3001 d64
+// dv64 1.1e-7 (9.0e-7); the first 64 outputs after a state of 500 tokens 6.4e-7 (1.4e-6), of a column
+// of v 2^-28 below the others 4.1e-7 (1.2e-6).
 //
-// Measured at B1 H16 N3001 d64 dv64 (us): prep 8 + export 66, pack 11 + apply 54, where
+// Measured at B1 H16 N3001 d64 dv64 (us): prep 8 + export 66, pack 9 + apply 65, where
 // phi written to memory and GEMMs took 1210.
 //
 //   sprep_kernel    64-token chunks of k and v transposed to rows of tokens, once
 //   sexport_kernel  state rows from those: work-group = (head, 32 value columns, four i0), the
 //                   chunks through an LDS ring; parts of the sequence where heads are few, added
 //                   by scombine_kernel in order (no atomics)
-//   spack_kernel    a state's rows as fp16 hi / lo MFMA fragments, 1 KB each, i-major
+//   spack_kernel    a state's rows as bf16 MFMA fragments in three parts, 1 KB each, i-major
 //   sapply_kernel   phi(a q) [S | z] added to a numerator and denominator, and the division
 #include <type_traits>
 
@@ -353,17 +353,16 @@ __global__ __launch_bounds__(256) void scombine_kernel(const float* __restrict__
 
 // ---------------------------------------------------------------- import
 // Fragments of a state: for every feature row i (0 .. DP - 1, then the linear row DP) and 16-wide
-// block J of j (from block i / 16; all blocks of the linear row), for every 32-column tile the
-// fp16 hi and lo parts of M_i[column][j] 2^-E_i as A operands (lane: column n, j = 16 J + 8 h ..),
+// block J of j (from block i / 16; all blocks of the linear row), for every 32-column tile the three
+// bf16 parts of M_i[column][j] as A operands (lane: column n, j = 16 J + 8 h ..),
 // M_i[.][j] = S(i, j) for j > i, S(i, i) / sqrt(2) (so that one factor a^2 / sqrt(d) serves the
-// row), zero for j < i.  Then Z(i, j), the K-sums the same way, as DT x DB x {hi, lo} fragments
-// with rows i, one exponent per row.
+// row), zero for j < i.  Then Z(i, j), the K-sums the same way, as DT x DB x 3 fragments with rows i.
 template <int DP>
 struct SPack {
   static constexpr int DB = DP / 16, DT = (DP + 31) / 32;
   static constexpr int NQ = 8 * DB * (DB + 1);     // quadratic blocks (i, J)
   static constexpr int NBLK = NQ + DB;             // + the linear row's
-  static constexpr int ZU = 2 * DT * DB;           // 1 KB units of Z
+  static constexpr int ZU = 3 * DT * DB;           // 1 KB units of Z
   static __host__ __device__ constexpr int first(int i) {   // block index of (i, i / 16)
     const int I = i / 16;
     return 16 * (I * DB - I * (I - 1) / 2) + (i - 16 * I) * (DB - I);
@@ -379,15 +378,12 @@ struct ApplyParams {
   const float* num;       // (BH, N, dv), without the state's part
   const float* den;       // (BH, N)
   void* out;
-  uint16_t* frag;         // [BH][NBLK][MT][2][512], then [BH][ZU][512]
+  uint16_t* frag;         // [BH][NBLK][MT][3][512], then [BH][ZU][512]
   uint16_t* zfrag;
-  int* E;                 // [BH][2 DP + 1]: rows, linear row (DP), rows of Z; kNoRow for all-zero rows
   int BH, N, d, dv;
   float c_lin, c_off, eps;
   int normalize, out_f32;
 };
-
-constexpr int kNoRow = -100000;
 
 // Work-group (i, head): i < DP a feature row, DP the linear row; its state rows (j >= i) through
 // LDS, once.
@@ -396,17 +392,11 @@ __global__ __launch_bounds__(256) void spack_kernel(const ApplyParams p) {
   using SP = SPack<DP>;
   constexpr int DB = SP::DB;
   __shared__ float row[DP * (32 * MT + 1)];
-  __shared__ u32 wm[2][4];
   const int tid = threadIdx.x, bh = blockIdx.x / (DP + 1), i = blockIdx.x - bh * (DP + 1), d = p.d, dv = p.dv, ld = dv + 1;
   const float* __restrict__ S = p.state + (size_t)bh * feat(d) * ld;
   const int j0 = i < DP ? i : 0, cnt = i < d || i == DP ? d - j0 : 0;   // rows j0 .. d - 1 (none past d)
   // row j0 of a quadratic i is its square; the others follow each other in memory
   const float* __restrict__ rest = i < DP ? S + (size_t)(off_row(d, i) - 1) * ld : S + ld;
-  u32 m = 0u, mz = 0u;
-  const auto fin = [](float y) {
-    const u32 b = __builtin_bit_cast(u32, __builtin_fabsf(y));
-    return b < 0x7f800000u ? b : 0u;
-  };
   constexpr int PF = 8;   // loads in flight per thread
   for (int x0 = tid; x0 < cnt * ld; x0 += 256 * PF) {
     float y[PF];
@@ -420,71 +410,59 @@ __global__ __launch_bounds__(256) void spack_kernel(const ApplyParams p) {
       if (x0 + 256 * u < cnt * ld) row[x0 + 256 * u] = y[u];
   }
   __syncthreads();
-  {   // largest finite entries of the value columns and of the K-sum column: wave w rows w, w + 4, ...
-    const int lane = tid & 63;
-    for (int r = tid >> 6; r < cnt; r += 4) {
-      for (int c = lane; c < dv; c += 64) m = max(m, fin(row[r * ld + c]));
-      if (lane == 0) mz = max(mz, fin(row[r * ld + dv]));
-    }
-  }
-  m = wave_max_u32(m);
-  mz = wave_max_u32(mz);
-  if ((tid & 63) == 0) {
-    wm[0][tid >> 6] = m;
-    wm[1][tid >> 6] = mz;
-  }
-  __syncthreads();
-  m = max(max(wm[0][0], wm[0][1]), max(wm[0][2], wm[0][3]));
-  mz = max(max(wm[1][0], wm[1][1]), max(wm[1][2], wm[1][3]));
-  // largest entry in [2^14, 2^15)
-  const int E = m == 0u ? 0 : (int)(m >> 23) - 127 - 14, EZ = mz == 0u ? 0 : (int)(mz >> 23) - 127 - 14;
-  int* Eh = p.E + (size_t)bh * (2 * DP + 1);
-  if (tid == 0) Eh[i] = m == 0u ? kNoRow : E;
-  if (tid == 0 && i < DP) Eh[DP + 1 + i] = mz == 0u ? kNoRow : EZ;
-  // a 16-byte unit: column c, rows j .. j + 7; hi, and lo 512 halves later
-  auto put = [&](uint16_t* dst, int j, int c, int e) {
-    u32x4 hi, lo;
+  // a 16-byte unit: column c, rows j .. j + 7; the second and third parts 512 and 1024 halves later.  A
+  // part is the upper half of the word, exactly what it leaves the next one; infinities leave nothing.
+  auto put = [&](uint16_t* dst, int j, int c) {
+    u32x4 p[3];
 #pragma unroll
     for (int x = 0; x < 4; ++x) {
-      float y[2];
+      u32 b[2][3];
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
         const int r = j + 2 * x + t - j0;
-        y[t] = r >= 0 && r < cnt && c < ld ? __builtin_ldexpf(row[r * ld + c], -e) : 0.f;
+        float y = r >= 0 && r < cnt && c < ld ? row[r * ld + c] : 0.f;
+        const bool fin = __builtin_fabsf(y) < __builtin_inff();
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          b[t][k] = y != y ? 0x7fc00000u : __builtin_bit_cast(u32, y) & 0xffff0000u;
+          y = fin ? y - __builtin_bit_cast(float, b[t][k]) : 0.f;
+        }
       }
-      hi[x] = pack_f16x2(y[0], y[1]);
-      lo[x] = pack_f16x2(y[0] - f16_lo_to_f32(hi[x]), y[1] - f16_hi_to_f32(hi[x]));
+#pragma unroll
+      for (int k = 0; k < 3; ++k) p[k][x] = (b[0][k] >> 16) | b[1][k];
     }
-    *reinterpret_cast<u32x4*>(dst) = hi;
-    *reinterpret_cast<u32x4*>(dst + 512) = lo;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) *reinterpret_cast<u32x4*>(dst + 512 * k) = p[k];
   };
   const int J0 = i < DP ? i / 16 : 0, b0 = i < DP ? SP::first(i) : SP::NQ;
-  uint16_t* dst = p.frag + ((size_t)bh * SP::NBLK + b0) * (MT * 1024);
+  uint16_t* dst = p.frag + ((size_t)bh * SP::NBLK + b0) * (MT * 1536);
   for (int x = tid; x < (DB - J0) * MT * 64; x += 256) {
     const int l = x & 63, mt = (x >> 6) % MT, J = J0 + (x >> 6) / MT, c = 32 * mt + (l & 31);
-    put(dst + ((size_t)(J - J0) * MT + mt) * 1024 + 8 * l, 16 * J + 8 * (l >> 5), c < dv ? c : ld, E);
+    put(dst + ((size_t)(J - J0) * MT + mt) * 1536 + 8 * l, 16 * J + 8 * (l >> 5), c < dv ? c : ld);
   }
   if (i < DP && tid < 2 * DB) {   // Z's row i: lanes i % 32 and i % 32 + 32 of its fragments
     const int J = tid >> 1, h = tid & 1;
-    put(p.zfrag + (size_t)bh * SP::ZU * 512 + (size_t)((i >> 5) * DB + J) * 1024 + 8 * ((i & 31) + 32 * h),
-        16 * J + 8 * h, dv, EZ);
+    put(p.zfrag + (size_t)bh * SP::ZU * 512 + (size_t)((i >> 5) * DB + J) * 1536 + 8 * ((i & 31) + 32 * h),
+        16 * J + 8 * h, dv);
   }
 }
 
 // Work-group: 128 QT queries of one head, 4 MT waves: wave w takes 32 QT queries (w % 4) and value
-// columns 32 (w / 4) .. + 31.  Per feature row i: Y = M_i q~ on MFMAs (A the row's fragments from
-// an LDS ring, B the wave's queries, resident), then acc += (q~_i 2^(E_i - E_max)) Y: 16 QT fused
-// multiply-adds against 2 QT x (blocks of the row) MFMAs.  Matrix-core bound once the ring's
-// copies are hidden: a fragment (1 KB) feeds QT MFMAs of four waves.  QT = 1 is taken where
-// 256-query work-groups would leave half of the CUs idle.
+// columns 32 (w / 4) .. + 31.  Per feature row i: Y = M_i q on MFMAs (A the row's fragments from
+// an LDS ring, B the wave's queries, resident), then acc += q_i Y: 16 QT fused multiply-adds against
+// 3 QT x (blocks of the row) MFMAs.  Matrix-core bound once the ring's copies are hidden: a fragment
+// (1 KB) feeds QT MFMAs of four waves.  QT = 1 is taken where 256-query work-groups would leave half of
+// the CUs idle, and at MT = 4, whose 16 waves have 128 VGPRs each (QT = 2 spills 27 of them: B2 H16
+// N3001 d64 dv128 238 us, 211 so).  (Two fp16 parts with an exponent per feature row took 54 us, and lost the bits of
+// columns far below the row's largest.)
 template <int DP, int MT, int QT, bool VEC>
 __global__ __launch_bounds__(256 * MT, MT) void sapply_kernel(const ApplyParams p) {
   using SP = SPack<DP>;
   constexpr int DB = SP::DB, DT = SP::DT, NBLK = SP::NBLK, TQ = 128 * QT;
   constexpr int GB = 4;                            // blocks per stage
-  constexpr int UB = 2 * MT, SU = GB * UB;         // 1 KB units per block and per stage
+  constexpr int UB = 3 * MT, SU = GB * UB;         // 1 KB units per block and per stage
   constexpr int CW = SU / (4 * MT);                // copies per wave and stage
-  constexpr int NST = (NBLK + GB - 1) / GB, NS = MT == 4 ? 3 : 4;
+  constexpr int NST = (NBLK + GB - 1) / GB, NS = MT == 4 ? 2 : 4;
   __shared__ __attribute__((aligned(16))) uint16_t ring[NS][SU * 512];
   __shared__ __attribute__((aligned(16))) uint16_t Aq[DP * TQ];
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), h = lane >> 5, n = lane & 31;
@@ -492,9 +470,8 @@ __global__ __launch_bounds__(256 * MT, MT) void sapply_kernel(const ApplyParams 
   const int N = p.N, d = p.d, dv = p.dv, ld = dv + 1;
   const int bh = blockIdx.x % p.BH, t0 = (blockIdx.x / p.BH) * TQ;
   const float* __restrict__ S = p.state + (size_t)bh * feat(d) * ld;
-  const int* __restrict__ Eh = p.E + (size_t)bh * (2 * DP + 1);
 
-  const u32x4 rf = buffer_rsrc(p.frag + (size_t)bh * NBLK * (MT * 1024), (u32)(NBLK * MT * 2048));
+  const u32x4 rf = buffer_rsrc(p.frag + (size_t)bh * NBLK * (MT * 1536), (u32)(NBLK * MT * 3072));
   auto issue = [&](int s) {   // past the last stage nothing is read, so that every wave's counts agree
     const u32 base = lds_addr(&ring[s % NS][0]);
 #pragma unroll
@@ -509,53 +486,30 @@ __global__ __launch_bounds__(256 * MT, MT) void sapply_kernel(const ApplyParams 
 #pragma unroll
   for (int s = 0; s < NS - 1; ++s) issue(s);
 
-  // ---- queries: fp16(q 2^-eq) fragments, eq such that a token's largest |q~| is in [64, 128)
+  // ---- queries: fragments, and a table [dim][query] for the factors q_i
   u32x4 qf[QT][DB];
-  int eq[QT];
 #pragma unroll
   for (int qt = 0; qt < QT; ++qt) {
     const int tok = t0 + 32 * QT * w + 32 * qt + n;
-    u32x4 x[DB];
-    u32 m = 0u;
 #pragma unroll
     for (int J = 0; J < DB; ++J) {
-      x[J] = load_row8<VEC>(p.q + ((size_t)bh * N + tok) * d, 16 * J + 8 * h, d, tok < N);
+      qf[qt][J] = load_row8<VEC>(p.q + ((size_t)bh * N + tok) * d, 16 * J + 8 * h, d, tok < N);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const u32 a = x[J][e] & 0x7fffu, b = (x[J][e] >> 16) & 0x7fffu;
-        m = max(m, max(a < 0x7f80u ? a : 0u, b < 0x7f80u ? b : 0u));
-      }
-    }
-    m = max(m, (u32)__shfl_xor((int)m, 32));
-    eq[qt] = m == 0u ? 0 : (int)(m >> 7) - 127 - 6;
-#pragma unroll
-    for (int J = 0; J < DB; ++J)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const u32 y = pack_f16x2(__builtin_ldexpf(bf16_lo_to_f32(x[J][e]), -eq[qt]),
-                                 __builtin_ldexpf(bf16_hi_to_f32(x[J][e]), -eq[qt]));
-        qf[qt][J][e] = y;
+      for (int e = 0; e < 4; ++e)
         if (mt == 0) {
           uint16_t* a = Aq + (16 * J + 8 * h + 2 * e) * TQ + 32 * QT * w + 32 * qt + n;
-          a[0] = (uint16_t)(y & 0xffffu);
-          a[TQ] = (uint16_t)(y >> 16);
+          a[0] = (uint16_t)(qf[qt][J][e] & 0xffffu);
+          a[TQ] = (uint16_t)(qf[qt][J][e] >> 16);
         }
-      }
+    }
   }
-  // lane i: row i's weight 2^(E_i - E_max) and its K-sum row's; its linear K-sum
-  const int er = lane < DP ? Eh[lane] : kNoRow, ezr = lane < DP ? Eh[DP + 1 + lane] : kNoRow;
-  const int emax = (int)wave_max_u32((u32)(er - 2 * kNoRow)) + 2 * kNoRow;
-  const int ezmax = (int)wave_max_u32((u32)(ezr - 2 * kNoRow)) + 2 * kNoRow;
-  const float wrow = er == kNoRow ? 0.f : __builtin_ldexpf(1.0f, er - emax);
-  const float zrow = ezr == kNoRow ? 0.f : __builtin_ldexpf(1.0f, ezr - ezmax);
-  const float zlin = lane < d ? S[(size_t)(1 + lane) * ld + dv] : 0.f;
-  const int el = Eh[DP];
+  const float zlin = lane < d ? S[(size_t)(1 + lane) * ld + dv] : 0.f;   // the linear K-sum of lane i
   const float z0 = S[dv];
   auto from_lane = [](float x, int l) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), l));
   };
 
-  // ---- denominator: q~^T Z q~ and the linear K-sums
+  // ---- denominator: q^T Z q and the linear K-sums
   float den[QT];
   {
     const u32x4* __restrict__ zf = reinterpret_cast<const u32x4*>(p.zfrag + (size_t)bh * SP::ZU * 512);
@@ -567,13 +521,13 @@ __global__ __launch_bounds__(256 * MT, MT) void sapply_kernel(const ApplyParams 
 #pragma unroll
       for (int J = 0; J < DB; ++J)
 #pragma unroll
-        for (int x = 0; x < 2; ++x) {
-          const u32x4 a = zf[((rt * DB + J) * 2 + x) * 64 + lane];
+        for (int x = 0; x < 3; ++x) {
+          const u32x4 a = zf[((rt * DB + J) * 3 + x) * 64 + lane];
 #pragma unroll
-          for (int qt = 0; qt < QT; ++qt) Y[qt][rt] = mfma32x32x16_f16(a, qf[qt][J], Y[qt][rt]);
+          for (int qt = 0; qt < QT; ++qt) Y[qt][rt] = mfma32x32x16(a, qf[qt][J], Y[qt][rt]);
         }
     }
-    __syncthreads();   // the q~ table
+    __syncthreads();   // the table of q
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt) {
       const uint16_t* aq = Aq + 32 * QT * w + 32 * qt + n;
@@ -584,19 +538,17 @@ __global__ __launch_bounds__(256 * MT, MT) void sapply_kernel(const ApplyParams 
         for (int r = 0; r < 16; ++r) {
           const int i0 = 32 * rt + c32_row(r, 0);   // row i0 + 4 h
           if (i0 >= DP) continue;
-          const float z = h ? from_lane(zrow, i0 + 4) : from_lane(zrow, i0);
-          dq = __builtin_fmaf(f16_lo_to_f32(aq[(i0 + 4 * h) * TQ]) * z, Y[qt][rt][r], dq);
+          dq = __builtin_fmaf(bf16_bits_to_f32(aq[(i0 + 4 * h) * TQ]), Y[qt][rt][r], dq);
         }
 #pragma unroll 4
       for (int i = 0; i < DP / 2; ++i) {   // lane half h sums rows h DP / 2 ..
         const float za = from_lane(zlin, i), zb = from_lane(zlin, i + DP / 2);
-        dl = __builtin_fmaf(f16_lo_to_f32(aq[(i + h * (DP / 2)) * TQ]), h ? zb : za, dl);
+        dl = __builtin_fmaf(bf16_bits_to_f32(aq[(i + h * (DP / 2)) * TQ]), h ? zb : za, dl);
       }
       dq += __shfl_xor(dq, 32);
       dl += __shfl_xor(dl, 32);
       const int tok = min(t0 + 32 * QT * w + 32 * qt + n, N - 1);
-      den[qt] = p.den[(size_t)bh * N + tok] + z0 + __builtin_ldexpf(dl * p.c_lin, eq[qt]) +
-                (ezmax == kNoRow ? 0.f : __builtin_ldexpf(dq * p.c_off, 2 * eq[qt] + ezmax));
+      den[qt] = p.den[(size_t)bh * N + tok] + z0 + dl * p.c_lin + dq * p.c_off;
     }
   }
 
@@ -617,12 +569,12 @@ __global__ __launch_bounds__(256 * MT, MT) void sapply_kernel(const ApplyParams 
         asm volatile("" ::: "memory");
         issue(b / GB + NS - 1);
       }
-      const u32x4* st = reinterpret_cast<const u32x4*>(&ring[(b / GB) % NS][((b & (GB - 1)) * UB + 2 * mt) * 512]);
+      const u32x4* st = reinterpret_cast<const u32x4*>(&ring[(b / GB) % NS][((b & (GB - 1)) * UB + 3 * mt) * 512]);
 #pragma unroll
-      for (int x = 0; x < 2; ++x) {
+      for (int x = 0; x < 3; ++x) {
         const u32x4 a = st[x * 64 + lane];
 #pragma unroll
-        for (int qt = 0; qt < QT; ++qt) Y[qt] = mfma32x32x16_f16(a, qf[qt][J], Y[qt]);
+        for (int qt = 0; qt < QT; ++qt) Y[qt] = mfma32x32x16(a, qf[qt][J], Y[qt]);
       }
       ++b;
     }
@@ -635,10 +587,9 @@ __global__ __launch_bounds__(256 * MT, MT) void sapply_kernel(const ApplyParams 
 #pragma unroll
       for (int qt = 0; qt < QT; ++qt) Y[qt] = splat16(0.f);
       row(I, Y);
-      const float wi = from_lane(wrow, i);
 #pragma unroll
       for (int qt = 0; qt < QT; ++qt) {
-        const float a = f16_lo_to_f32(Aq[i * TQ + 32 * QT * w + 32 * qt + n]) * wi;
+        const float a = bf16_bits_to_f32(Aq[i * TQ + 32 * QT * w + 32 * qt + n]);
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[qt][r] = __builtin_fmaf(a, Y[qt][r], acc[qt][r]);
       }
@@ -681,8 +632,7 @@ __global__ __launch_bounds__(256 * MT, MT) void sapply_kernel(const ApplyParams 
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int r = 4 * q4 + e;
-        const float x = (emax == kNoRow ? 0.f : __builtin_ldexpf(acc[qt][r] * p.c_off, 2 * eq[qt] + emax)) +
-                        (el == kNoRow ? 0.f : __builtin_ldexpf(Yl[qt][r] * p.c_lin, eq[qt] + el));
+        const float x = acc[qt][r] * p.c_off + Yl[qt][r] * p.c_lin;
         y[e] = (num[qt][q4][e] + (x + s0[q4][e])) * inv;
       }
       store_out4<VEC>(p.out, p.out_f32 != 0, ob, 32 * mt + 8 * q4 + 4 * h, dv, y);
@@ -726,14 +676,13 @@ size_t export_bytes(int BH, int N, int d, int dv) {
 }
 
 struct ApplyLayout {
-  size_t z, e, total;
+  size_t z, total;
 };
 ApplyLayout apply_layout(int BH, int d, int dv) {
   const int DP = dp_of(d), DB = DP / 16, DT = (DP + 31) / 32, nblk = 8 * DB * (DB + 1) + DB;
   ApplyLayout L{};
-  L.z = up256((size_t)BH * nblk * mt_of(dv) * 2048);
-  L.e = L.z + up256((size_t)BH * 2 * DT * DB * 1024);
-  L.total = L.e + up256((size_t)BH * (2 * DP + 1) * 4);
+  L.z = up256((size_t)BH * nblk * mt_of(dv) * 3072);
+  L.total = L.z + up256((size_t)BH * 3 * DT * DB * 1024);
   return L;
 }
 
@@ -747,17 +696,19 @@ int launch_apply(const ApplyParams& p, hipStream_t stream) {
   const bool vec = p.d % 8 == 0 && p.dv % 4 == 0 && aligned(p.q, 16) && aligned(p.out, 16) && aligned(p.num, 16);
   const unsigned wg2 = (unsigned)p.BH * (unsigned)((p.N + 255) / 256), wg1 = (unsigned)p.BH * (unsigned)((p.N + 127) / 128);
   const dim3 block(256 * MT);
-  if ((int)wg1 > device_cu_count()) {
-    if (vec)
-      hipLaunchKernelGGL((sapply_kernel<DP, MT, 2, true>), dim3(wg2), block, 0, stream, p);
-    else
-      hipLaunchKernelGGL((sapply_kernel<DP, MT, 2, false>), dim3(wg2), block, 0, stream, p);
-  } else {
-    if (vec)
-      hipLaunchKernelGGL((sapply_kernel<DP, MT, 1, true>), dim3(wg1), block, 0, stream, p);
-    else
-      hipLaunchKernelGGL((sapply_kernel<DP, MT, 1, false>), dim3(wg1), block, 0, stream, p);
+  if constexpr (MT < 4) {
+    if ((int)wg1 > device_cu_count()) {
+      if (vec)
+        hipLaunchKernelGGL((sapply_kernel<DP, MT, 2, true>), dim3(wg2), block, 0, stream, p);
+      else
+        hipLaunchKernelGGL((sapply_kernel<DP, MT, 2, false>), dim3(wg2), block, 0, stream, p);
+      return (int)hipGetLastError();
+    }
   }
+  if (vec)
+    hipLaunchKernelGGL((sapply_kernel<DP, MT, 1, true>), dim3(wg1), block, 0, stream, p);
+  else
+    hipLaunchKernelGGL((sapply_kernel<DP, MT, 1, false>), dim3(wg1), block, 0, stream, p);
   return (int)hipGetLastError();
 }
 
@@ -869,7 +820,6 @@ int la_based_state_apply(const void* q, int in_dtype, const float* state, const 
   p.out = out;
   p.frag = static_cast<uint16_t*>(workspace);
   p.zfrag = reinterpret_cast<uint16_t*>(static_cast<char*>(workspace) + L.z);
-  p.E = reinterpret_cast<int*>(static_cast<char*>(workspace) + L.e);
   p.BH = B * H;
   p.N = N;
   p.d = d;
