@@ -43,6 +43,27 @@ def test_edges(B, H, N, d, dv, scale):
     assert torch.equal(K.based_parallel(q, k, v, scale=scale), y.bfloat16())
 
 
+@pytest.mark.parametrize("dv", [32, 64])
+@pytest.mark.parametrize("scale", [None, 0.3])
+def test_d16_denominators_from_fp32_sums(dv, scale):
+    """d = 16 calls on small grids that return denominators sum u in fp32: q.k sums 17 products in fp32, whose
+    error e moves p by (1 + |s|) e, and N fp32 sums; nothing of fp16's 2^-11.  The output is that of a call
+    without."""
+    import kernels as K
+    N = 900
+    q, k, v = rand_qkv(1, 4, N, 16, dv, seed=dv, dtype=torch.bfloat16, scale_qk=1.0)
+    y, den = K.based_parallel(q.cuda(), k.cuda(), v.cuda(), scale=scale, out_dtype=torch.float32, return_den=True)
+    assert torch.equal(y, K.based_parallel(q.cuda(), k.cuda(), v.cuda(), scale=scale, out_dtype=torch.float32))
+    q, k, c = q.double(), k.double(), 0.25 if scale is None else scale
+    s = c * q @ k.transpose(-2, -1)
+    one = torch.tril(torch.ones(N, N, dtype=torch.float64))
+    p = (1.0 + s + 0.5 * s * s) * one
+    reach = c * q.abs() @ k.abs().transpose(-2, -1) + 1.0
+    bound = ((1.0 + s.abs()) * 18 * 2.0 ** -24 * reach * one + (N / 8 + 16) * 2.0 ** -24 * (p + 2 * one)).sum(-1)
+    off = ((den.double().cpu() - p.sum(-1)).abs() / bound).max().item()
+    assert off < 1, off
+
+
 @pytest.mark.parametrize("dv", [32, 64, 128])
 def test_v_exponents(dv):
     """Blocks of V that differ by many powers of two (one of them zero): each wave takes the largest

@@ -187,9 +187,13 @@ __global__ __launch_bounds__(256) void wide_pack_kernel(const WideParams p) {
 
 // ---------------------------------------------------------------- attention
 // KS: 16-wide steps of d; MT: 32-wide tiles of dv; QT: 32-query tiles per wave; NKH: waves sharing a
-// query group (2: each takes one 32-key half of every block).  UNIT: 1/c scales to exactly 1/2.
-template <int KS, int MT, int QT, int NKH, bool UNIT, bool ANY>
-__global__ __launch_bounds__(256, KS == 1 && MT == 1 ? 3 : 2) void wide_kernel(const WideParams p) {
+// query group (2: each takes one 32-key half of every block).  UNIT: 1/c scales to exactly 1/2.  ROWS:
+// calls of the packed kernel's shapes that return denominators, which that kernel takes from fp32
+// statistics: row sums of u in fp32 beside those of its fp16 form, which divide the output as in calls
+// without (B2 H4 N2048 d16 dv64, q and k four times the benchmark's, denominators of rows 64 to 512:
+// 1.0e-5 off from the fp16 sums, 3.6e-8 so, packed 3.3e-6).
+template <int KS, int MT, int QT, int NKH, bool UNIT, bool ANY, bool ROWS>
+__global__ __launch_bounds__(256, KS == 1 && MT == 1 && !ROWS ? 3 : 2) void wide_kernel(const WideParams p) {
   constexpr int DV = 32 * MT, NQW = 4 / NKH, BM = 32 * QT * NQW;
   constexpr int UB = NKH;                           // blocks per step (two 32-key units per wave either way)
   constexpr int UK = 2 * KS, UV = 4 * MT;           // 1 KB copy units of a block
@@ -360,10 +364,10 @@ __global__ __launch_bounds__(256, KS == 1 && MT == 1 ? 3 : 2) void wide_kernel(c
   }
 
   f32x16 acc[QT][MT];
-  float rsum[QT];
+  float rsum[QT], rsx[QT];
 #pragma unroll
   for (int qt = 0; qt < QT; ++qt) {
-    rsum[qt] = 0.f;
+    rsum[qt] = rsx[qt] = 0.f;
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) acc[qt][mt] = splat16(0.f);
   }
@@ -405,6 +409,7 @@ __global__ __launch_bounds__(256, KS == 1 && MT == 1 ? 3 : 2) void wide_kernel(c
           const float b0 = b[qt][8 * m + 2 * c], b1 = b[qt][8 * m + 2 * c + 1];
           pf[qt][m][c] = NEAR ? sq_plus_f16x2(b0 * f, b1 * f, cc) : sq_plus_f16x2(b0, b1, -inv_c2);
           rsum[qt] = dot2_f16(pf[qt][m][c], NEAR ? ones : kOnes, rsum[qt]);
+          if (ROWS) rsx[qt] += __builtin_fmaf(b0, b0, -inv_c2) + __builtin_fmaf(b1, b1, -inv_c2);
         }
   };
   auto P = [&](const uint16_t* st, int ks, const u32x4 (&pf)[QT][2]) {
@@ -465,7 +470,9 @@ __global__ __launch_bounds__(256, KS == 1 && MT == 1 ? 3 : 2) void wide_kernel(c
           x[0][qt][m][c] = pack_f16x2(in0 ? u0 : 0.f, in1 ? u1 : 0.f);
           x[1][qt][m][c] = (in0 ? whi & 0xffffu : 0u) | (in1 ? whi & 0xffff0000u : 0u);
           x[2][qt][m][c] = (in0 ? wlo & 0xffffu : 0u) | (in1 ? wlo & 0xffff0000u : 0u);
-          if (act[qt]) rsum[qt] = dot2_f16(x[0][qt][m][c], kOnes, rsum[qt]);
+          if (!act[qt]) continue;
+          rsum[qt] = dot2_f16(x[0][qt][m][c], kOnes, rsum[qt]);
+          if (ROWS) rsx[qt] += (in0 ? u0 : 0.f) + (in1 ? u1 : 0.f);
         }
     }
     Pscaled(st, ks, x, !diag ? 1 : p.ones_lo != 0u ? 3 : 2, act, e);
@@ -599,26 +606,31 @@ __global__ __launch_bounds__(256, KS == 1 && MT == 1 ? 3 : 2) void wide_kernel(c
   static_assert(NKH == 1 || QT == 2, "a wave pair finishes one tile each");
   const int e0 = NKH == 2 ? kh : 0;
   f32x16 fin[QE][MT];
-  float rs[QE];
+  float rs[QE], rx[QE];
   if constexpr (NKH == 2) {
-    float* mine = reinterpret_cast<float*>(&ring[0][0]) + wv * ((16 * MT + 1) * 64) + lane;
-    float* other = reinterpret_cast<float*>(&ring[0][0]) + (wv ^ 1) * ((16 * MT + 1) * 64) + lane;
+    constexpr int PW = (16 * MT + 2) * 64;   // floats of a wave's part
+    static_assert(4 * PW * 4 <= (int)sizeof(ring), "parts fit in the ring");
+    float* mine = reinterpret_cast<float*>(&ring[0][0]) + wv * PW + lane;
+    float* other = reinterpret_cast<float*>(&ring[0][0]) + (wv ^ 1) * PW + lane;
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
       for (int r = 0; r < 16; ++r) mine[(16 * mt + r) * 64] = kh ? acc[0][mt][r] : acc[1][mt][r];
     mine[16 * MT * 64] = kh ? rsum[0] : rsum[1];
+    if (ROWS) mine[16 * MT * 64 + 64] = kh ? rsx[0] : rsx[1];
     __syncthreads();
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
       for (int r = 0; r < 16; ++r) fin[0][mt][r] = (kh ? acc[1][mt][r] : acc[0][mt][r]) + other[(16 * mt + r) * 64];
     rs[0] = (kh ? rsum[1] : rsum[0]) + other[16 * MT * 64];
+    rx[0] = ROWS ? (kh ? rsx[1] : rsx[0]) + other[16 * MT * 64 + 64] : 0.f;
     __syncthreads();   // read before the output tiles take their place
   } else {
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt) {
       rs[qt] = rsum[qt];
+      rx[qt] = rsx[qt];
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) fin[qt][mt] = acc[qt][mt];
     }
@@ -642,7 +654,8 @@ __global__ __launch_bounds__(256, KS == 1 && MT == 1 ? 3 : 2) void wide_kernel(c
       const float r2 = rs[qe] + __shfl_xor(rs[qe], 32);
       const float den = (float)(ANY ? BN * jraw : query + 1) + fscale * r2;
       const float inv = p.normalize ? 1.0f / (den + p.eps) : 1.0f;
-      if (p.den != nullptr && h == 0 && query < N) p.den[hrow + query] = den;
+      const float x2 = ROWS ? rx[qe] + __shfl_xor(rx[qe], 32) : 0.f;
+      if (p.den != nullptr && h == 0 && query < N) p.den[hrow + query] = ROWS ? (float)(query + 1) + fscale * x2 : den;
 #pragma unroll
       for (int ct = 0; ct < MT; ct += CT) {
 #pragma unroll
@@ -682,12 +695,18 @@ int launch_main(const WideParams& pp, hipStream_t stream) {
   constexpr int BM = 128 * QT / NKH;
   p.nqb = (p.N + BM - 1) / BM;
   const dim3 grid((unsigned)(p.nqb * p.BH)), block(256);
+  if constexpr (KS == 1 && MT <= 2) {
+    if (p.kmx == nullptr && p.d == 16 && p.den != nullptr) {
+      hipLaunchKernelGGL((wide_kernel<KS, MT, QT, NKH, false, false, true>), grid, block, 0, stream, p);
+      return (int)hipGetLastError();
+    }
+  }
   if (p.kmx != nullptr)
-    hipLaunchKernelGGL((wide_kernel<KS, MT, QT, NKH, false, true>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((wide_kernel<KS, MT, QT, NKH, false, true, false>), grid, block, 0, stream, p);
   else if (p.inv_c == 0.5f && p.inv_c2 == 0.25f)
-    hipLaunchKernelGGL((wide_kernel<KS, MT, QT, NKH, true, false>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((wide_kernel<KS, MT, QT, NKH, true, false, false>), grid, block, 0, stream, p);
   else
-    hipLaunchKernelGGL((wide_kernel<KS, MT, QT, NKH, false, false>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((wide_kernel<KS, MT, QT, NKH, false, false, false>), grid, block, 0, stream, p);
   return (int)hipGetLastError();
 }
 
