@@ -247,3 +247,28 @@ def test_strided_arguments():
     assert call(k=(49152, 64, 380)) == -8 and call(ptr=x.data_ptr() + 2) == -8 and call(k=(0, -64, 384)) == -2
     assert call(N=64) == -5 and call(d=60) == -5 and call(d=72) == -5 and call(k=(49152, 64, 56)) == -5
     assert call(bytes_=n - 1) == -6 and call(N=0) == 0
+
+
+@pytest.mark.parametrize("B,H,N,dv", [(1, 1, 65, 64), (2, 3, 200, 40), (1, 2, 1100, 64), (2, 4, 129, 24), (1, 3, 640, 32)])
+def test_v_aligned_to_8_bytes_only(B, H, N, dv):
+    """d = 16 calls on small grids whose V is not 16-byte aligned stay on the packed kernel, with 128-query
+    work-groups; the whole call and the pre-pass apart."""
+    from kernels import _lib
+    L = _lib.lib()
+    q, k, v = (x.cuda() for x in rand_qkv(B, H, N, 16, dv, seed=N, dtype=torch.bfloat16, scale_qk=0.7))
+    buf = torch.empty(v.numel() + 4, dtype=torch.bfloat16, device="cuda")
+    buf[4:] = v.view(-1)
+    n = int(L.la_based_parallel_workspace_bytes(B, H, N, 16, dv, 1))
+    st = torch.cuda.current_stream().cuda_stream
+    outs = []
+    for apart in (False, True):
+        ws = torch.full((n,), 0x7f, dtype=torch.uint8, device="cuda")
+        out, den = torch.empty(B, H, N, dv, device="cuda"), torch.empty(B, H, N, device="cuda")
+        if apart:
+            assert L.la_based_parallel_pack(k.data_ptr(), buf[4:].data_ptr(), 1, B, H, N, 16, dv, ws.data_ptr(), n, st) == 0
+        f = L.la_based_parallel_fwd_packed if apart else L.la_based_parallel_fwd
+        assert f(q.data_ptr(), k.data_ptr(), buf[4:].data_ptr(), 1, out.data_ptr(), 0, den.data_ptr(), B, H, N, 16, dv,
+                 0.25, 1e-6, 1, ws.data_ptr(), n, st) == 0
+        outs.append(out)
+    off, offd = _check(q, k, v, outs[0], den, 0.25)
+    assert off < 1 and offd < 1 and torch.equal(*outs), (off, offd)
