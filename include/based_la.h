@@ -65,7 +65,9 @@ const char* la_status_string(int status);
  * aligned (may be NULL when that is 0).  It holds V repacked as fp16 V^T blocks and prefix
  * sums over 64-key blocks of the column sums of V, of k and of k k^T for the bf16, d = 16,
  * dv % 8 == 0, dv <= 64 kernel; for the other bf16 shapes, and for that one on small grids, fp16
- * V^T blocks with an exponent and fp32 column sums each; for fp32 inputs on small grids (2 to 255 query blocks of 128
+ * V^T blocks with an exponent and fp32 column sums each (the other shapes also accept 256 bytes per
+ * head, B H 256, and then run a slower kernel that keeps no blocks; both halves of a split call take
+ * the same size); for fp32 inputs on small grids (2 to 255 query blocks of 128
  * tokens in all heads together) the partial numerators and row sums of every (query block,
  * pair of 64-key blocks), which a second kernel adds; its contents on return are unspecified.
  * Limits: 1 <= d <= 128, 1 <= dv <= 128, scale > 0 and finite, eps >= 0 and finite.

@@ -272,3 +272,27 @@ def test_v_aligned_to_8_bytes_only(B, H, N, dv):
         outs.append(out)
     off, offd = _check(q, k, v, outs[0], den, 0.25)
     assert off < 1 and offd < 1 and torch.equal(*outs), (off, offd)
+
+
+@pytest.mark.parametrize("apart", [False, True])
+def test_workspace_of_the_maxima_alone(apart):
+    """256 bytes a head, which these shapes took before the wide kernel, still suffice."""
+    from kernels import _lib
+    L = _lib.lib()
+    B, H, N, d, dv = 1, 3, 300, 64, 64
+    q, k, v = (x.cuda() for x in rand_qkv(B, H, N, d, dv, seed=5, dtype=torch.bfloat16, scale_qk=0.7))
+    assert int(L.la_based_parallel_workspace_bytes(B, H, N, d, dv, 1)) > 256 * H
+    st = torch.cuda.current_stream().cuda_stream
+    ws = torch.full((256 * H + 64,), 0x7f, dtype=torch.uint8, device="cuda")
+    out = torch.empty(B, H, N, dv, device="cuda")
+    f = L.la_based_parallel_fwd_packed if apart else L.la_based_parallel_fwd
+
+    def call(n):
+        if apart:
+            assert L.la_based_parallel_pack(k.data_ptr(), v.data_ptr(), 1, B, H, N, d, dv, ws.data_ptr(), 256 * H, st) == 0
+        return f(q.data_ptr(), k.data_ptr(), v.data_ptr(), 1, out.data_ptr(), 0, None, B, H, N, d, dv, 0.125, 1e-6, 1,
+                 ws.data_ptr(), n, st)
+
+    assert call(256 * H) == 0 and call(256 * H - 1) == -6
+    assert _check(q, k, v, out, torch.zeros(1), 0.125)[0] < 1
+    assert (ws[256 * H:] == 0x7f).all()

@@ -843,6 +843,10 @@ size_t parallel_workspace_bytes(int BH, int N, int d, int dv, bool in_f32) {
   return (size_t)BH * nb64 * (vt_block_bytes(dv) + (size_t)stats_width(DV) * 4);
 }
 
+size_t parallel_workspace_least(int BH, int N, int d, int dv, bool in_f32) {
+  return in_f32 || packed_shape(d, dv) ? parallel_workspace_bytes(BH, N, d, dv, in_f32) : vrange_bytes(BH);
+}
+
 int launch_based_parallel_fp32(const ParallelArgs& a, hipStream_t stream);
 
 bool wide_parallel_call(int BH, int N, int d, int dv) {   // the rule is explained in launch_based_parallel
@@ -912,7 +916,8 @@ int launch_based_parallel(const ParallelArgs& a, hipStream_t stream) {
                       a.workspace_bytes >= parallel_workspace_bytes(a.BH, a.N, a.d, a.dv, false) &&
                       (size_t)p.nb64 * vt_block_bytes(a.dv) < ((size_t)1 << 30) && (size_t)a.N * 32 < ((size_t)1 << 30);
   // The wide kernel takes its shapes unless a tensor is not 16-byte aligned (its copies and stores
-  // are whole 16-byte units); then, and for d > 64, d % 8 or dv % 8, the register-staged kernel.  A
+  // are whole 16-byte units) or the workspace holds the maxima alone (256 bytes a head, the size that
+  // these shapes had before it); then, and for d > 64, d % 8 or dv % 8, the register-staged kernel.  A
   // pre-pass on its own also leaves the maxima of that one, for a later call whose q or out is not
   // aligned.  B2 H16, whole call, register-staged / wide: d64 dv64 N2048 63 / 36 us, N8192
   // 453 / 266 us; d32 dv64 N8192 268 / 218; d64 dv128 N8192 593 / 420; B1 H2 N200 d64 18.0 / 18.0.
@@ -924,7 +929,8 @@ int launch_based_parallel(const ParallelArgs& a, hipStream_t stream) {
   // stream, and it needs no V^T block.
   const bool al16 = ((reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.k) |
                       reinterpret_cast<uintptr_t>(a.v) | reinterpret_cast<uintptr_t>(a.out)) & 15) == 0;
-  if (al16 && wide_parallel_call(a.BH, a.N, a.d, a.dv)) {
+  if (al16 && wide_parallel_call(a.BH, a.N, a.d, a.dv) &&
+      a.workspace_bytes >= parallel_workspace_bytes(a.BH, a.N, a.d, a.dv, false)) {
     if (a.stages == 1)
       hipLaunchKernelGGL(vrange_kernel, dim3((unsigned)VR, (unsigned)a.BH), dim3(256), 0, stream, p.v, p.N, p.dv,
                          const_cast<u32*>(p.vmax));

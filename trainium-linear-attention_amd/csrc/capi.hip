@@ -78,7 +78,7 @@ int parallel_entry(const void* q, const void* k, const void* v, int in_dtype, vo
   if (!finite_f(scale) || !(scale > 0.f) || !finite_f(eps) || eps < 0.f) return LA_ERR_BAD_SCALAR;
   if ((long long)B * H * N == 0) return LA_OK;
   if (den_or_null != nullptr && !al(den_or_null, 4)) return LA_ERR_BAD_ALIGNMENT;
-  const size_t need = la::parallel_workspace_bytes(B * H, N, d, dv, in_dtype == LA_F32);
+  const size_t need = la::parallel_workspace_least(B * H, N, d, dv, in_dtype == LA_F32);
   if (need > 0 && (workspace == nullptr || workspace_bytes < need)) return LA_ERR_WORKSPACE;
   if (need > 0 && !al(workspace, 16)) return LA_ERR_BAD_ALIGNMENT;
   // the packed kernels copy q, k, v^T rows 16 bytes at a time and store out 8 bytes at a time;

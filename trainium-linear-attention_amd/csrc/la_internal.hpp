@@ -101,6 +101,7 @@ struct FeatureMapArgs {
 // and returns 0, a negative LA_ERR_* code, or a positive hipError_t.
 int launch_based_parallel(const ParallelArgs& a, hipStream_t stream);
 size_t parallel_workspace_bytes(int BH, int N, int d, int dv, bool in_f32);
+size_t parallel_workspace_least(int BH, int N, int d, int dv, bool in_f32);   // without the wide kernel's part
 int f32_split_slots(int BH, int N);                         // fp32 key split: slots per head, or 0
 int f32_x6_split_parts(int BH, int N, int d, int dv);       // fp32 three-term key split: parts, or 0
 size_t f32_split_workspace_bytes(int BH, int N, int d, int dv);   // partials of either split (or 0)
