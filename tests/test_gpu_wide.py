@@ -230,6 +230,16 @@ def test_strided_projection_equals_copies(B, N, H, d):
     assert y is not None and torch.equal(y, K.solution_nki(q, k, v).transpose(1, 2).reshape(B, N, H * d))
 
 
+@pytest.mark.parametrize("B,N,H,d", [(8, 4096, 16, 16), (1, 64, 2, 64), (1, 300, 2, 72)])
+def test_refused_projections_allocate_nothing(B, N, H, d):
+    """Shapes that the strided kernel does not take (the packed kernel's grids, one block, other dims)."""
+    from kernels import pytorch_attention as P
+    qkv = torch.zeros(B, N, 3, H, d, dtype=torch.bfloat16, device="cuda")
+    before = torch.cuda.memory_stats()["allocation.all.allocated"]
+    assert P.parallel_from_projection(qkv, 1e-6) is None
+    assert torch.cuda.memory_stats()["allocation.all.allocated"] == before
+
+
 def test_strided_arguments():
     import ctypes
 
@@ -247,6 +257,12 @@ def test_strided_arguments():
     assert call(k=(49152, 64, 380)) == -8 and call(ptr=x.data_ptr() + 2) == -8 and call(k=(0, -64, 384)) == -2
     assert call(N=64) == -5 and call(d=60) == -5 and call(d=72) == -5 and call(k=(49152, 64, 56)) == -5
     assert call(bytes_=n - 1) == -6 and call(N=0) == 0
+
+    def supported(N=128, d=64, k=(49152, 64, 384), out=(8192, 64, 128)):
+        return L.la_based_parallel_strided_supported(1, 2, N, d, 64, S(*k), S(*k), S(*out))
+
+    assert supported() == 0 and supported(k=(49152, 64, 380)) == -8 and supported(k=(0, -64, 384)) == -2
+    assert supported(N=64) == -5 and supported(d=72) == -5 and supported(out=(8192, 64, 56)) == -5 and supported(N=-1) == -2
 
 
 @pytest.mark.parametrize("B,H,N,dv", [(1, 1, 65, 64), (2, 3, 200, 40), (1, 2, 1100, 64), (2, 4, 129, 24), (1, 3, 640, 32)])

@@ -134,6 +134,22 @@ int la_based_parallel_fwd_packed(const void* q, const void* k, const void* v, in
                         workspace, workspace_bytes, hip_stream, 2);
 }
 
+int la_based_parallel_strided_supported(int B, int H, int N, int d, int dv, const long long* k_strides,
+                                        const long long* v_strides, const long long* out_strides) {
+  if (B < 0 || H < 0 || N < 0 || d < 1 || dv < 1) return LA_ERR_BAD_SHAPE;
+  if ((long long)B * H > 0x7fffffffLL || (long long)N * (d > dv ? d : dv) > 0x7fffffffLL) return LA_ERR_BAD_SHAPE;
+  if (k_strides == nullptr || v_strides == nullptr || out_strides == nullptr) return LA_ERR_NULL_POINTER;
+  for (int i = 0; i < 3; ++i) {
+    if (k_strides[i] < 0 || v_strides[i] < 0 || out_strides[i] < 0) return LA_ERR_BAD_SHAPE;
+    if ((k_strides[i] | v_strides[i] | out_strides[i]) & 7) return LA_ERR_BAD_ALIGNMENT;
+  }
+  if (!la::wide_parallel_call(B * H, N, d, dv) || k_strides[2] < d || v_strides[2] < dv || out_strides[2] < dv ||
+      k_strides[2] > (1 << 24) || v_strides[2] > (1 << 24) || out_strides[2] > (1 << 24) ||
+      !la::wide_shape(N, d, dv, k_strides[2], v_strides[2]))
+    return LA_ERR_UNSUPPORTED_DIM;
+  return LA_OK;
+}
+
 int la_based_parallel_fwd_strided(const void* q, const void* k, const void* v, void* out, int B, int H, int N, int d,
                                   int dv, const long long* k_strides, const long long* v_strides,
                                   const long long* out_strides, float scale, float eps, void* workspace,
@@ -144,13 +160,8 @@ int la_based_parallel_fwd_strided(const void* q, const void* k, const void* v, v
   if ((long long)B * H * N == 0) return LA_OK;
   if (k_strides == nullptr || v_strides == nullptr || out_strides == nullptr) return LA_ERR_NULL_POINTER;
   if (!al(q, 16) || !al(k, 16) || !al(v, 16) || !al(out, 16)) return LA_ERR_BAD_ALIGNMENT;
-  for (int i = 0; i < 3; ++i) {
-    if (k_strides[i] < 0 || v_strides[i] < 0 || out_strides[i] < 0) return LA_ERR_BAD_SHAPE;
-    if ((k_strides[i] | v_strides[i] | out_strides[i]) & 7) return LA_ERR_BAD_ALIGNMENT;
-  }
-  if (!la::wide_parallel_call(B * H, N, d, dv) || k_strides[2] < d || v_strides[2] < dv || out_strides[2] < dv ||
-      k_strides[2] > (1 << 24) || v_strides[2] > (1 << 24) || out_strides[2] > (1 << 24) || !la::wide_shape(N, d, dv, k_strides[2], v_strides[2]))
-    return LA_ERR_UNSUPPORTED_DIM;
+  rc = la_based_parallel_strided_supported(B, H, N, d, dv, k_strides, v_strides, out_strides);
+  if (rc != LA_OK) return rc;
   const size_t need = la::parallel_workspace_bytes(B * H, N, d, dv, false);
   if (workspace == nullptr || workspace_bytes < need) return LA_ERR_WORKSPACE;
   if (!al(workspace, 16)) return LA_ERR_BAD_ALIGNMENT;

@@ -18,7 +18,6 @@ LIB_PATH = os.environ.get("BASED_LA_LIB", os.path.join(_PKG, "libbased_la.so"))
 
 LA_F32 = 0
 LA_BF16 = 1
-LA_ERR_UNSUPPORTED_DIM = -5
 
 _lib = None
 _lock = threading.Lock()
@@ -77,6 +76,8 @@ _SIGNATURES = {
     "la_based_parallel_fwd_strided": (_c_int, [_c_void, _c_void, _c_void, _c_void, _c_int, _c_int, _c_int, _c_int,
                                                _c_int, _c_void, _c_void, _c_void, _c_float, _c_float, _c_void,
                                                _c_size, _c_void]),
+    "la_based_parallel_strided_supported": (_c_int, [_c_int, _c_int, _c_int, _c_int, _c_int, _c_void, _c_void,
+                                                     _c_void]),
     "la_taylor_feature_map": (_c_int, [_c_void, _c_int, _c_void, _c_int, ctypes.c_longlong, _c_int, _c_void]),
 }
 

@@ -106,17 +106,17 @@ def parallel_from_projection(qkv, eps):
         return None
     _lib.require_gpu(qkv)
     L = _lib.lib()
-    ws_bytes = int(L.la_based_parallel_workspace_bytes(b, h, t, d, d, _lib.LA_BF16))
-    out = torch.empty(b, t, h * d, dtype=qkv.dtype, device=qkv.device)
-    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=qkv.device)
     row = h * d
     strides = ctypes.c_longlong * 3
     s_in, s_out = strides(3 * t * row, d, 3 * row), strides(t * row, d, row)
+    if L.la_based_parallel_strided_supported(b, h, t, d, d, s_in, s_in, s_out) != 0:
+        return None
+    ws_bytes = int(L.la_based_parallel_workspace_bytes(b, h, t, d, d, _lib.LA_BF16))
+    out = torch.empty(b, t, row, dtype=qkv.dtype, device=qkv.device)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=qkv.device)
     p = qkv.data_ptr()
     rc = L.la_based_parallel_fwd_strided(p, p + 2 * row, p + 4 * row, _lib.ptr(out), b, h, t, d, d, s_in, s_in, s_out,
                                          1.0 / math.sqrt(d), float(eps), _lib.ptr(ws), ws_bytes, _lib.stream_of(qkv))
-    if rc == _lib.LA_ERR_UNSUPPORTED_DIM:
-        return None
     _lib.check(rc, "la_based_parallel_fwd_strided")
     return out
 
