@@ -122,8 +122,9 @@ int la_based_parallel_fwd_packed(const void* q, const void* k, const void* v, in
  * state_out_or_null set): a caller continues such a sequence with la_based_chunked_fwd_num_den
  * and the state's contraction with phi(q) (la_based_state_apply and la_based_state_export of
  * based_la_ext.h for bf16; the Python layer uses la_taylor_feature_map and fp32 GEMMs for fp32).
- * Both are linear in N; aligned bf16 calls of 513 to 8192 tokens (12288 for d > 16) run the
- * parallel form instead, which is faster there, in the same workspace.
+ * Both are linear in N; aligned bf16 calls of more than 512 tokens run the parallel form instead as
+ * long as it is faster, in the same workspace: up to 11500 tokens at d = 16 and 12300 to 16300 above
+ * with few heads, 3700 and 5800 to 14000 with many.
  */
 size_t la_based_chunked_workspace_bytes(int B, int H, int N, int d, int dv, int chunk);
 

@@ -97,6 +97,23 @@ def test_general_long_d64():
         assert e < TOL
 
 
+@pytest.mark.parametrize("d,dv,B,H,N", [(16, 72, 8, 16, 3700), (8, 128, 1, 2, 11500), (32, 64, 1, 8, 12700),
+                                        (64, 64, 4, 16, 12300), (48, 128, 1, 1, 12300)])
+def test_both_sides_of_the_route_limit(d, dv, B, H, N):
+    """The longest call that runs the parallel kernel (wide_chunked_limit) and the one token longer that runs
+    the segment path, with 16-byte rows: fp64 rows over the sequence, and rows of both calls, whose keys are
+    the same, against each other."""
+    K = _kernels()
+    q, k, v = rand_qkv(B, H, N + 1, d, dv, seed=d + dv, dtype=torch.bfloat16)
+    rows = torch.tensor([0, 511, 512, 1000, N // 2, N - 1])
+    ys = [K.based_chunked(*to_dev(q[:, :, :n], k[:, :, :n], v[:, :, :n]), out_dtype=torch.float32).cpu() for n in (N, N + 1)]
+    for b, h in ((0, 0), (B - 1, H - 1)):
+        want = rows_fp64(q, k, v, b, h, rows)
+        for y in ys:
+            assert ref.rel_err(y[b, h, rows], want) < TOL
+    assert 0.0 < ((ys[0] - ys[1][:, :, :N]).norm() / ys[0].norm()).item() < 1e-3
+
+
 def test_general_d64_many_heads():
     """B2 H16 N4096 d64 dv64 (the reference's chunked head dim over 32 heads): more state
     work-groups than CUs, so two share a CU and the sweep alternates their wave priorities.

@@ -898,19 +898,39 @@ size_t general_chunked_bytes(int BH, int N, int d, int dv, bool in_f32) {
   return glayout(BH, N, d, dv).total;
 }
 
+// Sequences of several segments up to this many tokens run the parallel kernel on the whole sequence: its
+// work grows with N^2, this path's with N, but its rate per operation is about five times this path's
+// (us, this path / parallel, B2 H16: d64 dv64 N1024 101 / 26, N8192 425 / 286, N12288 646 / 592, N14336
+// 761 / 795; d64 dv128 N16384 2137 / 1680; d32 dv64 N8192 293 / 228, N12288 440 / 473; d16 dv128 N4096
+// 188 / 114, N8192 323 / 363).  Where both take the same time, measured over d 8 to 64, dv 32 to 128 and 1 to
+// 128 heads: per feature tiles and value tiles, in hundreds of tokens, at up to 8, at 16, 32, 64 and from
+// 128 heads, in between by the logarithm of the heads.  Few heads: both latency-bound; many: this path gains
+// work-groups, which the parallel one has at any count.  (Below 8 heads it is the smallest of 1 to 8: at one
+// head of d32 dv64 the parallel form would still win by 20 % from 12700 to 16000 tokens.)
+int wide_chunked_limit(int BH, int d, int dv) {
+  static const short kLimit[4][3][5] = {   // dv <= 32, <= 64, more
+      {{122, 80, 67, 68, 48}, {115, 84, 66, 52, 37}, {115, 84, 66, 52, 37}},         // d <= 16
+      {{127, 105, 110, 75, 58}, {127, 105, 110, 75, 58}, {136, 142, 127, 84, 74}},   // d <= 32
+      {{133, 133, 135, 90, 83}, {133, 123, 108, 84, 75}, {123, 164, 135, 114, 95}},   // d <= 48
+      {{163, 185, 148, 133, 107}, {155, 165, 135, 123, 98}, {152, 204, 200, 160, 140}},   // d <= 64
+  };
+  const short* L = kLimit[dp_of(d) / 16 - 1][dv <= 32 ? 0 : dv <= 64 ? 1 : 2];
+  if (BH <= 8) return 100 * L[0];
+  if (BH >= 128) return 100 * L[4];
+  const double x = __builtin_log2((double)BH) - 3.0;
+  const int i = (int)x;
+  return (int)(100.0 * (L[i] + (x - i) * (L[i + 1] - L[i])));
+}
+
 int launch_general_chunked(const ChunkedArgs& a, hipStream_t stream) {
   if (!general_chunked_shape(a.d, a.dv, a.in_f32)) return LA_ERR_UNSUPPORTED_DIM;
   if (a.in_f32) return launch_general_chunked_f32(a, stream);
   const int DP = dp_of(a.d), DVT = dvt_of(a.dv);
-  // Sequences of several segments up to kWideMax tokens run the parallel kernel on the whole sequence
-  // (its work grows with N^2, this path's with N, but at about five times the rate per operation): us,
-  // this path / parallel: B2 H16 d64 dv64 N1024 102 / 23, N8192 428 / 264, N16384 868 / 953; d32 dv64
-  // N8192 297 / 216; B1 H4 N16384 141 / 139; B2 H16 d16 dv128 N4096 190 / 106, N8192 339 / 338; d64 dv128
-  // N8192 1035 / 422.  One segment keeps this path: no workspace, one launch.
+  // One segment keeps this path: no workspace, one launch.
   {
-    const int kWideMax = DP == 16 ? 8192 : 12288;
     const size_t need = general_chunked_bytes(a.BH, a.N, a.d, a.dv, false);
-    if (a.N > GL && a.N <= kWideMax && wide_shape(a.N, a.d, a.dv) && wide_workspace_bytes(a.BH, a.N, a.dv) <= need &&
+    if (a.N > GL && a.N <= wide_chunked_limit(a.BH, a.d, a.dv) && wide_shape(a.N, a.d, a.dv) &&
+        wide_workspace_bytes(a.BH, a.N, a.dv) <= need &&
         ((reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.k) | reinterpret_cast<uintptr_t>(a.v) |
           reinterpret_cast<uintptr_t>(a.out)) & 15) == 0) {
       if (a.workspace == nullptr || a.workspace_bytes < need) return LA_ERR_WORKSPACE;

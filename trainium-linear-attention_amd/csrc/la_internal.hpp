@@ -138,6 +138,7 @@ int launch_based_chunked(const ChunkedArgs& a, hipStream_t stream);
 // dv <= 128; bf16 in chunked_general.hip, fp32 in chunked_general_f32.hip).
 bool general_chunked_shape(int d, int dv, bool in_f32);
 size_t general_chunked_bytes(int BH, int N, int d, int dv, bool in_f32);   // workspace, (size_t)-1 if unsupported
+int wide_chunked_limit(int BH, int d, int dv);   // most tokens of a bf16 call that the wide kernel takes
 int launch_general_chunked(const ChunkedArgs& a, hipStream_t stream);
 size_t general_chunked_f32_bytes(int BH, int N, int d, int dv);
 int launch_general_chunked_f32(const ChunkedArgs& a, hipStream_t stream);

@@ -17,8 +17,9 @@ Two chunked paths: the recurrence kernel for bf16 inputs with d = 16 and dv <= 6
 configuration), and for other head dims and fp32 inputs (d <= 64, dv <= 128) a segment-state
 path (state prefixes of 512-token segments in the feature basis, then every query's contraction
 with its segment's prefix plus the quadratic form inside the segment; fp32 throughout for fp32
-inputs).  Both are linear in the sequence length; bf16 calls of the latter with 16-byte rows and 513
-to 8192 tokens (12288 for d > 16) run the parallel form inside the library, which is faster there.
+inputs).  Both are linear in the sequence length; bf16 calls of the latter with 16-byte rows and more
+than 512 tokens run the parallel form inside the library as long as that is faster (up to 3700 to
+20000 tokens by head dims and number of heads), with errors no larger.
 Shapes outside both are computed by the fused parallel kernel, which evaluates the same
 function (numerator or normalised) on the GPU.  ``chunk_size`` is the reference's argument
 (any value >= 1); the kernel's recurrence runs 128-token chunks (``la_based_chunked_chunk_used``

@@ -151,7 +151,7 @@ CHUNKED_MIN_T = 256
 # dims and for fp32 inputs (d <= 64, dv <= 128).  Measured on MI355X, B2 H16 (whole calls, ms,
 # chunked / fused): bf16 d64 dv64 N = 16384 0.864 / 0.953, d32 dv64 B1 H4 0.141 / 0.139; fp32 d16 dv64
 # N = 8192 0.774 / 0.864.  The fused kernel's work grows with N^2, the chunked paths' with N (whose
-# bf16 calls run the fused kernel themselves up to 8192 or 12288 tokens).
+# bf16 calls run the fused kernel's form themselves as long as it is faster).
 GENERAL_CHUNKED_MIN_T = 16384
 
 
