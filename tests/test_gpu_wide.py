@@ -43,6 +43,26 @@ def test_edges(B, H, N, d, dv, scale):
     assert torch.equal(K.based_parallel(q, k, v, scale=scale), y.bfloat16())
 
 
+@pytest.mark.parametrize("H,N,dv,wide", [(2, 43520, 32, True), (2, 43777, 32, False), (3, 43520, 64, True), (32, 4090, 64, False),
+                                         (8, 16128, 32, True), (8, 16129, 32, False)])
+def test_d16_grids_on_both_sides_of_the_route_limits(H, N, dv, wide):
+    """Fewer 256-query work-groups than two per CU (4/3 with fewer than 8 heads and dv <= 32) run the wide
+    kernel, others the packed one; fp64 rows of the last head on either side."""
+    import ctypes
+
+    import kernels as K
+    from kernels import _lib
+    from tests.helpers import rows_fp64
+    S = ctypes.c_longlong * 3
+    s = [S(0, N * w, w) for w in (16, dv)]
+    assert _lib.lib().la_based_parallel_strided_supported(1, H, N, 16, dv, s[0], s[1], s[1]) == (0 if wide else -5)
+    q, k, v = rand_qkv(1, H, N, 16, dv, seed=N, dtype=torch.bfloat16, scale_qk=0.25)
+    y = K.based_parallel(q.cuda(), k.cuda(), v.cuda(), out_dtype=torch.float32).cpu()
+    rows = torch.tensor([0, 63, 255, 256, N // 2, N - 1])
+    want = rows_fp64(q, k, v, 0, H - 1, rows)
+    assert ((y[0, H - 1, rows].double() - want).norm() / want.norm()).item() < 1e-4
+
+
 @pytest.mark.parametrize("dv", [32, 64])
 @pytest.mark.parametrize("scale", [None, 0.3])
 def test_d16_denominators_from_fp32_sums(dv, scale):

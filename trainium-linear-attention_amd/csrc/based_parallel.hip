@@ -850,7 +850,8 @@ size_t parallel_workspace_least(int BH, int N, int d, int dv, bool in_f32) {
 int launch_based_parallel_fp32(const ParallelArgs& a, hipStream_t stream);
 
 bool wide_parallel_call(int BH, int N, int d, int dv) {   // the rule is explained in launch_based_parallel
-  const bool few = (long long)((N + 255) / 256) * BH < 2LL * device_cu_count();
+  const long long wg256 = (long long)((N + 255) / 256) * BH, cus = device_cu_count();
+  const bool few = dv <= 32 && BH < 8 ? 3 * wg256 < 4 * cus : wg256 < 2 * cus;
   return wide_shape(N, d, dv) && (packed_shape(d, dv) ? few : N > BN) &&
          vrange_bytes(BH) + wide_workspace_bytes(BH, N, dv) <= parallel_workspace_bytes(BH, N, d, dv, false);
 }
@@ -922,10 +923,12 @@ int launch_based_parallel(const ParallelArgs& a, hipStream_t stream) {
   // aligned.  B2 H16, whole call, register-staged / wide: d64 dv64 N2048 63 / 36 us, N8192
   // 453 / 266 us; d32 dv64 N8192 268 / 218; d64 dv128 N8192 593 / 420; B1 H2 N200 d64 18.0 / 18.0.
   // Of the packed kernel's shapes it takes those whose 256-query work-groups do not fill the CUs
-  // twice: its pre-pass needs no scan and no k k^T, which counts more there than the row sums that it
-  // adds per key (packed / wide, us: B2 H16 d16 dv64 N256 19.5 / 15.7, N2048 33.5 / 30.2, N3000
-  // 50.8 / 48.5, N4096, which fills them, 67.1 / 71.7, N8192 183 / 199; dv32 N2048 27.5 / 22.7, N4096
-  // 53.1 / 56.6).  A single 64-key block of another shape stays register-staged: there is nothing to
+  // twice: its pre-pass needs no scan and no k k^T, and its 128-query work-groups share their keys, which
+  // counts more there than the row sums that it adds per key (packed / wide, us, dv64: 32 heads N2048 32.4 /
+  // 28.6, N3840, 480 work-groups, 64.6 / 60.7, N3968, 512 of them, 63.7 / 70.4; 8 heads N8192 75.0 / 68.2,
+  // N15872 202 / 192; 1 head N32768 222 / 203, N102400, 400, 951 / 968).  dv <= 32 with fewer than 8 heads
+  // ends at 4/3 (1 head N65536, 256, 383 / 360, N102400 708 / 758; 4 heads N20480, 320, 139.1 / 138.8,
+  // N25600, 400, 192 / 201; 8 heads N15872, 496, 144 / 136).  A single 64-key block of another shape stays register-staged: there is nothing to
   // stream, and it needs no V^T block.
   const bool al16 = ((reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.k) |
                       reinterpret_cast<uintptr_t>(a.v) | reinterpret_cast<uintptr_t>(a.out)) & 15) == 0;
