@@ -206,7 +206,7 @@ def test_decode_argument_errors():
 def test_decode_workspace_sizes_and_errors():
     lib = _lib()
     ws = lib.la_based_decode_workspace_bytes
-    # A head's state of F (dv + 1) <= 10240 floats is held in LDS by one work-group: no
+    # A head's state of F (dv + 1) <= 10240 floats is one work-group's: no
     # workspace (d = 16: F = 153, so dv <= 65).  Larger states: B*H heads split into R row
     # groups of the F rows until about 1024 work-groups launch, at least 8 rows each: R = 20 for
     # 2 heads, 8 for 128, 2 for 640, 1 for 1024 (no workspace); one fp32 partial sum per group
@@ -292,7 +292,7 @@ def test_parallel_workspace_sizes():
     assert ws(2, 16, 8192, 16, 64, 1) == 32 * 128 * (9216 + 4 * (64 + 160))
     assert ws(1, 1, 65, 16, 32, 1) == 2 * (5120 + 4 * (32 + 160))
     assert ws(1, 1, 64, 16, 64, 0) == 0        # fp32 inputs: no workspace
-    # other bf16 shapes (register-staged kernel): 64 partial maxima of |v| per head
+    # other bf16 shapes of one key block (register-staged kernel): 64 partial maxima of |v| per head
     assert ws(1, 1, 64, 32, 64, 1) == 256       # d != 16
     assert ws(1, 1, 64, 16, 60, 1) == 256       # dv % 8 != 0
     assert ws(2, 3, 64, 16, 72, 1) == 6 * 256   # dv > 64

@@ -1,10 +1,12 @@
-"""GPU parity of the segment-state chunked path (head dims other than 16: d <= 64, dv <= 128,
+"""GPU parity of chunked calls at head dims other than the d = 16 recurrence's (d <= 64, dv <= 128,
 bf16) against the fp64 oracle.
 
-The path cuts the sequence into 512-token segments: a state kernel writes every segment's
-exclusive state prefix in the feature basis (fp16 with per-tile exponents), an output kernel
-contracts every query's features with its segment's prefix and adds the quadratic form over
-the segment's own keys.  Lengths around the segment and tile boundaries (255/256/257,
+The segment-state path cuts the sequence into 512-token segments: a state kernel writes every
+segment's exclusive state prefix in the feature basis (fp16 with per-tile exponents), an output
+kernel contracts every query's features with its segment's prefix and adds the quadratic form over
+the segment's own keys.  It runs one segment, rows that are not 16-byte aligned (d or dv not in eights
+here) and long sequences; aligned calls between those run the wide kernel (test_gpu_routes.py has more
+of the former).  Lengths around the segment and tile boundaries (255/256/257,
 511/512/513, 1023/1024/1025) check the hand-over between the two parts.  Bar as for the other
 bf16 paths: max|y - y_ref| / rms(y_ref) < 2e-2, fp32 output against fp64 on the same
 bf16-rounded inputs.
@@ -61,8 +63,8 @@ def test_general_wrappers_and_batch():
 
 @pytest.mark.parametrize("case", ["v_x1e4", "v_x1e-5", "qk_x8", "v_steps"])
 def test_general_range(case):
-    """Feature, state and value ranges: V scaled by 1e4 and 1e-5, large scores (q, k x 8: |s|
-    up to ~150) and V steps of 1e3 between segments (the state prefixes' exponents change)."""
+    """V scaled by 1e4 and 1e-5, large scores (q, k x 8: |s| up to ~150) and V steps of 1e3 between
+    512-token stretches, on the wide kernel."""
     K = _kernels()
     N, d, dv = 1800, 64, 64
     q, k, v = rand_qkv(1, 2, N, d, dv, seed=5, dtype=torch.float32)
@@ -84,7 +86,7 @@ def test_general_range(case):
 
 
 def test_general_long_d64():
-    """B1 H2 N 16384 d64: fp64 rows spread over the sequence (last rows of late segments)."""
+    """B1 H2 N 16384 d64, the segment path: fp64 rows spread over the sequence (last rows of late segments)."""
     K = _kernels()
     N = 16384
     q, k, v = rand_qkv(1, 2, N, 64, 64, seed=21, dtype=torch.bfloat16)
@@ -115,8 +117,7 @@ def test_both_sides_of_the_route_limit(d, dv, B, H, N):
 
 
 def test_general_d64_many_heads():
-    """B2 H16 N4096 d64 dv64 (the reference's chunked head dim over 32 heads): more state
-    work-groups than CUs, so two share a CU and the sweep alternates their wave priorities.
+    """B2 H16 N4096 d64 dv64 (the reference's chunked head dim over 32 heads), on the wide kernel.
     The first 1024 rows of every head against the dense fp64 oracle and rows across the later
     segments of every head against fp64 rows."""
     K = _kernels()

@@ -204,10 +204,11 @@ def test_single_hip_runtime_and_native_library():
     assert len(rts) == 1
 
 
-@pytest.mark.parametrize("B,H,N,dv", [(1, 2, 777, 64), (2, 8, 1024, 32)])
+@pytest.mark.parametrize("B,H,N,dv", [(1, 2, 777, 64), (2, 8, 1024, 32), (4, 64, 300, 64)])
 def test_pack_then_packed_kernel_equals_fused_call(B, H, N, dv):
     """la_based_parallel_pack + la_based_parallel_fwd_packed is la_based_parallel_fwd, bit for
-    bit, including a second k and v packed into the same workspace."""
+    bit, including a second k and v packed into the same workspace.  These grids are the wide kernel's;
+    the last one the packed kernel's."""
     from kernels import _lib
     L = _lib.lib()
     d = 16
@@ -262,8 +263,9 @@ def test_solution_dispatch_by_length(N, d, dv, dtype):
                                       (1, 3, 129, 32)])
 def test_packed_work_group_sizes(B, H, N, dv):
     """The packed kernel runs 256-query work-groups when they fill every CU's slots (two per CU
-    at dv = 64, three at dv = 32: the first two shapes at 256 CUs) and 128-query ones below that;
-    ragged N in both."""
+    at dv = 64, three at dv = 32: the first two shapes at 256 CUs) and 128-query ones below that (the
+    third; at dv = 64 only where V is 8-byte aligned); the last two shapes are the wide kernel's.
+    Ragged N in all."""
     K = _kernels()
     q, k, v = rand_qkv(B, H, N, 16, dv, seed=N + dv + H, dtype=torch.bfloat16, scale_qk=0.5)
     y, den = K.based_parallel(*to_dev(q, k, v), out_dtype=torch.float32, return_den=True)

@@ -43,8 +43,8 @@ def _run(path, q, k, v, normalize=True):
     return K.based_chunked(qd, kd, vd, normalize=normalize, out_dtype=torch.float32)
 
 
-# (d, dv): the packed parallel kernel (d 16, dv % 8 == 0, dv <= 64), the register-staged one
-# (d 32; dv 96) and the chunked kernel's shapes
+# (d, dv): the wide parallel kernel at these grids, and the chunked kernel's shapes (test_gpu_routes.py has
+# the packed kernel's grids, and the segment-state path beyond the wide kernel's lengths)
 PAR_SHAPES = [(16, 64), (16, 40), (32, 64), (16, 96)]
 
 
@@ -211,10 +211,8 @@ def test_sliding_range(vscale, qk, W):
 
 
 def test_general_zero_key_dims_large_v():
-    """Segment-state path (d = 64): keys zero in dims 16..63 over the first 512-token segment, so
-    the work-groups of feature groups built from those dims see an all-zero state prefix (stored
-    as zeros, whatever scale the slot's other part sets), with V scaled by 1e10: finite outputs
-    at the bf16 bar against fp64."""
+    """Chunked call at d = 64 (the wide kernel at this length): keys zero in dims 16..63 over the first
+    512 tokens, with V scaled by 1e10: finite outputs at the bf16 bar against fp64."""
     q, k, v = _scaled(1, 2, 1500, 64, 64, seed=18, vscale=1e10, qk=0.5)
     k = k.clone()
     k[:, :, :512, 16:] = 0
@@ -231,8 +229,8 @@ def test_unbalanced_q_k(path, d, kscale):
     """q divided and k multiplied by the same factor (the scores are unchanged): the parallel
     kernels at 1e4; the d = 16 chunk recurrence, whose features are fp16 products of
     sqrt(scale) q and sqrt(scale) k, at 100 (max |k| about 450 here, inside its limit of 1024);
-    the bf16 segment-state path, whose q-side features are fp16 in units of max |[scale q, 1]|,
-    at 30 (the stated range of both)."""
+    the bf16 chunked path at d = 64 at 30, the stated range of the segment-state kernels (here the wide
+    kernel)."""
     q, k, v = rand_qkv(1, 2, 700, d, 64, seed=3, dtype=torch.float32)
     q, k, v = (q / kscale).bfloat16(), (k * kscale).bfloat16(), v.bfloat16()
     want, _, _ = ref.based_dense(q, k, v)
@@ -261,8 +259,7 @@ def test_v_extreme_scales(vscale, path, d, B, H, N):
 
 
 def test_general_v_tiny_prefix():
-    """Segment-state path (d = 64): the first 600 tokens' V 1e-20 times the rest, so the first
-    segment's prefix is 1e-20 below the later ones (the head exponent comes from the largest)."""
+    """Chunked call at d = 64 (the wide kernel at this length): the first 600 tokens' V 1e-20 times the rest."""
     q, k, v = _scaled(1, 2, 1500, 64, 64, seed=20)
     t = torch.ones(1, 2, 1500, 1)
     t[:, :, :600] = 1e-20

@@ -1,4 +1,4 @@
-"""The wide parallel kernel (bf16, d <= 64 and dv <= 128 in eights, other than d = 16 with dv <= 64) at
+"""The wide parallel kernel (bf16, d <= 64 and dv <= 128 in eights; at d = 16 with dv <= 64 on small grids) at
 the edges of its tiles, against 64 bits.  Bound: p = 1 + r with r rounded to fp16 (2^-11 relative) and
 everything else in fp32, in the numerator and in the row sum, so |y - y64| <= (2^-11 + 2^-13)
 (sum |r| |v| + |y| sum |r|) / den + N 2^-24 sum p |v| / den."""
@@ -240,7 +240,7 @@ def test_chunked_calls_small_value_columns():
 @pytest.mark.parametrize("B,N,H,d", [(1, 65, 2, 64), (3, 200, 4, 24), (2, 257, 16, 16), (2, 2048, 32, 64), (1, 130, 3, 8)])
 def test_strided_projection_equals_copies(B, N, H, d):
     """q, k, v read in place in a (b, t, 3, h, d) projection and the heads written merged: bit for bit
-    what the same kernel gives on contiguous copies; the rows around the output stay untouched."""
+    what the same kernel gives on contiguous copies."""
     import kernels as K
     from kernels import pytorch_attention as P
     g = torch.Generator(device="cuda").manual_seed(N)
@@ -248,6 +248,43 @@ def test_strided_projection_equals_copies(B, N, H, d):
     y = P.parallel_from_projection(qkv, 1e-6)
     q, k, v = qkv.permute(2, 0, 3, 1, 4).contiguous().unbind(0)
     assert y is not None and torch.equal(y, K.solution_nki(q, k, v).transpose(1, 2).reshape(B, N, H * d))
+
+
+@pytest.mark.parametrize("B,H,N,d,dv", [(2, 3, 65, 64, 40), (3, 2, 200, 24, 72), (1, 5, 130, 16, 48), (2, 128, 257, 8, 24)])
+def test_strides_wider_than_the_data(B, H, N, d, dv):
+    """q and k, v and the output each with batch, head and token strides of their own that leave gaps, the
+    output inside a buffer of sentinels: values of the contiguous call, every element between, before and
+    after them untouched."""
+    import ctypes
+
+    import kernels as K
+    from kernels import _lib
+    L = _lib.lib()
+    q, k, v = (x.cuda() for x in rand_qkv(B, H, N, d, dv, seed=N + d, dtype=torch.bfloat16, scale_qk=0.7))
+    S = ctypes.c_longlong * 3
+
+    def strides(w, head_gap, row_gap, batch_gap):
+        head = w + head_gap
+        row = H * head + row_gap
+        return (N * row + batch_gap, head, row)
+
+    def place(x, st, lead, fill=float("nan")):
+        buf = torch.full((lead + B * st[0] + 64,), fill, dtype=torch.bfloat16, device="cuda")
+        view = buf[lead:].as_strided((B, H, N, x.shape[-1]), (*st, 1))
+        view.copy_(x)
+        return buf, view
+
+    sk, sv, so = strides(d, 8, 16, 24), strides(dv, 0, 8, 64), strides(dv, 16, 40, 8)
+    (_, qv), (_, kv), (_, vv) = place(q, sk, 64), place(k, sk, 8), place(v, sv, 16)
+    out, ov = place(torch.full_like(v, -7.0), so, 64, -7.0)
+    n = int(L.la_based_parallel_workspace_bytes(B, H, N, d, dv, 1))
+    ws = torch.full((n + 64,), 0x7f, dtype=torch.uint8, device="cuda")
+    assert L.la_based_parallel_fwd_strided(qv.data_ptr(), kv.data_ptr(), vv.data_ptr(), ov.data_ptr(), B, H, N, d, dv,
+                                           S(*sk), S(*sv), S(*so), 1.0 / math.sqrt(d), 1e-6, ws.data_ptr(), n,
+                                           torch.cuda.current_stream().cuda_stream) == 0
+    assert torch.equal(ov, K.based_parallel(q, k, v))
+    ov.fill_(-7.0)
+    assert (out == -7.0).all() and (ws[n:] == 0x7f).all()
 
 
 @pytest.mark.parametrize("B,N,H,d", [(8, 4096, 16, 16), (1, 64, 2, 64), (1, 300, 2, 72)])

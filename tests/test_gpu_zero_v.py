@@ -44,9 +44,10 @@ def _run(path, q, k, v):
     raise ValueError(path)
 
 
-# (path, d, dv, dtype, B, H, N): the packed parallel kernel, the register-staged one, the fp32
-# three-term kernel, the d = 16 chunk recurrence (one-chunk segments at B1 H2, four-chunk
-# segments at B2 H16), the segment-state path (bf16 d64, fp32 d16)
+# (path, d, dv, dtype, B, H, N): the wide parallel kernel (d 16 and 32), the fp32 three-term kernel, the
+# d = 16 chunk recurrence (one-chunk segments at B1 H2, four-chunk segments at B2 H16), the chunked call at
+# d 64 (the wide kernel) and the fp32 segment-state path (test_gpu_routes.py: the packed kernel, the bf16
+# segment-state path)
 CASES = [
     ("parallel", 16, 64, torch.bfloat16, 1, 2, 1100),
     ("parallel", 32, 64, torch.bfloat16, 1, 2, 1100),
