@@ -365,9 +365,10 @@ __device__ __forceinline__ void gram_update(const uint16_t* KT, f32x16& G, int g
 // The bound is the k and v read (waits on it are 57 % of the wave cycles; MFMAs keep the matrix cores
 // 23 % busy, LDS its port 38 %): 168 MB in 47 us = 3.5 TB/s at B1 H16 N65536.  Splitting the features
 // instead (five waves on one block each, shared tables, a barrier per chunk) read every V^T operand
-// five times and took 58 us; whole calls: B1 H4 N32768 63.4 -> 57.1 us, B2 H16 N2048 34.2 -> 32.8,
-// B2 H16 N8192 1.00 to 1.02 times as fast, B1 H16 N65536 155 -> 152 (no better while two values spilled: scratch makes a
-// launch slower by about a microsecond; hence the packed addresses, and the lane id read anew below).
+// five times and took 58 us; whole calls, where this pass shares the time with the output pass: B1 H4
+// N32768 63.4 -> 57.1 us, B2 H16 N2048 34.2 -> 32.8, inside the spread at B2 H16 N8192 (53.7 -> 53.3) and
+// B1 H16 N65536 (158.9 -> 157.6).  Scratch makes a launch slower by about a microsecond; hence the packed
+// addresses, and the lane id read anew below.
 // A wave's tables of 32 tokens: rows of 80 bytes, eight of which start in eight different groups of
 // four banks (the 16-byte operand reads); the extra halves per octet of rows spread the octets that one
 // staging store writes at once.  Row and token offsets are immediates of one address per table.
@@ -938,10 +939,9 @@ __device__ __forceinline__ void output_wave(LT& L, const ChunkParams& p, int bh,
   constexpr bool GRAM = W == kGramWave;
   const int tid = threadIdx.x;
   int lane = tid & 63;
-  // In the layer kernel the lane's range is hidden from the compiler: with it known, address
-  // arithmetic is folded into forms that cost registers (254 -> 250) and time (B2 H16 N8192
-  // 84.6 -> 83.1 us, N3001 45.9 -> 45.8; the chunked output kernel is about 1 % slower so).
-  if constexpr (LAYER) asm("" : "+v"(lane));
+  // The lane's range hidden from this compiler: B2 H16 N3001 d_sw 64 45.6 -> 45.3 us;
+  // the layer at d_sw 32 and the chunked output kernel are 1 to 2 % slower so.
+  if constexpr (DSW == 64) asm("" : "+v"(lane));
   const int r = lane & 31, h = lane >> 5;
   const int N = p.N, dv = p.dv;
   const size_t hrow = (size_t)bh * N;
