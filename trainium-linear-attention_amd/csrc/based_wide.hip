@@ -70,12 +70,11 @@ struct WideParams {
 
 // V^T rows: 64 keys = eight 16-byte units; unit 2 m + h of a row holds keys 16 m + 4 h + {0..3, 8..11}
 // (the order of a score accumulator's registers, so a unit is a whole A operand of the P.V MFMA),
-// stored at unit ^ wswz(row).  K rows of 2 KS 16-byte chunks: chunk c at c ^ kwz(key).  Both make
+// stored at unit ^ swz64(row).  K rows of 2 KS 16-byte chunks: chunk c at c ^ kwz(key).  Both make
 // the 16 lanes of a ds_read_b128 pass touch all 64 banks once.
-__device__ __forceinline__ int wswz(int r) { return ((r >> 2) & 7) ^ ((r & 2) << 1); }
 template <int KS>
 __device__ __forceinline__ int kwz(int key) {
-  return KS == 1 ? ((key >> 2) ^ (key >> 3)) & 1 : KS == 2 ? (key >> 2) & 3 : wswz(key);
+  return KS == 1 ? ((key >> 2) ^ (key >> 3)) & 1 : KS == 2 ? (key >> 2) & 3 : swz64(key);
 }
 
 constexpr u32 kCoarse = 0x80000000u;
@@ -152,7 +151,7 @@ __global__ __launch_bounds__(256) void wide_pack_kernel(const WideParams p) {
       const float g0 = __builtin_ldexpf(f0, -eb), g1 = __builtin_ldexpf(f1, -eb);
       const u32 y = pack_f16x2(g0, g1);
       if (ANY && (f16_lo_to_f32(y) != g0 || f16_hi_to_f32(y) != g1)) lost[row] = 1u;
-      *reinterpret_cast<u32*>(&img[row * BN + ((unit ^ wswz(row)) << 3) + e]) = y;
+      *reinterpret_cast<u32*>(&img[row * BN + ((unit ^ swz64(row)) << 3) + e]) = y;
     }
   }
   __syncthreads();
@@ -380,7 +379,7 @@ __global__ __launch_bounds__(256, KS == 1 && MT == 1 && !ROWS ? 3 : 2) void wide
   };
   auto vfrag = [&](const uint16_t* st, int ks, int m, int mt) {
     const int row = 32 * mt + n;
-    return *reinterpret_cast<const u32x4*>(st + UK * 512 + row * BN + (((4 * ks + 2 * m + h) ^ wswz(row)) << 3));
+    return *reinterpret_cast<const u32x4*>(st + UK * 512 + row * BN + (((4 * ks + 2 * m + h) ^ swz64(row)) << 3));
   };
   // pieces of a full 32-key unit: scores b = K Q^T + 1/c; u = b b - 1/c^2 in fp16 and its row sums;
   // acc += V^T u^T
@@ -730,21 +729,18 @@ int launch_wide(const WideParams& p, int stages, hipStream_t stream) {
   }
 }
 
-int mt_of(int dv) { return dv <= 32 ? 1 : dv <= 64 ? 2 : 4; }
-size_t up256(size_t x) { return (x + 255) & ~(size_t)255; }
-
 }  // namespace
 
 bool wide_shape(int N, int d, int dv) { return wide_shape(N, d, dv, d, dv); }
 
 bool wide_shape(int N, int d, int dv, long long krow, long long vrow) {   // rows of krow, vrow elements
   const size_t nb = ((size_t)N + BN - 1) / BN;
-  return d % 8 == 0 && d <= 64 && dv % 8 == 0 && dv <= 128 && nb * (size_t)(32 * mt_of(dv) * BN * 2) < ((size_t)1 << 30) && (unsigned long long)N * krow * 2 < ((size_t)1 << 30) &&
+  return d % 8 == 0 && d <= 64 && dv % 8 == 0 && dv <= 128 && nb * (size_t)(32 * dv_tiles(dv) * BN * 2) < ((size_t)1 << 30) && (unsigned long long)N * krow * 2 < ((size_t)1 << 30) &&
          (unsigned long long)N * vrow * 2 < ((size_t)1 << 30);
 }
 
 size_t wide_workspace_bytes(int BH, int N, int dv) {
-  const size_t nb = ((size_t)N + BN - 1) / BN, DV = 32 * mt_of(dv);
+  const size_t nb = ((size_t)N + BN - 1) / BN, DV = 32 * dv_tiles(dv);
   return up256(BH * nb * DV * BN * 2) + up256(BH * nb * DV * 4) + 2 * up256(BH * nb * 4);
 }
 
@@ -768,7 +764,7 @@ int launch_wide_parallel(const ParallelArgs& a, void* workspace, bool any_range,
     p.os[i] = st != nullptr ? st->out[i] : n[i] * a.dv;
   }
   p.nb = (a.N + BN - 1) / BN;
-  const size_t DV = 32 * mt_of(a.dv), blocks = (size_t)a.BH * p.nb;
+  const size_t DV = 32 * dv_tiles(a.dv), blocks = (size_t)a.BH * p.nb;
   char* ws = static_cast<char*>(workspace);
   p.vt = reinterpret_cast<uint16_t*>(ws);
   p.sums = reinterpret_cast<float*>(ws + up256(blocks * DV * BN * 2));
@@ -784,7 +780,7 @@ int launch_wide_parallel(const ParallelArgs& a, void* workspace, bool any_range,
   p.normalize = a.normalize ? 1 : 0;
   p.out_f32 = a.out_f32 ? 1 : 0;
   p.xcd_cus = device_cu_count() / 8;
-  const int ks = a.d <= 16 ? 1 : a.d <= 32 ? 2 : 4, mt = mt_of(a.dv);
+  const int ks = a.d <= 16 ? 1 : a.d <= 32 ? 2 : 4, mt = dv_tiles(a.dv);
 #define LA_WIDE(K, M) \
   if (ks == K && mt == M) return launch_wide<K, M>(p, a.stages, stream)
   LA_WIDE(1, 1);

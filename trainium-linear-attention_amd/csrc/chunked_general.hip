@@ -776,7 +776,6 @@ __global__ __launch_bounds__(256, DVT == 4 ? 1 : 2) void gout_kernel(const GPara
 }
 
 int dp_of(int d) { return 16 * ((d + 15) / 16); }
-int dvt_of(int dv) { return dv <= 32 ? 1 : dv <= 64 ? 2 : 4; }
 
 // Parts of the state sweep: when the (head, work-group) pairs fill less than half of 256 CUs,
 // enough parts for two work-groups per CU (the totals pass sweeps all but the last part a second
@@ -825,7 +824,7 @@ GLayout glayout_dp(int BH, int nseg, int DVT) {
 }
 
 GLayout glayout(int BH, int N, int d, int dv) {
-  const int nseg = (N + GL - 1) / GL, DP = dp_of(d), DVT = dvt_of(dv);
+  const int nseg = (N + GL - 1) / GL, DP = dp_of(d), DVT = dv_tiles(dv);
   switch (DP) {
     case 16: return glayout_dp<16>(BH, nseg, DVT);
     case 32: return glayout_dp<32>(BH, nseg, DVT);
@@ -925,7 +924,7 @@ int wide_chunked_limit(int BH, int d, int dv) {
 int launch_general_chunked(const ChunkedArgs& a, hipStream_t stream) {
   if (!general_chunked_shape(a.d, a.dv, a.in_f32)) return LA_ERR_UNSUPPORTED_DIM;
   if (a.in_f32) return launch_general_chunked_f32(a, stream);
-  const int DP = dp_of(a.d), DVT = dvt_of(a.dv);
+  const int DP = dp_of(a.d), DVT = dv_tiles(a.dv);
   // One segment keeps this path: no workspace, one launch.
   {
     const size_t need = general_chunked_bytes(a.BH, a.N, a.d, a.dv, false);

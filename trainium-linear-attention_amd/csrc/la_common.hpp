@@ -136,6 +136,10 @@ __device__ __forceinline__ u32 wave_max_u32(u32 x) {
 // Row (key / dv index) of element i of a 32x32 accumulator held by lane group h.
 __device__ __forceinline__ int c32_row(int i, int h) { return 8 * (i >> 2) + 4 * h + (i & 3); }
 
+// Rows of 64 two-byte elements in LDS, eight 16-byte units each: unit u of row r sits at u ^ swz64(r), so
+// that a fragment read (one unit of 32 rows) touches all 64 banks once per 16-lane pass.
+__device__ __forceinline__ int swz64(int r) { return ((r >> 2) & 7) ^ ((r & 2) << 1); }
+
 // ---- global -> LDS copies (buffer_load_dwordx4 ... lds)
 //
 // A raw buffer descriptor over [base, base + bytes): stride 0, num_records in bytes; dword 3

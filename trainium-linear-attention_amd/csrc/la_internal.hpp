@@ -145,6 +145,9 @@ int launch_general_chunked_f32(const ChunkedArgs& a, hipStream_t stream);
 bool layer_fused_shape(int d, int dv, int dsw, int window);   // shapes of chunked_layer_kernel
 int launch_based_layer(const LayerArgs& a, hipStream_t stream);
 int launch_feature_map(const FeatureMapArgs& a, hipStream_t stream);
+// Workspace regions start on 256-byte boundaries; value columns in 32-wide tiles: 1, 2 or 4.
+inline size_t up256(size_t x) { return (x + 255) & ~(size_t)255; }
+inline int dv_tiles(int dv) { return dv <= 32 ? 1 : dv <= 64 ? 2 : 4; }
 int device_cu_count();   // compute units of the current device (256 when the query fails)
 bool identity_shape(int d, int dv);
 size_t identity_workspace_bytes(int BH, int N, int d, int dv);

@@ -35,11 +35,7 @@ namespace la {
 namespace {
 
 constexpr int TC = 64;          // tokens per chunk of the export (a transposed row: 128 bytes)
-// The eight 16-byte units of transposed row r sit at unit ^ tswz(r): a fragment read (one unit of
-// 32 rows) touches all 64 banks once per 16-lane pass, and the transposing 8-byte writes (rows
-// four apart) are two-way at most.
-__device__ __forceinline__ int tswz(int r) { return ((r >> 2) & 7) ^ ((r & 2) << 1); }
-
+// Rows are swizzled by swz64; the transposing 8-byte writes (rows four apart) are two-way conflicts at most.
 __host__ __device__ __forceinline__ long long feat(int d) { return 1 + d + (long long)d * (d + 1) / 2; }
 // First off-diagonal feature row of x_i x_j, j > i (row of j = i + 1).
 __host__ __device__ __forceinline__ int off_row(int d, int i) { return 1 + 2 * d + i * (2 * d - i - 1) / 2; }
@@ -85,7 +81,7 @@ __device__ __forceinline__ u32 store44(uint16_t* dst, int row, int t0, const u32
       y[i] = (c & 1) ? x[i][c >> 1] >> 16 : x[i][c >> 1] & 0xffffu;
       m = max(m, y[i] & 0x7fffu);
     }
-    *reinterpret_cast<u32x2*>(dst + (row + c) * TC + (((t0 >> 3) ^ tswz(row + c)) << 3) + (t0 & 4)) =
+    *reinterpret_cast<u32x2*>(dst + (row + c) * TC + (((t0 >> 3) ^ swz64(row + c)) << 3) + (t0 & 4)) =
         (u32x2){y[0] | (y[1] << 16), y[2] | (y[3] << 16)};
   }
   return m;
@@ -186,7 +182,7 @@ __global__ __launch_bounds__(512, 4) void sexport_kernel(const ExportParams p) {
 #pragma unroll
   for (int s = 0; s < NS - 1; ++s) issue(s);
   auto frag = [&](const uint16_t* st, int row, int u) {
-    return *reinterpret_cast<const u32x4*>(st + row * TC + ((u ^ tswz(row)) << 3));
+    return *reinterpret_cast<const u32x4*>(st + row * TC + ((u ^ swz64(row)) << 3));
   };
   // stage s of this wave landed (NS - 2 later ones may be in flight), then every wave's; every wave
   // is past stage s - 1, whose place the next copies take.  Returns this wave's chunk.
@@ -641,9 +637,6 @@ __global__ __launch_bounds__(256 * MT, MT) void sapply_kernel(const ApplyParams 
 }
 
 int dp_of(int d) { return 16 * ((d + 15) / 16); }
-int mt_of(int dv) { return dv <= 32 ? 1 : dv <= 64 ? 2 : 4; }
-size_t up256(size_t x) { return (x + 255) & ~(size_t)255; }
-
 // Parts of the sequence of an export: one when the (head, column tile, i0 group) work-groups fill
 // the CUs, else enough for two per CU, of at least four 64-token chunks.
 void export_plan(int BH, int N, int d, int dv, ExportParams& p) {
@@ -681,7 +674,7 @@ struct ApplyLayout {
 ApplyLayout apply_layout(int BH, int d, int dv) {
   const int DP = dp_of(d), DB = DP / 16, DT = (DP + 31) / 32, nblk = 8 * DB * (DB + 1) + DB;
   ApplyLayout L{};
-  L.z = up256((size_t)BH * nblk * mt_of(dv) * 3072);
+  L.z = up256((size_t)BH * nblk * dv_tiles(dv) * 3072);
   L.total = L.z + up256((size_t)BH * 3 * DT * DB * 1024);
   return L;
 }
@@ -714,7 +707,7 @@ int launch_apply(const ApplyParams& p, hipStream_t stream) {
 
 template <int DP>
 int launch_apply_mt(const ApplyParams& p, hipStream_t stream) {
-  switch (mt_of(p.dv)) {
+  switch (dv_tiles(p.dv)) {
     case 1: return launch_apply<DP, 1>(p, stream);
     case 2: return launch_apply<DP, 2>(p, stream);
     default: return launch_apply<DP, 4>(p, stream);
