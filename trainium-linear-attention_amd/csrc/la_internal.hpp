@@ -121,7 +121,8 @@ struct WideStrides {   // element strides {batch, head, token}; k's serve q
   long long k[3], v[3], out[3];
 };
 size_t wide_workspace_bytes(int BH, int N, int dv);
-// any_range: |s| of any size (the packed and register-staged kernels hold up to about 430).
+// any_range: chunked calls, with |s| and V of any size (the packed and register-staged kernels hold |s| up
+// to about 430); contiguous tensors.
 int launch_wide_parallel(const ParallelArgs& a, void* workspace, bool any_range, hipStream_t stream,
                          const WideStrides* st = nullptr);
 // Whether la_based_parallel_fwd runs an aligned call of this shape on it.

@@ -141,10 +141,10 @@ def ref_based_attn(q, k, v, eps=1e-6):
 
 
 # Sequence length from which ``solution`` uses the chunked (linear-time) kernel.  Measured on
-# MI355X at d=16, dv=64, bf16 (B1 H2, B2 H16, B8 H16; N = 256 .. 16384, whole forward of each
-# path): the chunked forward was faster at every length, from 0.014 vs 0.015 ms at N=256 to
-# 0.084 vs 0.762 ms at B2 H16 N=16384; shorter sequences were not measured and stay on the
-# fused kernel.
+# MI355X at d=16, dv=64, bf16 (whole forwards, ms, chunked / fused): B8 H16 0.034 / 0.036 at N = 1024,
+# 0.263 / 2.760 at N = 16384; B2 H16 0.030 / 0.029 at N = 2048, 0.084 / 0.660 at N = 16384.  Down to
+# N = 256 the fused kernel is 2 to 8 us faster (0.018 / 0.013 at B2 H16); the line lies where it did
+# when it was not.
 CHUNKED_MIN_T = 256
 
 # Sequence length from which ``solution`` uses the segment-state chunked path for the other head
