@@ -49,10 +49,10 @@ int la_based_parallel_fwd_strided(const void* q, const void* k, const void* v, v
                                   const long long* v_strides, const long long* out_strides, float scale,
                                   float eps, void* workspace, size_t workspace_bytes, void* hip_stream);
 
-/* Whether la_based_parallel_fwd_strided takes 16-byte aligned tensors of these sizes and strides (LA_OK, or
- * the error it would return), for a caller that would rather copy than allocate an output for nothing. */
-int la_based_parallel_strided_supported(int B, int H, int N, int d, int dv, const long long* k_strides,
-                                        const long long* v_strides, const long long* out_strides);
+/* The workspace of la_based_parallel_fwd_strided (that of la_based_parallel_fwd), 0 for sizes and strides that
+ * it does not take: a caller that would then copy asks before it allocates an output. */
+size_t la_based_parallel_strided_workspace_bytes(int B, int H, int N, int d, int dv, const long long* k_strides,
+                                                 const long long* v_strides, const long long* out_strides);
 
 #ifdef __cplusplus
 }

@@ -248,6 +248,8 @@ def test_export_of_a_sequence_past_2_32_bytes_of_chunks():
     assert (out[0][:, :, 0, dv] == N).all()
     out[1][:, :, 0, dv] = N
     assert ((out[0] - out[1]).norm() / out[1][:, :, 1:].norm()).item() < 1e-5
+    del k, v, out
+    torch.cuda.empty_cache()
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
@@ -268,3 +270,5 @@ def test_chunked_sequence_past_2_32_bytes(dtype):
     p = 1 + s + 0.5 * s * s
     want = p @ v1[0, 0].double().cpu()
     assert ((num - want).norm() / want.norm()).item() < (0.1 if dtype == torch.bfloat16 else 1e-6)
+    del q, k, v
+    torch.cuda.empty_cache()

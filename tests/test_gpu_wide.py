@@ -55,7 +55,7 @@ def test_d16_grids_on_both_sides_of_the_route_limits(H, N, dv, wide):
     from tests.helpers import rows_fp64
     S = ctypes.c_longlong * 3
     s = [S(0, N * w, w) for w in (16, dv)]
-    assert _lib.lib().la_based_parallel_strided_supported(1, H, N, 16, dv, s[0], s[1], s[1]) == (0 if wide else -5)
+    assert (_lib.lib().la_based_parallel_strided_workspace_bytes(1, H, N, 16, dv, s[0], s[1], s[1]) > 0) == wide
     q, k, v = rand_qkv(1, H, N, 16, dv, seed=N, dtype=torch.bfloat16, scale_qk=0.25)
     y = K.based_parallel(q.cuda(), k.cuda(), v.cuda(), out_dtype=torch.float32).cpu()
     rows = torch.tensor([0, 63, 255, 256, N // 2, N - 1])
@@ -315,11 +315,11 @@ def test_strided_arguments():
     assert call(N=64) == -5 and call(d=60) == -5 and call(d=72) == -5 and call(k=(49152, 64, 56)) == -5
     assert call(bytes_=n - 1) == -6 and call(N=0) == 0
 
-    def supported(N=128, d=64, k=(49152, 64, 384), out=(8192, 64, 128)):
-        return L.la_based_parallel_strided_supported(1, 2, N, d, 64, S(*k), S(*k), S(*out))
+    def need(N=128, d=64, k=(49152, 64, 384), out=(8192, 64, 128)):
+        return L.la_based_parallel_strided_workspace_bytes(1, 2, N, d, 64, S(*k), S(*k), S(*out))
 
-    assert supported() == 0 and supported(k=(49152, 64, 380)) == -8 and supported(k=(0, -64, 384)) == -2
-    assert supported(N=64) == -5 and supported(d=72) == -5 and supported(out=(8192, 64, 56)) == -5 and supported(N=-1) == -2
+    assert need() == n and need(k=(49152, 64, 380)) == 0 and need(k=(0, -64, 384)) == 0 and need(N=0) == 0
+    assert need(N=64) == 0 and need(d=72) == 0 and need(out=(8192, 64, 56)) == 0 and need(N=-1) == 0
 
 
 @pytest.mark.parametrize("B,H,N,dv", [(1, 1, 65, 64), (2, 3, 200, 40), (1, 2, 1100, 64), (2, 4, 129, 24), (1, 3, 640, 32)])

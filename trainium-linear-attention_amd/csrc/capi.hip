@@ -134,8 +134,8 @@ int la_based_parallel_fwd_packed(const void* q, const void* k, const void* v, in
                         workspace, workspace_bytes, hip_stream, 2);
 }
 
-int la_based_parallel_strided_supported(int B, int H, int N, int d, int dv, const long long* k_strides,
-                                        const long long* v_strides, const long long* out_strides) {
+static int strided_shape(int B, int H, int N, int d, int dv, const long long* k_strides, const long long* v_strides,
+                         const long long* out_strides) {
   if (B < 0 || H < 0 || N < 0 || d < 1 || dv < 1) return LA_ERR_BAD_SHAPE;
   if ((long long)B * H > 0x7fffffffLL || (long long)N * (d > dv ? d : dv) > 0x7fffffffLL) return LA_ERR_BAD_SHAPE;
   if (k_strides == nullptr || v_strides == nullptr || out_strides == nullptr) return LA_ERR_NULL_POINTER;
@@ -150,6 +150,12 @@ int la_based_parallel_strided_supported(int B, int H, int N, int d, int dv, cons
   return LA_OK;
 }
 
+size_t la_based_parallel_strided_workspace_bytes(int B, int H, int N, int d, int dv, const long long* k_strides,
+                                                 const long long* v_strides, const long long* out_strides) {
+  if ((long long)B * H * N == 0 || strided_shape(B, H, N, d, dv, k_strides, v_strides, out_strides) != LA_OK) return 0;
+  return la::parallel_workspace_bytes(B * H, N, d, dv, false);
+}
+
 int la_based_parallel_fwd_strided(const void* q, const void* k, const void* v, void* out, int B, int H, int N, int d,
                                   int dv, const long long* k_strides, const long long* v_strides,
                                   const long long* out_strides, float scale, float eps, void* workspace,
@@ -160,7 +166,7 @@ int la_based_parallel_fwd_strided(const void* q, const void* k, const void* v, v
   if ((long long)B * H * N == 0) return LA_OK;
   if (k_strides == nullptr || v_strides == nullptr || out_strides == nullptr) return LA_ERR_NULL_POINTER;
   if (!al(q, 16) || !al(k, 16) || !al(v, 16) || !al(out, 16)) return LA_ERR_BAD_ALIGNMENT;
-  rc = la_based_parallel_strided_supported(B, H, N, d, dv, k_strides, v_strides, out_strides);
+  rc = strided_shape(B, H, N, d, dv, k_strides, v_strides, out_strides);
   if (rc != LA_OK) return rc;
   const size_t need = la::parallel_workspace_bytes(B * H, N, d, dv, false);
   if (workspace == nullptr || workspace_bytes < need) return LA_ERR_WORKSPACE;

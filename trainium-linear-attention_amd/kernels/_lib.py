@@ -76,8 +76,8 @@ _SIGNATURES = {
     "la_based_parallel_fwd_strided": (_c_int, [_c_void, _c_void, _c_void, _c_void, _c_int, _c_int, _c_int, _c_int,
                                                _c_int, _c_void, _c_void, _c_void, _c_float, _c_float, _c_void,
                                                _c_size, _c_void]),
-    "la_based_parallel_strided_supported": (_c_int, [_c_int, _c_int, _c_int, _c_int, _c_int, _c_void, _c_void,
-                                                     _c_void]),
+    "la_based_parallel_strided_workspace_bytes": (_c_size, [_c_int, _c_int, _c_int, _c_int, _c_int, _c_void, _c_void,
+                                                            _c_void]),
     "la_taylor_feature_map": (_c_int, [_c_void, _c_int, _c_void, _c_int, ctypes.c_longlong, _c_int, _c_void]),
 }
 

@@ -109,9 +109,9 @@ def parallel_from_projection(qkv, eps):
     row = h * d
     strides = ctypes.c_longlong * 3
     s_in, s_out = strides(3 * t * row, d, 3 * row), strides(t * row, d, row)
-    if L.la_based_parallel_strided_supported(b, h, t, d, d, s_in, s_in, s_out) != 0:
+    ws_bytes = int(L.la_based_parallel_strided_workspace_bytes(b, h, t, d, d, s_in, s_in, s_out))
+    if ws_bytes == 0:
         return None
-    ws_bytes = int(L.la_based_parallel_workspace_bytes(b, h, t, d, d, _lib.LA_BF16))
     out = torch.empty(b, t, row, dtype=qkv.dtype, device=qkv.device)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=qkv.device)
     p = qkv.data_ptr()
