@@ -242,17 +242,21 @@ __global__ __launch_bounds__(256, KS == 1 && MT == 1 && !ROWS ? 3 : 2) void wide
     for (int t = 0; t < UB; ++t) {
       const int j = UB * s + t;
       const u32 lds = lds_addr(&ring[(s % NSR) * UB + t][0]);
+      // one branch per block: a choice of resource per copy made one each, and 5 % of the chunked loop
+      auto copies = [&](const u32x4& r, const int (&off)[CW], int step) {
 #pragma unroll
-      for (int x = 0; x < CW; ++x) {
-        const int u = 4 * x + wv;
-        const bool isk = u < UK;
-        if (ANY && !isk && j >= jraw) {
-          lds_copy16(rw, lds + 1024 * u, j < nblk && woff[x] != kOffOutOfRange ? woff[x] + j * (BN * vrow) : kOffOutOfRange);
-          continue;
+        for (int x = 0; x < CW; ++x) {
+          const int u = 4 * x + wv;
+          const bool isk = u < UK;
+          const int o = isk ? uoff[x] : off[x];
+          lds_copy16(isk ? rk : r, lds + 1024 * u,
+                     j < nblk && o != kOffOutOfRange ? o + j * (isk ? BN * krow : step) : kOffOutOfRange);
         }
-        const int off = j < nblk && uoff[x] != kOffOutOfRange ? uoff[x] + j * (isk ? BN * krow : DV * BN * 2) : kOffOutOfRange;
-        lds_copy16(isk ? rk : rv, lds + 1024 * u, off);
-      }
+      };
+      if (ANY && j >= jraw)
+        copies(rw, woff, BN * vrow);
+      else
+        copies(rv, uoff, DV * BN * 2);
     }
   };
 #pragma unroll
@@ -279,49 +283,52 @@ __global__ __launch_bounds__(256, KS == 1 && MT == 1 && !ROWS ? 3 : 2) void wide
   // both in most heads); mixed: more.  ANY: fast: blocks before jb0 as u and V^T
   bool near = false, mixed = false, fast = true;
   if constexpr (ANY) {
-    u32 km = 0u, bad = 0u;
-    for (int j = tid; j < jb0; j += 256) {
-      const int e = ebs[j];
-      const u32 m = p.kmx[(size_t)bh * p.nb + j];
-      emax = max(emax, e);
-      emin = min(emin, e == -128 ? emin : e);
-      km = max(km, m & ~kCoarse);
-      bad |= m & kCoarse;
-    }
-    float l1 = 0.f;   // the largest sum of |q| of the wave's queries (NaN: above every number)
+    fast = jraw > 0;
+    if (fast) {
+      u32 km = 0u, bad = 0u;
+      for (int j = tid; j < jb0; j += 256) {
+        const int e = ebs[j];
+        const u32 m = p.kmx[(size_t)bh * p.nb + j];
+        emax = max(emax, e);
+        emin = min(emin, e == -128 ? emin : e);
+        km = max(km, m & ~kCoarse);
+        bad |= m & kCoarse;
+      }
+      float l1 = 0.f;   // the largest sum of |q| of the wave's queries (NaN: above every number)
 #pragma unroll
-    for (int qt = 0; qt < QT; ++qt) {
-      float y = 0.f;
+      for (int qt = 0; qt < QT; ++qt) {
+        float y = 0.f;
 #pragma unroll
-      for (int kk = 0; kk < KS; ++kk)
+        for (int kk = 0; kk < KS; ++kk)
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          y += __builtin_fabsf(bf16_lo_to_f32(qf[qt][kk][e])) + __builtin_fabsf(bf16_hi_to_f32(qf[qt][kk][e]));
-      y += __shfl_xor(y, 32);
-      l1 = __builtin_bit_cast(float, max(__builtin_bit_cast(u32, l1), __builtin_bit_cast(u32, y)));
-    }
-    const u32 st[5] = {wave_max_u32((u32)(emax + 1024)), wave_max_u32((u32)((1 << 21) - emin)), wave_max_u32(km),
-                       wave_max_u32(__builtin_bit_cast(u32, l1)), wave_max_u32(bad)};
-    if (lane == 0)
+          for (int e = 0; e < 4; ++e)
+            y += __builtin_fabsf(bf16_lo_to_f32(qf[qt][kk][e])) + __builtin_fabsf(bf16_hi_to_f32(qf[qt][kk][e]));
+        y += __shfl_xor(y, 32);
+        l1 = __builtin_bit_cast(float, max(__builtin_bit_cast(u32, l1), __builtin_bit_cast(u32, y)));
+      }
+      const u32 st[5] = {wave_max_u32((u32)(emax + 1024)), wave_max_u32((u32)((1 << 21) - emin)), wave_max_u32(km),
+                         wave_max_u32(__builtin_bit_cast(u32, l1)), wave_max_u32(bad)};
+      if (lane == 0)
 #pragma unroll
-      for (int i = 0; i < 5; ++i) wst[wv][i] = st[i];
-    __syncthreads();
-    u32 all[5];
-#pragma unroll
-    for (int i = 0; i < 5; ++i)
-      all[i] = (u32)__builtin_amdgcn_readfirstlane((int)max(max(wst[0][i], wst[1][i]), max(wst[2][i], wst[3][i])));
-    emax = (int)all[0] - 1024;
-    emin = (1 << 21) - (int)all[1];
-    // u in fp16: |b| = |q~ k + 1/c| <= 240 keeps b^2 - 1/c^2 below 57600
-    const float bound = __builtin_bit_cast(float, all[3]) * __builtin_bit_cast(float, all[2] << 16) + p.inv_c;
-    fast = __builtin_amdgcn_readfirstlane(jraw > 0 && emin >= emax - 8 && all[4] == 0u && bound <= 240.f);
-    near = emin < emax;
-    if (jraw > 0 && !fast) {   // the copies under way are of the wrong kind
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        for (int i = 0; i < 5; ++i) wst[wv][i] = st[i];
       __syncthreads();
-      jraw = 0;
+      u32 all[5];
 #pragma unroll
-      for (int s = 0; s < NSR - 1; ++s) issue(s);
+      for (int i = 0; i < 5; ++i)
+        all[i] = (u32)__builtin_amdgcn_readfirstlane((int)max(max(wst[0][i], wst[1][i]), max(wst[2][i], wst[3][i])));
+      emax = (int)all[0] - 1024;
+      emin = (1 << 21) - (int)all[1];
+      // u in fp16: |b| = |q~ k + 1/c| <= 240 keeps b^2 - 1/c^2 below 57600
+      const float bound = __builtin_bit_cast(float, all[3]) * __builtin_bit_cast(float, all[2] << 16) + p.inv_c;
+      fast = __builtin_amdgcn_readfirstlane(emin >= emax - 8 && all[4] == 0u && bound <= 240.f);
+      near = emin < emax;
+      if (!fast) {   // the copies under way are of the wrong kind
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        jraw = 0;
+#pragma unroll
+        for (int s = 0; s < NSR - 1; ++s) issue(s);
+      }
     }
   } else {
     if (live)
@@ -335,8 +342,9 @@ __global__ __launch_bounds__(256, KS == 1 && MT == 1 && !ROWS ? 3 : 2) void wide
     near = emin < emax;
     mixed = live && emin < emax - 8;
   }
-  // ---- column sums of V over the blocks before each query group's diagonal block
-  {
+  // ---- column sums of V over the blocks before each query group's diagonal block (`precise` counts the 1 of
+  // p itself)
+  if (fast) {
     constexpr int PARTS = 256 / DV, PF = 8;
     float* psum = reinterpret_cast<float*>(&ring[(NSR - 1) * UB][0]);   // the last step's place, still free
     const float* __restrict__ sm = p.sums + (size_t)bh * p.nb * DV + tid % DV;
@@ -357,9 +365,11 @@ __global__ __launch_bounds__(256, KS == 1 && MT == 1 && !ROWS ? 3 : 2) void wide
         for (int x = 0; x < PARTS; ++x) t += psum[x * DV + c];
         if (!ANY)
           for (int j = jb0; j < min(jd, p.nb); ++j) t += p.sums[((size_t)bh * p.nb + j) * DV + c];
-        vsl[qg][c] = fast ? t : 0.f;   // `precise` counts the 1 of p itself
+        vsl[qg][c] = t;
       }
     __syncthreads();   // psum read before the ring takes its place
+  } else {
+    for (int c = tid; c < NQW * DV; c += 256) vsl[c / DV][c % DV] = 0.f;   // read after the loops' barriers
   }
 
   f32x16 acc[QT][MT];
