@@ -33,8 +33,7 @@
 // depends on no later key or value.  Relative error of fp32 outputs, rows before / from 512, against
 // the segment path's: B1 H4 N4096 d64 dv64, q and k of the benchmark 2.6e-6 / 3.2e-6 (2.6e-6 / 1.9e-4),
 // four times as large 2.5e-6 / 4.9e-5 (2.5e-6 / 1.9e-4), sixteen times 2.4e-6 / 2.0e-4 (2.4e-6 / 2.7e-4).
-// The blocks that run `precise` cost B2 H16 N8192 d64 dv64 3 % (265 -> 273 us), N1024 24.0 -> 26.8 with the
-// pre-pass's part; all of them, for
+// The blocks that run `precise` cost B2 H16 N8192 d64 dv64 3 % (265 -> 273 us); all of them, for
 // scores out of range, 432 us (the segment path 423).
 //
 // Measured (pre-pass + kernel, us; the register-staged kernel and its max pass before): B2 H16 d64 dv64
